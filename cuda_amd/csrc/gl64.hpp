@@ -22,6 +22,7 @@
 
 #define GL_P 0xFFFFFFFF00000001ull
 #define GL_EPS 0x00000000FFFFFFFFull  // 2^64 - P = 2^32 - 1
+#define GL_R GL_EPS                   // 2^64 mod P: the factor of tables in Montgomery form
 
 typedef uint64_t u64;
 typedef uint32_t u32;
@@ -80,7 +81,8 @@ GL_HD void gl_mul_wide(u64 a, u64 b, u64 &hi, u64 &lo) {
     u64 p00 = (u64)a0 * b0;
     u64 t = (u64)a0 * b1 + (p00 >> 32);        // < 2^64
     u64 u = (u64)a1 * b0 + (u32)t;             // < 2^64
-    u64 v = (u64)a1 * b1 + ((t >> 32) + (u >> 32));
+    u64 v = (u64)a1 * b1 + (t >> 32);          // < 2^64
+    v += u >> 32;
     lo = (u << 32) | (u32)p00;
     hi = v;
 }
@@ -89,6 +91,36 @@ GL_HD u64 gl_mul(u64 a, u64 b) {
     u64 hi, lo;
     gl_mul_wide(a, b, hi, lo);
     return gl_reduce128(hi, lo);
+}
+
+// a b 2^-64 mod P.  Montgomery reduction with radix 2^64 (Montgomery 1985): with lo = x1:x0
+// and P^-1 = 2^32 + 1 (mod 2^64), q = lo P^-1 = lo + (x0 << 32), and
+// q P / 2^64 rounded up is q - (q >> 32) minus the carry of the sum that formed q, so the
+// result is hi - that, plus P on borrow.  Canonical for a canonical b (hi <= P - 1 then) and
+// any 64-bit a.  The tables hold their factors times GL_R = 2^64 mod P, so
+// gl_mmul(x, table) is the plain product; a square or a product of two field values leaves a
+// factor 2^-64, which the large path's unweighting table takes back.  The reduction is 8 VALU instructions
+// where gl_reduce128 takes 13 (whole product 20 against 25 as compiled for gfx950).
+GL_HD u64 gl_mmul(u64 a, u64 b) {
+    u64 hi, lo;
+    gl_mul_wide(a, b, hi, lo);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const u32 x0 = (u32)lo;
+    u32 e, f, g, d, k;
+    const u32 q1 = __builtin_addc((u32)(lo >> 32), x0, 0u, &e);
+    const u32 b0 = __builtin_subc(x0, q1, e, &f);
+    const u32 b1 = __builtin_subc(q1, 0u, f, &k);
+    const u32 r0 = __builtin_subc((u32)hi, b0, 0u, &g);
+    const u32 r1 = __builtin_subc((u32)(hi >> 32), b1, g, &d);
+    const u32 s0 = __builtin_subc(r0, d ? 0xFFFFFFFFu : 0u, 0u, &g);
+    const u32 s1 = __builtin_subc(r1, 0u, g, &k);
+    return ((u64)s1 << 32) | s0;
+#else
+    const u64 q = lo + (lo << 32);
+    const u64 b2 = q - (q >> 32) - (q < lo ? 1 : 0);
+    const u64 r = hi - b2;
+    return hi < b2 ? r - GL_EPS : r;
+#endif
 }
 
 // a^2 mod P.  On the device the general product is the faster square: its four

@@ -535,7 +535,7 @@ __global__ void lnt_k_field_ops(const u64 *a, const u64 *b, u32 count, u64 *out)
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
     const u64 x = a[i], y = b[i];
-    u64 *o = out + (u64)i * 8;
+    u64 *o = out + (u64)i * 9;
     o[0] = gl_add(x, y);
     o[1] = gl_sub(x, y);
     o[2] = gl_mul(x, y);
@@ -544,6 +544,7 @@ __global__ void lnt_k_field_ops(const u64 *a, const u64 *b, u32 count, u64 *out)
     o[5] = gl_mul_pow2(x, 48);
     o[6] = gl_sub_pow2(x, y, 84);
     o[7] = gl_sub_pow2(x, y, 132);
+    o[8] = gl_mmul(x, y);
 }
 
 extern "C" {
@@ -552,7 +553,7 @@ int lnt_selftest(int device, uint32_t count, uint64_t seed, uint64_t *mismatches
     if (!mismatches || count == 0) return fail(nullptr, LNT_INVALID_ARGUMENT, "bad argument");
     if (hipSetDevice(device) != hipSuccess) return fail(nullptr, LNT_DEVICE_ERROR, "hipSetDevice failed");
     // operands: canonical values with the edge cases first (0, 1, P-1, 2^32, EPS, ...)
-    std::vector<u64> a(count), b(count), out((size_t)count * 8);
+    std::vector<u64> a(count), b(count), out((size_t)count * 9);
     const u64 edge[] = {0, 1, 2, GL_P - 1, GL_P - 2, 1ull << 32, GL_EPS, (1ull << 63), GL_P >> 1, (GL_P >> 1) + 1};
     const u32 ne = sizeof edge / sizeof edge[0];
     u64 st = seed;
@@ -569,13 +570,13 @@ int lnt_selftest(int device, uint32_t count, uint64_t seed, uint64_t *mismatches
     }
     u64 *da = nullptr, *db = nullptr, *dout = nullptr;
     bool ok = hipMalloc(&da, (size_t)count * 8) == hipSuccess && hipMalloc(&db, (size_t)count * 8) == hipSuccess &&
-              hipMalloc(&dout, (size_t)count * 64) == hipSuccess &&
+              hipMalloc(&dout, (size_t)count * 72) == hipSuccess &&
               hipMemcpy(da, a.data(), (size_t)count * 8, hipMemcpyHostToDevice) == hipSuccess &&
               hipMemcpy(db, b.data(), (size_t)count * 8, hipMemcpyHostToDevice) == hipSuccess;
     if (ok) {
         hipLaunchKernelGGL(lnt_k_field_ops, dim3((count + 255) / 256), dim3(256), 0, 0, da, db, count, dout);
         ok = hipGetLastError() == hipSuccess &&
-             hipMemcpy(out.data(), dout, (size_t)count * 64, hipMemcpyDeviceToHost) == hipSuccess;
+             hipMemcpy(out.data(), dout, (size_t)count * 72, hipMemcpyDeviceToHost) == hipSuccess;
     }
     if (da) (void)hipFree(da);
     if (db) (void)hipFree(db);
@@ -583,11 +584,11 @@ int lnt_selftest(int device, uint32_t count, uint64_t seed, uint64_t *mismatches
     if (!ok) return fail(nullptr, LNT_DEVICE_ERROR, "lnt_selftest: device error");
     u64 bad = 0;
     for (u32 i = 0; i < count; i++) {
-        const u64 x = a[i], y = b[i], *o = &out[(size_t)i * 8];
-        const u64 want[8] = {gl_add(x, y),          gl_sub(x, y),          gl_mul(x, y),
+        const u64 x = a[i], y = b[i], *o = &out[(size_t)i * 9];
+        const u64 want[9] = {gl_add(x, y),          gl_sub(x, y),          gl_mul(x, y),
                              gl_sqr(x),             gl_mul_pow2(x, 12),    gl_mul_pow2(x, 48),
-                             gl_sub_pow2(x, y, 84), gl_sub_pow2(x, y, 132)};
-        for (int k = 0; k < 8; k++) bad += o[k] != want[k];
+                             gl_sub_pow2(x, y, 84), gl_sub_pow2(x, y, 132), gl_mmul(x, y)};
+        for (int k = 0; k < 9; k++) bad += o[k] != want[k];
     }
     *mismatches = bad;
     return LNT_OK;

@@ -50,6 +50,8 @@ struct LntParams {
                              // pairs at 2 * slot, the unweights at slot
     GView<const u64> tw4, itw4;  // 4-step twiddles (large path), natural slots, times the column
                                  // weight factor (unweight factor * n^-1)
+                                 // (all twiddle tables and the large path's unweights are in
+                                 // the Montgomery form that gl_mmul takes)
     GView<const u64> twr, itwr;  // row-line twiddles (C words)
     GView<const u64> twr2, itwr2;  // second-level row twiddles (3-phase rows: B^2 words)
     GView<const u64> twc, itwc;  // column-line twiddles (R words)
@@ -209,7 +211,7 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     dft_fwd<B1>(a);
     if (B2 > 1) {
 #pragma unroll
-        for (int rho = 1; rho < B1; rho++) a[rho] = gl_mul(a[rho], P.twc[(u64)rho * B2 + t]);
+        for (int rho = 1; rho < B1; rho++) a[rho] = gl_mmul(a[rho], P.twc[(u64)rho * B2 + t]);
     }
     LNT_SYNC();
 #pragma unroll
@@ -259,13 +261,13 @@ LNT_KFN void lnt_col_inv_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int rho = 0; rho < B1; rho++) {
         u64 v = lds[(u32)((brev_c<B1>(rho) * S + t) * K + cl)];
-        a[rho] = (B2 > 1 && rho > 0) ? gl_mul(v, P.itwc[(u64)rho * B2 + t]) : v;
+        a[rho] = (B2 > 1 && rho > 0) ? gl_mmul(v, P.itwc[(u64)rho * B2 + t]) : v;
     }
     dft_inv<B1>(a);
 #pragma unroll
     for (int j = 0; j < B1; j++) {
         const u64 idx = c + C * ((u64)t + (u64)B2 * j);
-        P.x[idx] = gl_mul(a[j], PF ? uv[PF ? j : 0] : P.uw[lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j))]);
+        P.x[idx] = gl_mmul(a[j], PF ? uv[PF ? j : 0] : P.uw[lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j))]);
     }
 }
 
@@ -379,7 +381,7 @@ LNT_KFN void lnt_col3_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
     }
     dft_fwd<BA>(a);
 #pragma unroll
-    for (int rho = 1; rho < BA; rho++) a[rho] = gl_mul(a[rho], P.twc[(u64)rho * A + t]);
+    for (int rho = 1; rho < BA; rho++) a[rho] = gl_mmul(a[rho], P.twc[(u64)rho * A + t]);
     LNT_SYNC();
 #pragma unroll
     for (int rho = 0; rho < BA; rho++) lds[(u32)((brev_c<BA>(rho) * RS + t) * KP + cl)] = a[rho];
@@ -406,7 +408,7 @@ LNT_KFN void lnt_col3_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
         const u64 tb = (u64)brev_c<BB>(k2) * BC;
 #pragma unroll
         for (int u = 0; u < BC; u++)
-            a[q * BC + u] = gl_mul(lds[(u32)((k1 * RS + BC * k2 + u) * KP + cl)], P.twc2[tb + u]);
+            a[q * BC + u] = gl_mmul(lds[(u32)((k1 * RS + BC * k2 + u) * KP + cl)], P.twc2[tb + u]);
         dft_fwd<BC>(a + q * BC);
     }
 #pragma unroll
@@ -434,7 +436,7 @@ LNT_KFN void lnt_col3_inv_body(int tid, int bid, LView lds, const LntParams &P) 
         dft_inv<BC>(a + q * BC);
 #pragma unroll
         for (int u = 0; u < BC; u++)
-            lds[(u32)((k1 * RS + BC * k2 + u) * KP + cl)] = gl_mul(a[q * BC + u], P.itwc2[tb + u]);
+            lds[(u32)((k1 * RS + BC * k2 + u) * KP + cl)] = gl_mmul(a[q * BC + u], P.itwc2[tb + u]);
     }
     LNT_SYNC();
     // phase 2 inverse
@@ -453,13 +455,13 @@ LNT_KFN void lnt_col3_inv_body(int tid, int bid, LView lds, const LntParams &P) 
 #pragma unroll
     for (int rho = 0; rho < BA; rho++) {
         u64 v = lds[(u32)((brev_c<BA>(rho) * RS + t) * KP + cl)];
-        a[rho] = rho ? gl_mul(v, P.itwc[(u64)rho * A + t]) : v;
+        a[rho] = rho ? gl_mmul(v, P.itwc[(u64)rho * A + t]) : v;
     }
     dft_inv<BA>(a);
 #pragma unroll
     for (int j = 0; j < BA; j++) {
         const u64 idx = c + C * ((u64)t + (u64)A * j);
-        P.x[idx] = gl_mul(a[j], uv[j]);
+        P.x[idx] = gl_mmul(a[j], uv[j]);
     }
 }
 
@@ -482,12 +484,12 @@ LNT_KFN void lnt_row_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int j = 0; j < B1; j++) {
         const u64 idx = base + t + (u64)B2 * j;
-        a[j] = gl_mul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
+        a[j] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
     }
     dft_fwd<B1>(a);
     if (B2 > 1) {
 #pragma unroll
-        for (int rho = 1; rho < B1; rho++) a[rho] = gl_mul(a[rho], P.twr[(u64)rho * B2 + t]);
+        for (int rho = 1; rho < B1; rho++) a[rho] = gl_mmul(a[rho], P.twr[(u64)rho * B2 + t]);
     }
 #pragma unroll
     for (int rho = 0; rho < B1; rho++) lds[lb + (u32)(brev_c<B1>(rho) * S + t)] = a[rho];
@@ -506,10 +508,10 @@ LNT_KFN void lnt_row_body(int tid, int bid, LView lds, const LntParams &P) {
         if (MODE == LNT_MULTIPLY) {
 #pragma unroll
             for (int i1 = 0; i1 < B2; i1++)
-                a[q * B2 + i1] = gl_mul(a[q * B2 + i1], P.f[base + (u64)t * B1 + q * B2 + i1]);
+                a[q * B2 + i1] = gl_mmul(a[q * B2 + i1], P.f[base + (u64)t * B1 + q * B2 + i1]);
         } else {
 #pragma unroll
-            for (int i1 = 0; i1 < B2; i1++) a[q * B2 + i1] = gl_sqr(a[q * B2 + i1]);
+            for (int i1 = 0; i1 < B2; i1++) a[q * B2 + i1] = gl_mmul(a[q * B2 + i1], a[q * B2 + i1]);
         }
         dft_inv<B2>(a + q * B2);
 #pragma unroll
@@ -520,13 +522,13 @@ LNT_KFN void lnt_row_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int rho = 0; rho < B1; rho++) {
         u64 v = lds[lb + (u32)(brev_c<B1>(rho) * S + t)];
-        a[rho] = (B2 > 1 && rho > 0) ? gl_mul(v, P.itwr[(u64)rho * B2 + t]) : v;
+        a[rho] = (B2 > 1 && rho > 0) ? gl_mmul(v, P.itwr[(u64)rho * B2 + t]) : v;
     }
     dft_inv<B1>(a);
 #pragma unroll
     for (int j = 0; j < B1; j++) {
         const u64 idx = base + t + (u64)B2 * j;
-        P.y[idx] = gl_mul(a[j], P.itw4[idx]);  // inverse 4-step twiddle
+        P.y[idx] = gl_mmul(a[j], P.itw4[idx]);  // inverse 4-step twiddle
     }
 }
 
@@ -558,7 +560,7 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int j = 0; j < B; j++) {
         const u64 idx = base + t + (u64)T * j;
-        a[j] = gl_mul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
+        a[j] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
     }
     // the inverse 4-step twiddles of the final store, fetched now so their latency hides
     // behind the transforms
@@ -569,7 +571,7 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
     }
     dft_fwd<B>(a);
 #pragma unroll
-    for (int rho = 1; rho < B; rho++) a[rho] = gl_mul(a[rho], P.twr[(u64)rho * T + t]);
+    for (int rho = 1; rho < B; rho++) a[rho] = gl_mmul(a[rho], P.twr[(u64)rho * T + t]);
 #pragma unroll
     for (int rho = 0; rho < B; rho++) lds[lb + (u32)(brev_c<B>(rho) * RS + (t / B) * (B + PAD) + t % B)] = a[rho];
     LNT_SYNC();
@@ -579,7 +581,7 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
     // (this thread rewrites exactly the slots it just read: no barrier needed)
     dft_fwd<B>(a);
 #pragma unroll
-    for (int rho = 1; rho < B; rho++) a[rho] = gl_mul(a[rho], P.twr2[(u64)rho * B + lo]);
+    for (int rho = 1; rho < B; rho++) a[rho] = gl_mmul(a[rho], P.twr2[(u64)rho * B + lo]);
 #pragma unroll
     for (int rho = 0; rho < B; rho++) lds[lb + (u32)(hi * RS + brev_c<B>(rho) * (B + PAD) + lo)] = a[rho];
     LNT_SYNC();
@@ -594,10 +596,10 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
     }
     if (MODE == LNT_MULTIPLY) {
 #pragma unroll
-        for (int i = 0; i < B; i++) a[i] = gl_mul(a[i], P.f[base + (u64)t * B + i]);
+        for (int i = 0; i < B; i++) a[i] = gl_mmul(a[i], P.f[base + (u64)t * B + i]);
     } else {
 #pragma unroll
-        for (int i = 0; i < B; i++) a[i] = gl_sqr(a[i]);
+        for (int i = 0; i < B; i++) a[i] = gl_mmul(a[i], a[i]);
     }
     dft_inv<B>(a);
 #pragma unroll
@@ -607,7 +609,7 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int rho = 0; rho < B; rho++) {
         u64 v = lds[lb + (u32)(hi * RS + brev_c<B>(rho) * (B + PAD) + lo)];
-        a[rho] = rho ? gl_mul(v, P.itwr2[(u64)rho * B + lo]) : v;
+        a[rho] = rho ? gl_mmul(v, P.itwr2[(u64)rho * B + lo]) : v;
     }
     dft_inv<B>(a);
 #pragma unroll
@@ -617,11 +619,11 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int rho = 0; rho < B; rho++) {
         u64 v = lds[lb + (u32)(brev_c<B>(rho) * RS + (t / B) * (B + PAD) + t % B)];
-        a[rho] = rho ? gl_mul(v, P.itwr[(u64)rho * T + t]) : v;
+        a[rho] = rho ? gl_mmul(v, P.itwr[(u64)rho * T + t]) : v;
     }
     dft_inv<B>(a);
 #pragma unroll
-    for (int j = 0; j < B; j++) P.y[base + t + (u64)T * j] = gl_mul(a[j], iv[MODE == LNT_FORWARD ? 0 : j]);
+    for (int j = 0; j < B; j++) P.y[base + t + (u64)T * j] = gl_mmul(a[j], iv[MODE == LNT_FORWARD ? 0 : j]);
 }
 
 // ------------------------------------------------------------------ mixed-radix 3-phase rows
@@ -656,12 +658,12 @@ LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int j = 0; j < BA; j++) {
         const u64 idx = base + t + (u64)A * j;
-        a[j] = gl_mul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
+        a[j] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
     }
     // phase 1
     dft_fwd<BA>(a);
 #pragma unroll
-    for (int rho = 1; rho < BA; rho++) a[rho] = gl_mul(a[rho], P.twr[(u64)rho * A + t]);
+    for (int rho = 1; rho < BA; rho++) a[rho] = gl_mmul(a[rho], P.twr[(u64)rho * A + t]);
 #pragma unroll
     for (int rho = 0; rho < BA; rho++) lds[pos(brev_c<BA>(rho), t)] = a[rho];
     LNT_SYNC();
@@ -689,7 +691,7 @@ LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
             const u64 tb = (u64)brev_c<BB>(k2) * BC;  // twr2 row of k2
             u64 e[BC];
 #pragma unroll
-            for (int u = 0; u < BC; u++) e[u] = gl_mul(lds[pos(k1, u + BC * k2)], P.twr2[tb + u]);
+            for (int u = 0; u < BC; u++) e[u] = gl_mmul(lds[pos(k1, u + BC * k2)], P.twr2[tb + u]);
             dft_fwd<BC>(e);
             const u64 so = base + (u64)I * BC;
             if (MODE == LNT_FORWARD) {
@@ -699,14 +701,14 @@ LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
             }
             if (MODE == LNT_MULTIPLY) {
 #pragma unroll
-                for (int i = 0; i < BC; i++) e[i] = gl_mul(e[i], P.f[so + i]);
+                for (int i = 0; i < BC; i++) e[i] = gl_mmul(e[i], P.f[so + i]);
             } else {
 #pragma unroll
-                for (int i = 0; i < BC; i++) e[i] = gl_sqr(e[i]);
+                for (int i = 0; i < BC; i++) e[i] = gl_mmul(e[i], e[i]);
             }
             dft_inv<BC>(e);
 #pragma unroll
-            for (int u = 0; u < BC; u++) lds[pos(k1, u + BC * k2)] = gl_mul(e[u], P.itwr2[tb + u]);
+            for (int u = 0; u < BC; u++) lds[pos(k1, u + BC * k2)] = gl_mmul(e[u], P.itwr2[tb + u]);
         }
     }
     if (MODE == LNT_FORWARD) return;
@@ -729,13 +731,13 @@ LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int rho = 0; rho < BA; rho++) {
         u64 v = lds[pos(brev_c<BA>(rho), t)];
-        a[rho] = rho ? gl_mul(v, P.itwr[(u64)rho * A + t]) : v;
+        a[rho] = rho ? gl_mmul(v, P.itwr[(u64)rho * A + t]) : v;
     }
     dft_inv<BA>(a);
 #pragma unroll
     for (int j = 0; j < BA; j++) {
         const u64 idx = base + t + (u64)A * j;
-        P.y[idx] = gl_mul(a[j], P.itw4[idx]);
+        P.y[idx] = gl_mmul(a[j], P.itw4[idx]);
     }
 }
 
@@ -797,7 +799,7 @@ LNT_KFN void lnt_small_body(int tid, LView lds, const LntParams &P, u32 iters, b
         dft_fwd<B1>(a);
         if (B2 > 1) {
 #pragma unroll
-            for (int rho = 1; rho < B1; rho++) a[rho] = gl_mul(a[rho], Ttw[(u64)rho * B2 + t]);
+            for (int rho = 1; rho < B1; rho++) a[rho] = gl_mmul(a[rho], Ttw[(u64)rho * B2 + t]);
         }
         LNT_SYNC();
 #pragma unroll
@@ -831,7 +833,7 @@ LNT_KFN void lnt_small_body(int tid, LView lds, const LntParams &P, u32 iters, b
 #pragma unroll
         for (int rho = 0; rho < B1; rho++) {
             u64 v = lds[(u32)(brev_c<B1>(rho) * S + t)];
-            a[rho] = (B2 > 1 && rho > 0) ? gl_mul(v, Titw[(u64)rho * B2 + t]) : v;
+            a[rho] = (B2 > 1 && rho > 0) ? gl_mmul(v, Titw[(u64)rho * B2 + t]) : v;
         }
         dft_inv<B1>(a);
         LNT_SYNC();
@@ -900,7 +902,7 @@ LNT_KFN void lnt_small3_body(int tid, LView lds, const LntParams &P, u32 iters, 
         }
         dft_fwd<B>(a);
 #pragma unroll
-        for (int rho = 1; rho < B; rho++) a[rho] = gl_mul(a[rho], Ttw[(u64)rho * T + t]);
+        for (int rho = 1; rho < B; rho++) a[rho] = gl_mmul(a[rho], Ttw[(u64)rho * T + t]);
 #pragma unroll
         for (int rho = 0; rho < B; rho++) lds[Z + (u32)(brev_c<B>(rho) * RS + hi * (B + 1) + lo)] = a[rho];
         LNT_SYNC();
@@ -909,7 +911,7 @@ LNT_KFN void lnt_small3_body(int tid, LView lds, const LntParams &P, u32 iters, 
         for (int b = 0; b < B; b++) a[b] = lds[Z + (u32)(hi * RS + b * (B + 1) + lo)];
         dft_fwd<B>(a);
 #pragma unroll
-        for (int rho = 1; rho < B; rho++) a[rho] = gl_mul(a[rho], Ttw2[(u64)rho * B + lo]);
+        for (int rho = 1; rho < B; rho++) a[rho] = gl_mmul(a[rho], Ttw2[(u64)rho * B + lo]);
 #pragma unroll
         for (int rho = 0; rho < B; rho++) lds[Z + (u32)(hi * RS + brev_c<B>(rho) * (B + 1) + lo)] = a[rho];
         LNT_SYNC();
@@ -937,7 +939,7 @@ LNT_KFN void lnt_small3_body(int tid, LView lds, const LntParams &P, u32 iters, 
 #pragma unroll
         for (int rho = 0; rho < B; rho++) {
             u64 v = lds[Z + (u32)(hi * RS + brev_c<B>(rho) * (B + 1) + lo)];
-            a[rho] = rho ? gl_mul(v, Titw2[(u64)rho * B + lo]) : v;
+            a[rho] = rho ? gl_mmul(v, Titw2[(u64)rho * B + lo]) : v;
         }
         dft_inv<B>(a);
 #pragma unroll
@@ -947,7 +949,7 @@ LNT_KFN void lnt_small3_body(int tid, LView lds, const LntParams &P, u32 iters, 
 #pragma unroll
         for (int rho = 0; rho < B; rho++) {
             u64 v = lds[Z + (u32)(brev_c<B>(rho) * RS + hi * (B + 1) + lo)];
-            a[rho] = rho ? gl_mul(v, Titw[(u64)rho * T + t]) : v;
+            a[rho] = rho ? gl_mmul(v, Titw[(u64)rho * T + t]) : v;
         }
         dft_inv<B>(a);
 #pragma unroll
@@ -962,12 +964,13 @@ LNT_KFN void lnt_small3_body(int tid, LView lds, const LntParams &P, u32 iters, 
 }
 
 // ------------------------------------------------------------------ tables
+// Twiddle tables are in Montgomery form (times GL_R) for gl_mmul.
 // Twiddles of a line of L = B1 * B2 words: tw[rho * B2 + t] = omega_L^(t * brev_B1(rho)).
 GL_HD u64 lnt_line_tw(u64 omega_L, u32 B1, u32 B2, u32 idx) {
     u32 rho = idx / B2, t = idx % B2;
     u32 br = 0;
     for (u32 b = 1, v = rho; b < B1; b <<= 1, v >>= 1) br = (br << 1) | (v & 1);
-    return gl_pow(omega_L, (u64)t * br);
+    return gl_mul(gl_pow(omega_L, (u64)t * br), GL_R);
 }
 
 // 4-step twiddle for slot idx = c + C * r', r' = t*B1 + q*B2 + rho' (column line B1 x B2):
@@ -979,7 +982,7 @@ GL_HD u64 lnt_tw4(u64 omega_n, u32 C, u32 B1, u32 B2, u64 idx) {
     u32 br = 0;
     for (u32 b = 1, v = rp; b < B2; b <<= 1, v >>= 1) br = (br << 1) | (v & 1);
     u64 kcol = (u64)B1 * br + (u64)t * (B1 / B2) + q;
-    return gl_pow(omega_n, (u64)c * kcol);
+    return gl_mul(gl_pow(omega_n, (u64)c * kcol), GL_R);
 }
 
 // 4-step twiddle of a 3-phase column (radices BA, BB, BC): slot s = t*BA + q*BC + rho
@@ -991,19 +994,22 @@ GL_HD u64 lnt_tw4_3(u64 omega_n, u32 C, u32 BA, u32 BB, u32 BC, u64 idx) {
     u32 br = 0;
     for (u32 b = 1, v = rho; b < BC; b <<= 1, v >>= 1) br = (br << 1) | (v & 1);
     const u64 kcol = k1 + (u64)BA * (k2 + (u64)BB * br);
-    return gl_pow(omega_n, (u64)c * kcol);
+    return gl_mul(gl_pow(omega_n, (u64)c * kcol), GL_R);
 }
 
-// Large-path weight tables (the factorisation at lnt_wexp): row slot 2r + h holds B^f_r,
-// times m when h = 1 (B = weight base, m = 1/2; or B = its inverse, m = 2 for unweights).
+// Large-path weight tables (the factorisation at lnt_wexp), row slots 2r + h.
+// Unweights: B^f_r (B the inverse weight base), times m = 2 when h = 1, times GL_R^2: one
+// GL_R for the Montgomery multiply that applies it, one for the 2^-64 the square left.
 GL_HD u64 lnt_row_factor(u64 B, u64 m, u32 p, u32 n, u32 C, u32 slot) {
-    const u64 v = gl_pow(B, lnt_wexp(p, n, (u64)C * (slot >> 1)));
+    const u64 v = gl_mul(gl_pow(B, lnt_wexp(p, n, (u64)C * (slot >> 1))), gl_mul(GL_R, GL_R));
     return (slot & 1) ? gl_mul(v, m) : v;
 }
-// Word i of the large-path weight table: the pair (w, -2^31 w) of slot i / 2
-// (gl_mul_biased takes both).
+// Weights: word i is half of the pair (w, -2^31 w) of slot i / 2 (gl_mul_biased takes both),
+// w = B^f_r, halved when h = 1.
 GL_HD u64 lnt_weight_pair(u64 Bw, u32 p, u32 n, u32 C, u32 i) {
-    const u64 w = lnt_row_factor(Bw, (GL_P + 1) / 2, p, n, C, i >> 1);
+    const u32 slot = i >> 1;
+    u64 w = gl_pow(Bw, lnt_wexp(p, n, (u64)C * (slot >> 1)));
+    if (slot & 1) w = gl_mul(w, (GL_P + 1) / 2);
     return (i & 1) ? gl_mul(w, GL_P - (1ull << 31)) : w;
 }
 // Column factor B^e_c times s (s = 1 for weights, n^-1 for unweights), c = idx mod C.

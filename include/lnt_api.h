@@ -99,8 +99,8 @@ uint32_t lnt_secured_log2_length(uint32_t p);
 int lnt_tune_export(char *buf, size_t len);
 int lnt_tune_import(const char *text);
 
-/* Self-test of the device field arithmetic (new): add, sub, mul, square and the shift
- * multiplies computed on the GPU for `count` operand pairs (edge values, then splitmix64
+/* Self-test of the device field arithmetic (new): add, sub, mul, square, the shift and the
+ * Montgomery multiplies computed on the GPU for `count` operand pairs (edge values, then splitmix64
  * draws from `seed`) and compared with the host forms; *mismatches = differing results. */
 int lnt_selftest(int device, uint32_t count, uint64_t seed, uint64_t *mismatches);
 

@@ -398,6 +398,7 @@ extern "C" uint32_t emu_levels(void *h) { return ((Emu *)h)->pl.levels; }
 extern "C" uint32_t emu_secured(uint32_t p) { return secured_log2_length(p); }
 extern "C" uint32_t emu_carry_levels(uint32_t p, uint32_t n) { return carry_levels(p, n); }
 extern "C" uint64_t emu_gl_mul_biased(uint32_t db, uint64_t w, uint64_t wb) { return gl_mul_biased(db, w, wb); }
+extern "C" uint64_t emu_gl_mmul(uint64_t a, uint64_t b) { return gl_mmul(a, b); }
 extern "C" int emu_digits_fit_31(uint32_t p, uint32_t n) {
     const uint32_t levels = carry_levels(p, n);
     return levels ? (int)digits_fit_31(p, n, levels) : -1;
