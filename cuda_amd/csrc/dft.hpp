@@ -64,3 +64,5 @@ GL_HD constexpr int brev_c(int v) {
     }
     return r;
 }
+// The same of a run-time value below 16.
+GL_HD int brev_v16(int v) { return (v & 1) << 3 | (v & 2) << 1 | (v & 4) >> 1 | (v & 8) >> 3; }

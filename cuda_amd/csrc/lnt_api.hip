@@ -605,6 +605,7 @@ static std::string describe(const Plan &pl) {
     } else {
         char row[64];
         if (pl.row3m) std::snprintf(row, sizeof row, "lnt_k_row3m<%u,%u,%u>", pl.row3m, pl.rBB, pl.rBC);
+        else if (pl.row3 == 16) std::snprintf(row, sizeof row, "lnt_k_row16");
         else if (pl.row3) std::snprintf(row, sizeof row, "lnt_k_row3<%u,%u>", pl.row3, pl.G);
         else std::snprintf(row, sizeof row, "lnt_k_row<%u,%u>", pl.row.B1, pl.row.B2);
         if (pl.col3)

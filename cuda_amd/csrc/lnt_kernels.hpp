@@ -39,6 +39,7 @@
 // preserved exactly (the carry out of digit n-1 enters digit 0 with weight 2^p = 1).
 #pragma once
 #include "dft.hpp"
+#include "mdft.hpp"
 #include "simt.hpp"
 
 struct LntParams {
@@ -624,6 +625,104 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
     dft_inv<B>(a);
 #pragma unroll
     for (int j = 0; j < B; j++) P.y[base + t + (u64)T * j] = gl_mmul(a[j], iv[MODE == LNT_FORWARD ? 0 : j]);
+}
+
+// ------------------------------------------------------------------ 4096-word rows on the matrix cores
+// The row pass for C = 4096 = 16^3 with the 16-point DFTs of mdft.hpp: one row per workgroup
+// of W = 16 / GW waves, GW groups of 16 DFTs per wave and phase (4 GW words per thread).  With
+// i = i1 + 256 j, i1 = a + 16 b; group h = GW w + g of wave w, lane (q, n):
+//   phase 1: DFTs i1 = 16 h + n over j -> k2, twiddle omega_C^(i1 k2)     (twr)
+//   phase 2: DFTs (k2 = h, a = n) over b -> kb, twiddle omega_256^(a kb)  (twr2)
+//   phase 3: DFTs (k2 = h, kb = n) over a; square (or the product modes); the inverse takes
+//            the result as it lies.
+// A wave keeps its k2 between phase 1 and the inverse phase 2, so only the exchanges around
+// these wait for the other waves.  LDS word (row r of 16 words, x) at 18 r + x: runs of 16 words
+// start 16-byte aligned and 16 neighbouring runs cover all 64 banks, so the reads of adjacent
+// word pairs are 128-bit and free of conflicts.  Transform-domain slot for MODE 1/2: base + 4 GW t + 4 g + place.
+constexpr u32 LNT_ROW16_LDS = 256 * 18;
+template <int GW, int MODE = LNT_SQUARE>
+LNT_KFN void lnt_row16_body(int tid, int bid, LView lds, const LntParams &P) {
+    const int w = LNT_UNIFORM(tid / 64), q = (tid % 64) / 16, n = tid % 16;
+    const u64 base = (u64)4096 * (u64)bid;
+    LntM16 M;
+    u64 z[4], tw[4];
+    // phase 1
+#pragma unroll 1
+    for (int h = GW * w; h < GW * w + GW; h++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int k = lnt_m16_word(q, e);
+            const u64 idx = base + 16 * h + n + 256 * k;
+            z[e] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
+            tw[e] = P.twr[256 * brev_v16(k) + 16 * h + n];
+        }
+        if (h == GW * w) lnt_m16_load(M, tid);
+        lnt_m16_dft(M, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[(u32)(288 * lnt_m16_word(q, v) + 18 * n + h)] = gl_mmul(z[v], tw[v]);
+    }
+    LNT_SYNC();
+    // phases 2 and 3, the pointwise step and their inverses
+#pragma unroll 1
+    for (int h = GW * w; h < GW * w + GW; h++) {
+        const u32 row = (u32)(288 * h), own = row + (u32)(18 * n + 2 * q);  // this lane's words of run n
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            z[e] = lds[own + lnt_m16_word(0, e)];
+            tw[e] = P.twr2[16 * brev_v16(lnt_m16_word(q, e)) + n];
+        }
+        lnt_m16_dft(M, z);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 4; v++) lds[(u32)(row + 18 * lnt_m16_word(q, v) + n)] = gl_mmul(z[v], tw[v]);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int e = 0; e < 4; e++) z[e] = lds[own + lnt_m16_word(0, e)];
+        if (MODE != LNT_FORWARD) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) tw[v] = P.itwr2[16 * brev_v16(n) + ((16 - lnt_m16_word(q, v)) & 15)];
+        }
+        lnt_m16_dft(M, z);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const u64 slot = base + 4 * GW * (u64)tid + 4 * (h - GW * w) + v;
+            if (MODE == LNT_FORWARD) P.y[slot] = z[v];
+            else z[v] = gl_mmul(z[v], MODE == LNT_MULTIPLY ? P.f[slot] : z[v]);
+        }
+        if (MODE == LNT_FORWARD) continue;
+        lnt_m16_dft(M, z);  // inverse phase 3: output place v is the word -k
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[(u32)(row + 18 * ((16 - lnt_m16_word(q, v)) & 15) + n)] = gl_mmul(z[v], tw[v]);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            z[e] = lds[own + lnt_m16_word(0, e)];
+            tw[e] = P.itwr[256 * brev_v16(h) + n + 16 * ((16 - lnt_m16_word(q, e)) & 15)];
+        }
+        lnt_m16_dft(M, z);  // inverse phase 2
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[(u32)(row + 18 * n + ((16 - lnt_m16_word(q, v)) & 15))] = gl_mmul(z[v], tw[v]);
+    }
+    if (MODE == LNT_FORWARD) return;
+    LNT_SYNC();
+    // inverse phase 1, inverse 4-step twiddle, store
+#pragma unroll 1
+    for (int h = GW * w; h < GW * w + GW; h++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            z[e] = lds[(u32)(288 * lnt_m16_word(q, e) + 18 * n + h)];
+            tw[e] = P.itw4[base + 16 * h + n + 256 * ((16 - lnt_m16_word(q, e)) & 15)];
+        }
+        lnt_m16_dft(M, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            P.y[base + 16 * h + n + 256 * ((16 - lnt_m16_word(q, v)) & 15)] = gl_mmul(z[v], tw[v]);
+    }
 }
 
 // ------------------------------------------------------------------ mixed-radix 3-phase rows

@@ -66,13 +66,19 @@ __global__ __launch_bounds__(G * B2) void lnt_k_row(LntParams P) {
     lnt_row_body<B1, B2, G, MODE>(threadIdx.x, blockIdx.x, LView{smem, W}, P);
 }
 
-// 256-thread rows of 16^3 (or 4 rows of 8^3) words in 32 KiB of LDS; 128 registers per
-// lane keep 4 waves per SIMD
+// workgroups of 4 rows of 8^3 words; 128 registers per lane keep 4 waves per SIMD
 template <int B, int G, int MODE>
 __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) void lnt_k_row3(LntParams P) {
     constexpr u32 W = G * B * B * B;
     __shared__ u64 smem[W];
     lnt_row3_body<B, G, MODE>(threadIdx.x, blockIdx.x, LView{smem, W}, P);
+}
+
+// 4096-word rows on the matrix cores
+template <int GW, int MODE>
+__global__ __launch_bounds__(1024 / GW) __attribute__((amdgpu_waves_per_eu(4))) void lnt_k_row16(LntParams P) {
+    __shared__ __align__(16) u64 smem[LNT_ROW16_LDS];
+    lnt_row16_body<GW, MODE>(threadIdx.x, blockIdx.x, LView{smem, LNT_ROW16_LDS}, P);
 }
 
 // 16 words per thread: two workgroups per CU fit the LDS when each wave stays within 128
@@ -179,6 +185,15 @@ __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) 
     const LntParams P = Ps[blockIdx.x / wgs];
     if (P.n == 0) return;  // an empty slot of the batch
     lnt_row3_body<B, G>(threadIdx.x, blockIdx.x % wgs, LView{smem, W}, P);
+}
+
+template <int GW>
+__global__ __launch_bounds__(1024 / GW) __attribute__((amdgpu_waves_per_eu(4))) void lnt_kb_row16(
+    const LntParams *__restrict__ Ps, u32 wgs) {
+    __shared__ __align__(16) u64 smem[LNT_ROW16_LDS];
+    const LntParams P = Ps[blockIdx.x / wgs];
+    if (P.n == 0) return;  // an empty slot of the batch
+    lnt_row16_body<GW>(threadIdx.x, blockIdx.x % wgs, LView{smem, LNT_ROW16_LDS}, P);
 }
 
 template <int BA, int BB, int BC>

@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #define LNT_SYNC() _Pragma("omp barrier")
+#define LNT_WAVE_SYNC() _Pragma("omp barrier")
 #define LNT_CHECK(cond, what)                                                      \
     do {                                                                           \
         if (!(cond)) {                                                             \
@@ -19,11 +20,22 @@
         }                                                                          \
     } while (0)
 #define LNT_KFN static inline
+#define LNT_UNIFORM(v) (v)
 #define LNT_OPAQUE(ptr) asm volatile("" : "+r"(ptr))
 #else
 #define LNT_SYNC() __syncthreads()
+// Orders the LDS accesses of one wave before and after it.  A wave's LDS instructions
+// complete in order, so only the compiler has to keep them so; no other wave is waited for.
+#define LNT_WAVE_SYNC()                                         \
+    do {                                                        \
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  \
+        __builtin_amdgcn_wave_barrier();                        \
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  \
+    } while (0)
 #define LNT_CHECK(cond, what) ((void)0)
 #define LNT_KFN __device__ __forceinline__
+// A value that is the same in every lane of the wave, as a scalar.
+#define LNT_UNIFORM(v) __builtin_amdgcn_readfirstlane(v)
 // Hide a (uniform) pointer's value from the optimiser so loads through it are not
 // hoisted out of a loop (which would pin whole tables in registers).
 #define LNT_OPAQUE(ptr) asm volatile("" : "+s"(ptr))

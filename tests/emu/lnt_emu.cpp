@@ -21,6 +21,7 @@ struct Emu {
     Plan pl;
     uint32_t p;
     bool prp, pending;
+    bool wide_rows = false;  // 4096-word rows with 16 waves instead of four
     std::vector<uint64_t> x, y, f, w, uw, tw4, itw4, twr, itwr, twr2, itwr2, twc, itwc, twc2, itwc2;
     std::vector<uint8_t> wid;
     LntParams P;
@@ -249,6 +250,16 @@ static void row3_sq(Emu *e, const LntParams &P, int mode) {
         });
 }
 
+template <int GW>
+static void row16_sq(Emu *e, const LntParams &P, int mode) {
+    for (uint32_t b = 0; b < e->pl.R; b++)
+        run_wg(1024 / GW, LNT_ROW16_LDS, [&](int tid, LView L) {
+            if (mode == LNT_FORWARD) lnt_row16_body<GW, LNT_FORWARD>(tid, b, L, P);
+            else if (mode == LNT_MULTIPLY) lnt_row16_body<GW, LNT_MULTIPLY>(tid, b, L, P);
+            else lnt_row16_body<GW>(tid, b, L, P);
+        });
+}
+
 template <int BA, int BB, int BC>
 static void row3m_sq(Emu *e, const LntParams &P, int mode) {
     const Plan &pl = e->pl;
@@ -325,7 +336,7 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
     if (pl.row3m == 32 && pl.rBB == 32 && pl.rBC == 16) row3m_sq<32, 32, 16>(e, P, mode), ok = true;
     if (pl.row3m == 16 && pl.rBB == 32 && pl.rBC == 16) row3m_sq<16, 32, 16>(e, P, mode), ok = true;
     if (pl.row3m == 16 && pl.rBB == 32 && pl.rBC == 32) row3m_sq<16, 32, 32>(e, P, mode), ok = true;
-    if (pl.row3 == 16) row3_sq<16, 1>(e, P, mode), ok = true;
+    if (pl.row3 == 16) (e->wide_rows ? row16_sq<1>(e, P, mode) : row16_sq<4>(e, P, mode)), ok = true;
     if (pl.row3 == 8) row3_sq<8, 4>(e, P, mode), ok = true;
 #define RW(b1, b2)                                                        \
     if (!ok && !pl.row3m && pl.row.B1 == b1 && pl.row.B2 == b2) {                      \
@@ -394,6 +405,7 @@ extern "C" void emu_set_digits(void *h, const uint64_t *d) {
     e->pending = false;
 }
 
+extern "C" void emu_wide_rows(void *h, int on) { ((Emu *)h)->wide_rows = on != 0; }
 extern "C" uint32_t emu_levels(void *h) { return ((Emu *)h)->pl.levels; }
 extern "C" uint32_t emu_secured(uint32_t p) { return secured_log2_length(p); }
 extern "C" uint32_t emu_carry_levels(uint32_t p, uint32_t n) { return carry_levels(p, n); }

@@ -120,6 +120,30 @@ def test_emulated_3phase_columns_match_oracle(p, n, lc, K):
     assert e.digits() == o.digits()
 
 
+def test_emulated_wide_4096_word_rows_match_oracle():
+    """4096-word rows on the matrix cores by 16 waves of one DFT group each (the CASES run them
+    by four waves): squarings, then a product through the forward and multiply modes."""
+    p, n = 1000003, 65536
+    rnd = random.Random(p + 16)
+    L = emu()
+    L.emu_mul.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    L.emu_wide_rows.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    o = OracleTest(p, n, True)
+    d = [rnd.getrandbits(wi) for wi in o.widths()]
+    o.set_digits(d)
+    e, f = Emu(p, n, True, 12), Emu(p, n, True, 12)
+    for t in (e, f):
+        L.emu_wide_rows(t.h, 1)
+        t.set_digits(d)
+    o.iterate(1)
+    e.iterate(1)
+    assert e.digits() == o.digits()
+    f.iterate(1)
+    assert L.emu_mul(e.h, f.h) == 0  # the square of the residue, as a product
+    o.iterate(1)
+    assert e.digits() == o.digits()
+
+
 @pytest.mark.parametrize("p,n", [(9689, 512), (86243, 4096)])
 def test_emulated_orbit_matches_gmp(p, n):
     g = golden(p, "LL")
@@ -156,6 +180,7 @@ def test_emulated_large_path_orbit_matches_oracle():
 
 @pytest.mark.parametrize("p,n,prp,lc", [(521, 32, True, 0), (9689, 512, False, 0), (86243, 4096, True, 0),
                                          (86243, 8192, True, 0), (400009, 32768, False, 0),
+                                         (1000003, 65536, True, 12), (1000003, 65536, False, 12),
                                          (1000003, 131072, True, 13), (1000003, 131072, False, -13)])
 def test_emulated_product_matches_python(p, n, prp, lc):
     """The forward / multiply kernel modes (used by the Gerbicz check): x <- x * y mod M_p
