@@ -947,119 +947,210 @@ LNT_KFN void lnt_small_body(int tid, LView lds, const LntParams &P, u32 iters, b
     for (int j = 0; j < B1; j++) P.x[(u64)t + B2 * j] = lds[(u32)(t + B2 * j)];
 }
 
-// ------------------------------------------------------------------ small residues, 3 phases
-// One workgroup of B^2 threads runs `iters` iterations on n = B^3 words (B = 16: 4096,
-// B = 8: 512), B words per thread in every phase (four waves at n = 4096 where the
-// 2-phase kernel runs one).  LDS: the residue in natural order (n words), then the
-// transform region (B * B * (B + 1) words, the 3-phase row layout).  MODEs as above.
-template <int B>
-constexpr u32 lnt_small3_lds() { return (u32)(B * B * B + B * B * (B + 1)); }
+// ------------------------------------------------------------------ small residues on the matrix cores
+// One workgroup of S waves runs `iters` iterations on n = 256 S words (S = 1, 2, 4, 8, 16), four
+// words per thread: n = 16 * 16 * S with the 16-point DFTs of mdft.hpp in phases 1 and 2 and an
+// S-point one in phase 3 (S = 2, 4 in registers, 8 and 16 on the matrix cores).  With
+// i = i1 + 16 S j, i1 = a + S b; wave w, lane (q, n), id = 16 w + n:
+//   phase 1: DFT i1 = id over j -> k2, twiddle omega_n^(i1 k2)                       (twr)
+//   phase 2: DFT (k2, a) = (id / S, id mod S) over b -> kb, twiddle omega_16S^(a kb) (twr2)
+//   phase 3: DFTs (k2, kb) over a, all k2 of one wave
+// One test is a chain of dependent steps on one compute unit, so what counts is its latency:
+// four words per thread put four times the waves of the former 16-word kernels to work on
+// it, a wave keeps its k2 from phase 2 to the inverse phase 2 (four barriers per iteration),
+// and up to S = 8 the factors of a thread's words stay in registers.  For n = 4096 that would
+// take more than the 128 registers of 16 waves: weights and twiddles are re-read (from the L2,
+// ahead of their use) and the unweights lie in LDS.
+// LDS: two regions, the residue (or its digits) in natural order in one while the other holds
+// the transform, runs of 16 words 18 apart as in the row kernel.  MODEs as above.
+template <int S>
+constexpr u32 lnt_small16_region() { return 288 * S; }
+template <int S>
+constexpr u32 lnt_small16_lds() { return 2 * lnt_small16_region<S>() + (S == 16 ? 256 * S : 0); }
 
-template <int B, int M, int MODE = LNT_SQUARE>
-LNT_KFN void lnt_small3_body(int tid, LView lds, const LntParams &P, u32 iters, bool sub2_first, bool ll) {
-    constexpr int T = B * B;
-    constexpr u32 N = B * B * B;
-    constexpr int RS = B * (B + 1);
-    constexpr u32 Z = N;  // transform region
-    const int t = tid, hi = t / B, lo = t % B;
+template <int S, int M, int MODE = LNT_SQUARE>
+LNT_KFN void lnt_small16_body(int tid, LView lds, const LntParams &P, u32 iters, bool sub2_first, bool ll) {
+    constexpr u32 N = 256 * S, L = 16 * S;
+    constexpr bool RES = S <= 8;                // factors live in registers
+    constexpr int KW = 16 / S;                  // k2 per wave
+    constexpr u32 U = 2 * lnt_small16_region<S>();  // unweights (S = 16)
+    const int w = LNT_UNIFORM(tid / 64);
+    int q = (tid % 64) / 16, n = tid % 16, id = 16 * w + n;
+    const u32 area = (u32)(288 * w);                // this wave's runs
+    // phase-3 layout of the wave's area: word (k2, kb, a)
+    auto p3 = [&](int k2l, int kb, int a) {
+        return area + (u32)(S == 16 ? 18 * kb + a : (16 * S + 2) * k2l + S * kb + a);
+    };
+    LntM16 Mx;
+    LntM8 M8;
+    lnt_m16_load(Mx, tid);
+    if (S == 8) lnt_m8_load(M8, Mx, tid);
+    u64 wv[4], wb[4], uv[4], tw1[4], itw1[4], tw2[4], itw2[4];
+    const u64 r2 = gl_mul(GL_R, GL_R);
+    // phase-3 places of this thread: S = 16 (w, kb = n, a = -word(q, v)), S = 8 (2w + g, n, -(2q + v)),
+    // S = 4 (4w + q, n, v), S = 2 (8w + 2q + c, n, v)
+    auto p3a = [&](int v) { return S == 16 ? (16 - lnt_m16_word(q, v)) & 15 : S == 8 ? (8 - 2 * q - (v & 1)) & 7 : S == 4 ? v : v & 1; };
+    auto load_w = [&]() {
 #pragma unroll
-    for (int j = 0; j < B; j++) lds[(u32)(t + T * j)] = P.x[(u64)t + T * j];
-    LNT_SYNC();
-    for (u32 it = 0; it < iters; it++) {
-        // tables re-read each iteration (from cache) instead of living in registers
-        const u64 *pw = P.w.p, *puw = P.uw.p, *ptw = P.twr.p, *pitw = P.itwr.p, *ptw2 = P.twr2.p,
-                  *pitw2 = P.itwr2.p;
-        LNT_OPAQUE(pw);
-        LNT_OPAQUE(puw);
-        LNT_OPAQUE(ptw);
-        LNT_OPAQUE(pitw);
-        LNT_OPAQUE(ptw2);
-        LNT_OPAQUE(pitw2);
-        const GView<const u64> Tw{pw, P.w.n}, Tuw{puw, P.uw.n}, Ttw{ptw, P.twr.n}, Titw{pitw, P.itwr.n},
-            Ttw2{ptw2, P.twr2.n}, Titw2{pitw2, P.itwr2.n};
-        // carry over this thread's chunk [t*B, (t+1)*B); halo = the M pre-carry words before it
-        {
-            const u32 g0 = (u32)t * B;
-            int64_t v[M + B];
-#pragma unroll
-            for (int j = 0; j < M; j++) v[j] = gl_to_i64(lds[(g0 + N - M + j) & (N - 1)]);
-#pragma unroll
-            for (int j = 0; j < B; j++) v[M + j] = gl_to_i64(lds[g0 + j]);
-            LNT_SYNC();  // every halo read before any chunk is overwritten
-            lnt_carry_run<M, B>(v, P.p, P.log_n, g0, P.levels, it == 0 ? sub2_first : ll);
-#pragma unroll
-            for (int j = 0; j < B; j++)
-                lds[g0 + j] = P.bias ? (u64)(u32)(v[M + j] + (int64_t(1) << 31)) : gl_from_i64(v[M + j]);
-            LNT_SYNC();
+        for (int e = 0; e < 4; e++) {
+            const u32 i = (u32)id + L * lnt_m16_word(q, e);
+            wv[e] = P.w[2 * i];
+            wb[e] = P.w[2 * i + 1];
         }
-        u64 a[B];
-        // phase 1: weight, B-point DFT over j (stride T), twiddle w_n^(t k1)
+    };
+    auto load_tw1 = [&]() {
 #pragma unroll
-        for (int j = 0; j < B; j++) {
-            const u32 i = (u32)(t + T * j);
-            a[j] = P.bias ? gl_mul_biased((u32)lds[i], Tw[2 * i], Tw[2 * i + 1]) : gl_mul(lds[i], Tw[2 * i]);
-        }
-        dft_fwd<B>(a);
+        for (int e = 0; e < 4; e++) tw1[e] = P.twr[L * brev_v16(lnt_m16_word(q, e)) + id];
+    };
+    auto load_tw2 = [&]() {
+        if (S == 1) return;
 #pragma unroll
-        for (int rho = 1; rho < B; rho++) a[rho] = gl_mmul(a[rho], Ttw[(u64)rho * T + t]);
+        for (int e = 0; e < 4; e++) tw2[e] = P.twr2[S * brev_v16(lnt_m16_word(q, e)) + id % S];
+    };
+    auto load_itw2 = [&]() {
+        if (S == 1) return;
 #pragma unroll
-        for (int rho = 0; rho < B; rho++) lds[Z + (u32)(brev_c<B>(rho) * RS + hi * (B + 1) + lo)] = a[rho];
-        LNT_SYNC();
-        // phase 2: thread (hi, lo) over the middle index
+        for (int v = 0; v < 4; v++) itw2[v] = P.itwr2[S * brev_v16(n) + p3a(v)];
+    };
+    auto load_itw1 = [&]() {
 #pragma unroll
-        for (int b = 0; b < B; b++) a[b] = lds[Z + (u32)(hi * RS + b * (B + 1) + lo)];
-        dft_fwd<B>(a);
-#pragma unroll
-        for (int rho = 1; rho < B; rho++) a[rho] = gl_mmul(a[rho], Ttw2[(u64)rho * B + lo]);
-#pragma unroll
-        for (int rho = 0; rho < B; rho++) lds[Z + (u32)(hi * RS + brev_c<B>(rho) * (B + 1) + lo)] = a[rho];
-        LNT_SYNC();
-        // phase 3, pointwise square (or product), inverse phase 3
-#pragma unroll
-        for (int i = 0; i < B; i++) a[i] = lds[Z + (u32)(hi * RS + lo * (B + 1) + i)];
-        dft_fwd<B>(a);
-        if (MODE == LNT_FORWARD) {
-#pragma unroll
-            for (int i = 0; i < B; i++) P.y[(u64)t * B + i] = a[i];
-            return;
-        }
-        if (MODE == LNT_MULTIPLY) {
-#pragma unroll
-            for (int i = 0; i < B; i++) a[i] = gl_mul(a[i], P.f[(u64)t * B + i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < B; i++) a[i] = gl_sqr(a[i]);
-        }
-        dft_inv<B>(a);
-#pragma unroll
-        for (int i = 0; i < B; i++) lds[Z + (u32)(hi * RS + lo * (B + 1) + i)] = a[i];
-        LNT_SYNC();
-        // inverse phase 2
-#pragma unroll
-        for (int rho = 0; rho < B; rho++) {
-            u64 v = lds[Z + (u32)(hi * RS + brev_c<B>(rho) * (B + 1) + lo)];
-            a[rho] = rho ? gl_mmul(v, Titw2[(u64)rho * B + lo]) : v;
-        }
-        dft_inv<B>(a);
-#pragma unroll
-        for (int b = 0; b < B; b++) lds[Z + (u32)(hi * RS + b * (B + 1) + lo)] = a[b];
-        LNT_SYNC();
-        // inverse phase 1, unweight, back to the residue region
-#pragma unroll
-        for (int rho = 0; rho < B; rho++) {
-            u64 v = lds[Z + (u32)(brev_c<B>(rho) * RS + hi * (B + 1) + lo)];
-            a[rho] = rho ? gl_mmul(v, Titw[(u64)rho * T + t]) : v;
-        }
-        dft_inv<B>(a);
-#pragma unroll
-        for (int j = 0; j < B; j++) {
-            const u32 i = (u32)(t + T * j);
-            lds[i] = gl_mul(a[j], Tuw[i]);
-        }
-        LNT_SYNC();
+        for (int v = 0; v < 4; v++)
+            itw1[v] = P.itwr[L * brev_v16(id / S) + id % S + S * ((16 - lnt_m16_word(q, v)) & 15)];
+    };
+    if (RES) {
+        load_w();
+        load_tw1();
+        load_tw2();
+        load_itw2();
+        load_itw1();
     }
 #pragma unroll
-    for (int j = 0; j < B; j++) P.x[(u64)t + T * j] = lds[(u32)(t + T * j)];
+    for (int v = 0; v < 4; v++) {
+        // unweight of output place v, times 2^128: one 2^64 for its Montgomery multiply and one
+        // for the factor 2^-64 that the pointwise product leaves
+        const u32 i = (u32)id + L * ((16 - lnt_m16_word(q, v)) & 15);
+        const u64 u = gl_mul(P.uw[i], r2);
+        if (RES) uv[v] = u;
+        else lds[U + i] = u;
+    }
+    u32 A = 0, B = lnt_small16_region<S>();
+#pragma unroll
+    for (int j = 0; j < 4; j++) lds[A + (u32)(tid + 64 * S * j)] = P.x[(u64)tid + 64 * S * j];
+    LNT_SYNC();
+    for (u32 it = 0; it < iters; it++) {
+        if (!RES) {
+            LNT_OPAQUE_LANE(tid);
+            n = tid % 16, q = (tid % 64) / 16, id = 16 * w + n;
+        }
+        const u32 t1 = (u32)(18 * (id % S) + id / S);  // place of i1 = id within a k2 of the transform region
+        const u32 own = (u32)(18 * id + 2 * q);        // this lane's words of run id
+        // carry of digits 4 tid .. 4 tid + 3 from the M pre-carry words before them on: A -> B
+        {
+            const u32 g0 = 4 * (u32)tid;
+            int64_t v[M + 4];
+#pragma unroll
+            for (int j = 0; j < M; j++) v[j] = gl_to_i64(lds[A + ((g0 + N - M + j) & (N - 1))]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[M + j] = gl_to_i64(lds[A + g0 + j]);
+            lnt_carry_run<M, 4>(v, P.p, P.log_n, g0, P.levels, it == 0 ? sub2_first : ll);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                lds[B + g0 + j] = P.bias ? (u64)(u32)(v[M + j] + (int64_t(1) << 31)) : gl_from_i64(v[M + j]);
+        }
+        if (!RES) {
+            load_w();
+            load_tw1();
+        }
+        LNT_SYNC();
+        u64 z[4];
+        // phase 1: weight, DFT over j, twiddle: B -> A
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const u64 d = lds[B + (u32)id + L * lnt_m16_word(q, e)];
+            z[e] = P.bias ? gl_mul_biased((u32)d, wv[e], wb[e]) : gl_mul(d, wv[e]);
+        }
+        lnt_m16_dft(Mx, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) lds[A + (u32)(18 * S * lnt_m16_word(q, v)) + t1] = gl_mmul(z[v], tw1[v]);
+        if (!RES) load_tw2();
+        LNT_SYNC();
+        // phase 2
+#pragma unroll
+        for (int e = 0; e < 4; e++) z[e] = lds[A + own + lnt_m16_word(0, e)];
+        LNT_WAVE_SYNC();
+        lnt_m16_dft(Mx, z);
+        if (S > 1) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) lds[A + p3(n / S, lnt_m16_word(q, v), n % S)] = gl_mmul(z[v], tw2[v]);
+            if (!RES && MODE != LNT_FORWARD) load_itw2();
+            LNT_WAVE_SYNC();
+            // phase 3
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                z[v] = lds[A + (S == 16  ? p3(0, n, 2 * q) + lnt_m16_word(0, v)
+                                : S == 8 ? p3(v / 2, n, 2 * q + v % 2)
+                                : S == 4 ? p3(q, n, v)
+                                         : p3(2 * q + v / 2, n, v % 2))];
+            LNT_WAVE_SYNC();
+        }
+        auto transform3 = [&](bool inverse) {
+            if (S == 16) lnt_m16_dft(Mx, z);
+            if (S == 8) {
+                u64 h[2] = {z[0], z[1]}, g[2] = {z[2], z[3]};
+                lnt_m8_dft(M8, Mx, h);
+                lnt_m8_dft(M8, Mx, g);
+                z[0] = h[0], z[1] = h[1], z[2] = g[0], z[3] = g[1];
+            }
+            if (S == 4) inverse ? dft_inv<4>(z) : dft_fwd<4>(z);
+            if (S == 2) {
+                inverse ? dft_inv<2>(z) : dft_fwd<2>(z);
+                inverse ? dft_inv<2>(z + 2) : dft_fwd<2>(z + 2);
+            }
+        };
+        transform3(false);
+        // pointwise
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (MODE == LNT_FORWARD) P.y[4 * (u64)tid + v] = z[v];
+            else z[v] = gl_mmul(z[v], MODE == LNT_MULTIPLY ? P.f[4 * (u64)tid + v] : z[v]);
+        }
+        if (MODE == LNT_FORWARD) return;
+        if (S > 1) {
+            transform3(true);
+            if (!RES) load_itw1();
+            // inverse phase-2 twiddle; runs (k2, a) of words kb again
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int k2l = S == 16 ? 0 : S == 8 ? v / 2 : S == 4 ? q : 2 * q + v / 2;
+                lds[A + area + (u32)(18 * (S * (k2l % KW) + p3a(v)) + n)] = gl_mmul(z[v], itw2[v]);
+            }
+            LNT_WAVE_SYNC();
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[e] = lds[A + own + lnt_m16_word(0, e)];
+            LNT_WAVE_SYNC();
+        }
+        // inverse phase 2: output place v is b = -k
+        lnt_m16_dft(Mx, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[A + (u32)(18 * id + ((16 - lnt_m16_word(q, v)) & 15))] = gl_mmul(z[v], itw1[v]);
+        LNT_SYNC();
+        // inverse phase 1, unweight: A -> B
+#pragma unroll
+        for (int e = 0; e < 4; e++) z[e] = lds[A + (u32)(18 * S * lnt_m16_word(q, e)) + t1];
+        lnt_m16_dft(Mx, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const u32 i = (u32)id + L * ((16 - lnt_m16_word(q, v)) & 15);
+            lds[B + i] = gl_mmul(z[v], RES ? uv[v] : lds[U + i]);
+        }
+        LNT_SYNC();
+        const u32 c = A;
+        A = B;
+        B = c;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) P.x[(u64)tid + 64 * S * j] = lds[A + (u32)(tid + 64 * S * j)];
 }
 
 // ------------------------------------------------------------------ tables

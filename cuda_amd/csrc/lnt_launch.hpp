@@ -23,11 +23,11 @@ __global__ __launch_bounds__(B2 < 64 ? 64 : B2) void lnt_k_small(LntParams P, u3
     lnt_small_body<B1, B2, M, MODE>(threadIdx.x, LView{smem, W}, P, iters, sub2_first != 0, ll != 0);
 }
 
-template <int B, int M, int MODE>
-__global__ __launch_bounds__(B * B) void lnt_k_small3(LntParams P, u32 iters, int sub2_first, int ll) {
-    constexpr u32 W = lnt_small3_lds<B>();
-    __shared__ u64 smem[W];
-    lnt_small3_body<B, M, MODE>(threadIdx.x, LView{smem, W}, P, iters, sub2_first != 0, ll != 0);
+template <int S, int M, int MODE>
+__global__ __launch_bounds__(64 * S) void lnt_k_small16(LntParams P, u32 iters, int sub2_first, int ll) {
+    constexpr u32 W = lnt_small16_lds<S>();
+    __shared__ __align__(16) u64 smem[W];
+    lnt_small16_body<S, M, MODE>(threadIdx.x, LView{smem, W}, P, iters, sub2_first != 0, ll != 0);
 }
 
 template <int B1, int B2, int K, int M>
@@ -107,13 +107,13 @@ __global__ __launch_bounds__(B2 < 64 ? 64 : B2) void lnt_kb_small(const LntParam
     lnt_small_body<B1, B2, M>(threadIdx.x, LView{smem, W}, P, iters, P.sub2 != 0, ll != 0);
 }
 
-template <int B, int M>
-__global__ __launch_bounds__(B * B) void lnt_kb_small3(const LntParams *__restrict__ Ps, u32 iters, int ll) {
-    constexpr u32 W = lnt_small3_lds<B>();
-    __shared__ u64 smem[W];
+template <int S, int M>
+__global__ __launch_bounds__(64 * S) void lnt_kb_small16(const LntParams *__restrict__ Ps, u32 iters, int ll) {
+    constexpr u32 W = lnt_small16_lds<S>();
+    __shared__ __align__(16) u64 smem[W];
     const LntParams P = Ps[blockIdx.x];
     if (P.n == 0) return;  // an empty slot of the batch
-    lnt_small3_body<B, M>(threadIdx.x, LView{smem, W}, P, iters, P.sub2 != 0, ll != 0);
+    lnt_small16_body<S, M>(threadIdx.x, LView{smem, W}, P, iters, P.sub2 != 0, ll != 0);
 }
 
 template <int B1, int B2, int K, int M>

@@ -65,7 +65,7 @@ static TableSizes table_sizes(const Plan &pl) {
     t.n = pl.n;
     t.large = !pl.small;
     t.Lr = pl.small ? pl.n : pl.C;
-    t.L2 = pl.row3m ? pl.rBB * pl.rBC : pl.row3 ? pl.row3 * pl.row3 : 0;
+    t.L2 = pl.small16 > 1 ? 16 * pl.small16 : pl.row3m ? pl.rBB * pl.rBC : pl.row3 ? pl.row3 * pl.row3 : 0;
     t.R = pl.small ? 0 : pl.R;
     t.A = (!pl.small && pl.col3) ? pl.R / pl.col3 : 0;
     t.W = pl.small ? 2 * pl.n : 4 * pl.R;
@@ -93,9 +93,13 @@ static void fill_tables(const Plan &pl, u32 p, const TablePtrs &t, hipStream_t s
         hipLaunchKernelGGL(lnt_k_weights, dim3((n + 255) / 256), dim3(256), 0, s, Bw, Binv, ninv, p, n, t.w, t.uw);
     const u32 Lr = z.Lr;
     u64 omr = gl_pow(554, (GL_P - 1) / Lr);
-    // row line twiddles: first phase B1 x B2 (3-phase rows: row3 x row3^2, row3m x rBB rBC)
-    const u32 rB1 = pl.row3m ? pl.row3m : pl.row3 ? pl.row3 : pl.row.B1;
-    const u32 rB2 = pl.row3m ? pl.rBB * pl.rBC : pl.row3 ? pl.row3 * pl.row3 : pl.row.B2;
+    // row line twiddles: first phase B1 x B2 (3-phase rows: row3 x row3^2, row3m x rBB rBC;
+    // one workgroup on the matrix cores: 16 x 16 small16)
+    const u32 rB1 = pl.small16 ? 16 : pl.row3m ? pl.row3m : pl.row3 ? pl.row3 : pl.row.B1;
+    const u32 rB2 = pl.small16 ? 16 * pl.small16
+                    : pl.row3m ? pl.rBB * pl.rBC
+                    : pl.row3  ? pl.row3 * pl.row3
+                               : pl.row.B2;
     hipLaunchKernelGGL(lnt_k_line_tw, dim3((Lr + 255) / 256), dim3(256), 0, s, omr, rB1, rB2, Lr, t.twr);
     hipLaunchKernelGGL(lnt_k_line_tw, dim3((Lr + 255) / 256), dim3(256), 0, s, gl_inv(omr), rB1, rB2, Lr, t.itwr);
     if (z.large) {
@@ -126,9 +130,11 @@ static void fill_tables(const Plan &pl, u32 p, const TablePtrs &t, hipStream_t s
                                pl.col.B2, n, Binv, ninv, p, t.itw4);
         }
     }
-    // second-phase row twiddles: a line of L2 = B2 words split (row3 x row3 or rBB x rBC)
+    // second-phase row twiddles: a line of L2 = B2 words split (row3 x row3, rBB x rBC or
+    // 16 x small16)
     if (z.L2) {
-        const u32 s1 = pl.row3m ? pl.rBB : pl.row3, s2 = pl.row3m ? pl.rBC : pl.row3;
+        const u32 s1 = pl.small16 ? 16 : pl.row3m ? pl.rBB : pl.row3;
+        const u32 s2 = pl.small16 ? pl.small16 : pl.row3m ? pl.rBC : pl.row3;
         u64 om2 = gl_pow(554, (GL_P - 1) / z.L2);
         hipLaunchKernelGGL(lnt_k_line_tw, dim3((z.L2 + 255) / 256), dim3(256), 0, s, om2, s1, s2, z.L2, t.twr2);
         hipLaunchKernelGGL(lnt_k_line_tw, dim3((z.L2 + 255) / 256), dim3(256), 0, s, gl_inv(om2), s1, s2, z.L2,

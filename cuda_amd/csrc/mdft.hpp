@@ -41,6 +41,23 @@ constexpr int LNT_M16_TILES = 12;
 struct LntM16Table {
     signed char b[LNT_M16_TILES * 64 * 16];
 };
+// The same for 8-point DFTs (omega_8 = 2^24, every entry 0 or +-1): lane (q, n) holds the words
+// 2q, 2q+1 of DFT n, one matrix instruction per tile (v, h).
+constexpr int LNT_M8_TILES = 4;
+struct LntM8Table {
+    signed char b[LNT_M8_TILES * 64 * 16];
+};
+constexpr LntM8Table lnt_m8_make() {
+    LntM8Table t{};
+    for (int tile = 0; tile < LNT_M8_TILES; tile++)
+        for (int lane = 0; lane < 64; lane++)
+            for (int byte = 0; byte < 16; byte++) {
+                const int row = lane % 16, k = 2 * (row / 4) + tile / 2, limb = 4 * (tile % 2) + row % 4;
+                const int j = 2 * (lane / 16) + byte / 8;
+                t.b[(tile * 64 + lane) * 16 + byte] = (signed char)lnt_m16_entry(limb, 2 * k, j, byte % 8);
+            }
+    return t;
+}
 constexpr LntM16Table lnt_m16_make() {
     LntM16Table t{};
     for (int tile = 0; tile < LNT_M16_TILES; tile++) {
@@ -86,6 +103,7 @@ GL_HD u32 lnt_limbs(const int (&l)[8], u64 dc, u32 k16, int km1, u32 &lo, u32 &t
 }
 
 constexpr u64 LNT_M16_DC = 2048ull * 0x01010101ull;  // 2048 R = DC + 2^32 DC
+constexpr u64 LNT_M8_DC = 1024ull * 0x01010101ull;   // 8 points: 1024 R
 
 #if defined(LNT_EMU)
 // Emulation: the words of a wave meet in an array between two barriers, and the sums run over
@@ -119,6 +137,34 @@ LNT_KFN void lnt_m16_dft(const LntM16 &M, u64 (&x)[4]) {
         }
         u32 lo, t;
         const u32 v0 = v == 0 ? lnt_limbs<true>(l, q == 0 ? LNT_M16_DC : 0, 65536, -1, lo, t)
+                              : lnt_limbs<false>(l, 0, 65536, -1, lo, t);
+        const u64 hi = (u64)v0 + t;
+        x[v] = ((hi << 32) | lo) + (hi >> 32 ? GL_EPS : 0);
+    }
+    LNT_SYNC();
+}
+static const LntM8Table lnt_m8_tab = lnt_m8_make();
+struct LntM8 {
+    int tid;
+};
+LNT_KFN void lnt_m8_load(LntM8 &M, const LntM16 &, int tid) { M.tid = tid; }
+LNT_KFN void lnt_m8_dft(const LntM8 &M, const LntM16 &, u64 (&x)[2]) {
+    const int tid = M.tid, q = (tid % 64) / 16, wb = tid & ~63, n = tid % 16;
+    for (int e = 0; e < 2; e++) lnt_emu_wave[tid][e] = x[e] ^ 0x8080808080808080ull;
+    LNT_SYNC();
+    for (int v = 0; v < 2; v++) {
+        int l[8];
+        for (int limb = 0; limb < 8; limb++) {
+            int sum = 0;
+            for (int qq = 0; qq < 4; qq++)
+                for (int byte = 0; byte < 16; byte++)
+                    sum += lnt_m8_tab.b[((2 * v + limb / 4) * 64 + 16 * qq + 4 * q + limb % 4) * 16 + byte] *
+                           (int)(signed char)(lnt_emu_wave[wb + 16 * qq + n][byte / 8] >> (8 * (byte % 8)));
+            l[limb] = sum + lnt_m16_offset(limb);
+            LNT_CHECK(l[limb] > 0 && l[limb] < 1 << 18, "limb range");
+        }
+        u32 lo, t;
+        const u32 v0 = v == 0 ? lnt_limbs<true>(l, q == 0 ? LNT_M8_DC : 0, 65536, -1, lo, t)
                               : lnt_limbs<false>(l, 0, 65536, -1, lo, t);
         const u64 hi = (u64)v0 + t;
         x[v] = ((hi << 32) | lo) + (hi >> 32 ? GL_EPS : 0);
@@ -179,6 +225,45 @@ LNT_KFN void lnt_m16_dft(const LntM16 &M, u64 (&x)[4]) {
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(c[0] | c[1] | c[2] | c[3]) != 0, 0)) {
 #pragma unroll
         for (int v = 0; v < 4; v++) x[v] += c[v] ? GL_EPS : 0;
+    }
+}
+
+static __device__ const LntM8Table lnt_m8_tab = lnt_m8_make();
+struct LntM8 {
+    lnt_v4i t[LNT_M8_TILES];
+    u64 dc;
+};
+LNT_KFN void lnt_m8_load(LntM8 &M, const LntM16 &, int tid) {
+    const int lane = tid & 63;
+#pragma unroll
+    for (int i = 0; i < LNT_M8_TILES; i++)
+        M.t[i] = *reinterpret_cast<const lnt_v4i *>(&lnt_m8_tab.b[(i * 64 + lane) * 16]);
+    M.dc = lane < 16 ? LNT_M8_DC : 0;
+}
+// The two words of this lane's 8-point DFT, in place; the offsets and constants are M16's.
+LNT_KFN void lnt_m8_dft(const LntM8 &M, const LntM16 &M16, u64 (&x)[2]) {
+    lnt_v4i b;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        b[2 * i] = (int)((u32)x[i] ^ 0x80808080u);
+        b[2 * i + 1] = (int)((u32)(x[i] >> 32) ^ 0x80808080u);
+    }
+    bool c[2];
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+        lnt_v4i d[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) d[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(M.t[2 * v + h], b, M16.o[h], 0, 0, 0);
+        const int l[8] = {d[0][0], d[0][1], d[0][2], d[0][3], d[1][0], d[1][1], d[1][2], d[1][3]};
+        u32 lo, t, hi;
+        const u32 v0 = v == 0 ? lnt_limbs<true>(l, M.dc, M16.k16, M16.km1, lo, t)
+                              : lnt_limbs<false>(l, 0, M16.k16, M16.km1, lo, t);
+        c[v] = __builtin_add_overflow(v0, t, &hi);
+        x[v] = ((u64)hi << 32) | lo;
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(c[0] | c[1]) != 0, 0)) {
+#pragma unroll
+        for (int v = 0; v < 2; v++) x[v] += c[v] ? GL_EPS : 0;
     }
 }
 #endif

@@ -22,6 +22,7 @@
 #define LNT_KFN static inline
 #define LNT_UNIFORM(v) (v)
 #define LNT_OPAQUE(ptr) asm volatile("" : "+r"(ptr))
+#define LNT_OPAQUE_LANE(v) ((void)0)
 #else
 #define LNT_SYNC() __syncthreads()
 // Orders the LDS accesses of one wave before and after it.  A wave's LDS instructions
@@ -39,6 +40,9 @@
 // Hide a (uniform) pointer's value from the optimiser so loads through it are not
 // hoisted out of a loop (which would pin whole tables in registers).
 #define LNT_OPAQUE(ptr) asm volatile("" : "+s"(ptr))
+// The same for a per-lane integer: addresses made from it are formed again in each iteration
+// of a loop instead of occupying registers across it.
+#define LNT_OPAQUE_LANE(v) asm volatile("" : "+v"(v))
 #endif
 
 // Global-memory and LDS views carrying their length so the emulation can check.

@@ -80,7 +80,14 @@ extern "C" void *emu_create3(uint32_t p, uint32_t n, int prp, uint32_t lc, uint3
         for (uint32_t i = 0; i < 2 * pl.R; i++) e->uw[i] = lnt_row_factor(Binv, 2, p, n, pl.C, i);
     }
     widths(p, n, e->wid);
-    if (pl.row3m) {
+    if (pl.small16) {
+        Line l1, l2;
+        l1.B1 = l2.B1 = 16;
+        l1.B2 = n / 16;
+        l2.B2 = pl.small16;
+        line_tables(n, l1, e->twr, e->itwr);
+        line_tables(16 * pl.small16, l2, e->twr2, e->itwr2);
+    } else if (pl.row3m) {
         Line l1, l2;
         l1.B1 = pl.row3m;
         l1.B2 = pl.rBB * pl.rBC;
@@ -189,21 +196,22 @@ static void small_iter(Emu *e, uint32_t k, const LntParams &P, bool sub2) {
     run_wg(B2, lds, [&](int tid, LView L) { lnt_small_body<B1, B2, M, MODE>(tid, L, P, k, sub2, !e->prp); });
 }
 
-template <int B, int M, int MODE = LNT_SQUARE>
-static void small3_iter(Emu *e, uint32_t k, const LntParams &P, bool sub2) {
-    run_wg(B * B, lnt_small3_lds<B>(), [&](int tid, LView L) { lnt_small3_body<B, M, MODE>(tid, L, P, k, sub2, !e->prp); });
+template <int S, int M, int MODE = LNT_SQUARE>
+static void small16_iter(Emu *e, uint32_t k, const LntParams &P, bool sub2) {
+    run_wg(64 * S, lnt_small16_lds<S>(),
+           [&](int tid, LView L) { lnt_small16_body<S, M, MODE>(tid, L, P, k, sub2, !e->prp); });
 }
 
-template <int B>
-static void small3_any(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mode) {
+template <int S>
+static void small16_any(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mode) {
     if (mode == LNT_FORWARD) {
-        if (e->pl.M == 4) small3_iter<B, 4, LNT_FORWARD>(e, 1, P, sub2);
-        else small3_iter<B, 8, LNT_FORWARD>(e, 1, P, sub2);
+        if (e->pl.M == 4) small16_iter<S, 4, LNT_FORWARD>(e, 1, P, sub2);
+        else small16_iter<S, 8, LNT_FORWARD>(e, 1, P, sub2);
     } else if (mode == LNT_MULTIPLY) {
-        if (e->pl.M == 4) small3_iter<B, 4, LNT_MULTIPLY>(e, 1, P, sub2);
-        else small3_iter<B, 8, LNT_MULTIPLY>(e, 1, P, sub2);
-    } else if (e->pl.M == 4) small3_iter<B, 4>(e, k, P, sub2);
-    else small3_iter<B, 8>(e, k, P, sub2);
+        if (e->pl.M == 4) small16_iter<S, 4, LNT_MULTIPLY>(e, 1, P, sub2);
+        else small16_iter<S, 8, LNT_MULTIPLY>(e, 1, P, sub2);
+    } else if (e->pl.M == 4) small16_iter<S, 4>(e, k, P, sub2);
+    else small16_iter<S, 8>(e, k, P, sub2);
 }
 
 template <int B1, int B2, int K, int M>
@@ -286,8 +294,11 @@ static void row_sq(Emu *e, const LntParams &P, int mode) {
 // Dispatch tables for the emulated sizes (a subset of the HIP build's).
 static bool run_small(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mode = LNT_SQUARE) {
     const Plan &pl = e->pl;
-    if (pl.row3 == 16) return small3_any<16>(e, k, P, sub2, mode), true;
-    if (pl.row3 == 8) return small3_any<8>(e, k, P, sub2, mode), true;
+    if (pl.small16 == 16) return small16_any<16>(e, k, P, sub2, mode), true;
+    if (pl.small16 == 8) return small16_any<8>(e, k, P, sub2, mode), true;
+    if (pl.small16 == 4) return small16_any<4>(e, k, P, sub2, mode), true;
+    if (pl.small16 == 2) return small16_any<2>(e, k, P, sub2, mode), true;
+    if (pl.small16 == 1) return small16_any<1>(e, k, P, sub2, mode), true;
 #define SM(b1, b2)                                                                          \
     if (pl.row.B1 == b1 && pl.row.B2 == b2) {                                               \
         if (mode == LNT_FORWARD) {                                                          \
