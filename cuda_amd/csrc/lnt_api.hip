@@ -187,6 +187,9 @@ static void drop_graph(lnt_ctx *c) {
 // Iterations per replay of the captured iteration graph.
 static constexpr uint32_t GRAPH_ITERS = 16;
 
+// Iterations per launch of a single-workgroup kernel, so that each launch stays short.
+static uint32_t small_chunk(const Plan &pl) { return pl.n >= 2048 ? 256 : 1024; }
+
 static bool launch_iteration(const Plan &pl, const LntParams &P, bool sub2, hipStream_t s) {
     return lnt_launch_col_fwd(pl, P, sub2, s) && lnt_launch_row(pl, P, s) && lnt_launch_col_inv(pl, P, s);
 }
@@ -220,8 +223,7 @@ static int square_buf(lnt_ctx *c, u64 *x, bool &pending, uint32_t k) {
     const bool ll = !c->prp;
     const LntParams P = params_for(c, x, c->y, nullptr);
     if (pl.small) {
-        // bounded launches keep each kernel short
-        const uint32_t chunk = pl.n >= 2048 ? 256 : 1024;
+        const uint32_t chunk = small_chunk(pl);
         while (k) {
             uint32_t s = k < chunk ? k : chunk;
             if (!lnt_launch_small(pl, P, s, ll && pending, ll, c->stream))
@@ -1022,8 +1024,11 @@ int lnt_gerbicz_stats(lnt_ctx *c, uint64_t *out, int cap) {
 // ------------------------------------------------------------------ batches
 // Many independent tests advanced together: members with the same plan shape form a
 // group that runs as one batched launch per kernel (per-test parameters in a device
-// array); one iteration of every group is captured as a hipGraph whose groups are
-// parallel branches, and each lnt_batch_iterate step replays it.
+// array).  Groups do not wait for each other inside a step: each runs its iterations on a
+// stream of its own, single-workgroup groups as one launch that loops over them, the others
+// as replays of a captured graph of GRAPH_ITERS iterations and the remainder one by one.
+// (Stepping all groups together, one graph launch per iteration with the groups as its
+// branches, spent 97 us per iteration on 24 tests of 2^11 .. 2^14 words.)
 
 struct lnt_batch {
     int device = 0;
@@ -1042,15 +1047,15 @@ struct lnt_batch {
         LntParams *d = nullptr;
         hipStream_t side = nullptr;
         hipEvent_t join = nullptr;
+        hipGraph_t graph = nullptr;  // GRAPH_ITERS iterations (not for single-workgroup tests)
+        hipGraphExec_t exec = nullptr;
     };
     std::vector<Group> groups;
     hipEvent_t fork = nullptr;
     hipEvent_t done = nullptr;  // end of the last batch_iterate: members' streams wait on it
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    bool dirty = true;      // the groups or their capacities changed: capture a new graph
+    bool dirty = true;      // the groups or their capacities changed: capture new graphs
     bool upload = false;    // parameters changed: copy them to the device before the next step
-    uint64_t captures = 0;  // graphs captured so far
+    uint64_t captures = 0;  // times the groups' graphs were captured
     std::string err;
 };
 
@@ -1072,11 +1077,10 @@ static int bfail(lnt_batch *b, int code, const std::string &m) {
 static bool same_group(const Plan &a, const Plan &b) { return same_kernels(a, b); }
 
 static void batch_release(lnt_batch *b) {
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
     for (auto &g : b->groups) {
+        if (g.side) (void)hipStreamSynchronize(g.side);
+        if (g.exec) (void)hipGraphExecDestroy(g.exec);
+        if (g.graph) (void)hipGraphDestroy(g.graph);
         if (g.d) (void)hipFree(g.d);
         if (g.side) (void)hipStreamDestroy(g.side);
         if (g.join) (void)hipEventDestroy(g.join);
@@ -1084,11 +1088,11 @@ static void batch_release(lnt_batch *b) {
     b->groups.clear();
 }
 
-// Launch one iteration of group g on stream s (all cap slots; empty ones return at once).
-static bool batch_group_step(lnt_batch::Group &g, hipStream_t s) {
-    if (g.pl.small) return lnt_launch_batch_small(g.pl, g.d, g.cap, 1, g.ll, s);
-    return lnt_launch_batch_col_fwd(g.pl, g.d, g.cap, s) && lnt_launch_batch_row(g.pl, g.d, g.cap, s) &&
-           lnt_launch_batch_col_inv(g.pl, g.d, g.cap, s);
+// Launch one iteration of the row/column group g on its stream (all cap slots; empty ones
+// return at once).
+static bool batch_group_step(lnt_batch::Group &g) {
+    return lnt_launch_batch_col_fwd(g.pl, g.d, g.cap, g.side) && lnt_launch_batch_row(g.pl, g.d, g.cap, g.side) &&
+           lnt_launch_batch_col_inv(g.pl, g.d, g.cap, g.side);
 }
 
 // The parameter block of member c in a batch launch (its "-2" flag from its own state).
@@ -1105,8 +1109,7 @@ static lnt_batch::Group *group_of(lnt_batch *b, const lnt_ctx *c) {
 }
 
 // Groups for the current members, each with room to grow (at least 8 slots, a power of
-// two, at least twice its members), their parameters, streams and the captured graph of
-// one iteration (every group a parallel branch forked from and joined to the batch stream).
+// two, at least twice its members), their parameters, streams and captured graphs.
 static int batch_build(lnt_batch *b) {
     batch_release(b);
     for (lnt_ctx *c : b->members) {
@@ -1128,35 +1131,26 @@ static int batch_build(lnt_batch *b) {
         for (u32 i = 0; i < cap; i++)
             if (g.ctxs[i]) g.h[i] = member_params(g.ctxs[i]);
         BHIPCHK(b, hipMalloc(&g.d, g.h.size() * sizeof(LntParams)), "hipMalloc (batch parameters)");
-        BHIPCHK(b, hipMemcpyAsync(g.d, g.h.data(), g.h.size() * sizeof(LntParams), hipMemcpyHostToDevice, b->stream),
-                "hipMemcpy (batch parameters)");
         BHIPCHK(b, hipStreamCreateWithFlags(&g.side, hipStreamNonBlocking), "hipStreamCreate");
         BHIPCHK(b, hipEventCreateWithFlags(&g.join, hipEventDisableTiming), "hipEventCreate");
+        if (g.pl.small) continue;
+        BHIPCHK(b, hipStreamBeginCapture(g.side, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+        bool ok = true;
+        for (uint32_t i = 0; i < GRAPH_ITERS && ok; i++) ok = batch_group_step(g);
+        hipError_t ec = hipStreamEndCapture(g.side, &g.graph);
+        if (!ok || ec != hipSuccess) return bfail(b, LNT_DEVICE_ERROR, "batch graph capture failed");
+        BHIPCHK(b, hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
-    BHIPCHK(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    BHIPCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    bool ok = true;
-    if (hipEventRecord(b->fork, b->stream) != hipSuccess) ok = false;
-    for (auto &g : b->groups) {
-        if (!ok) break;
-        ok = hipStreamWaitEvent(g.side, b->fork, 0) == hipSuccess && batch_group_step(g, g.side) &&
-             hipEventRecord(g.join, g.side) == hipSuccess && hipStreamWaitEvent(b->stream, g.join, 0) == hipSuccess;
-    }
-    hipError_t ec = hipStreamEndCapture(b->stream, &b->graph);
-    if (!ok || ec != hipSuccess) return bfail(b, LNT_DEVICE_ERROR, "batch graph capture failed");
-    BHIPCHK(b, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     b->dirty = false;
-    b->upload = false;
+    b->upload = true;
     b->captures++;
     return LNT_OK;
 }
 
-// Copy the groups' parameter slots to the device (after members joined, left or changed).
-static int batch_upload(lnt_batch *b) {
-    for (auto &g : b->groups)
-        BHIPCHK(b, hipMemcpyAsync(g.d, g.h.data(), g.h.size() * sizeof(LntParams), hipMemcpyHostToDevice, b->stream),
-                "hipMemcpy (batch parameters)");
-    b->upload = false;
+// Copy group g's parameter slots to the device, in the order of its stream.
+static int batch_upload(lnt_batch *b, lnt_batch::Group &g) {
+    BHIPCHK(b, hipMemcpyAsync(g.d, g.h.data(), g.h.size() * sizeof(LntParams), hipMemcpyHostToDevice, g.side),
+            "hipMemcpy (batch parameters)");
     return LNT_OK;
 }
 
@@ -1181,23 +1175,41 @@ static void batch_refresh(lnt_batch *b) {
 }
 
 // After an iteration every LL member owes its "-2": refresh the flags where they changed.
-static int batch_mark_pending(lnt_batch *b) {
-    for (auto &g : b->groups) {
-        bool changed = false;
-        for (u32 i = 0; i < g.cap; i++) {
-            lnt_ctx *c = g.ctxs[i];
-            if (!c) continue;
-            c->pending = true;
-            c->pristine = false;
-            u32 want = c->prp ? 0u : 1u;
-            if (g.h[i].sub2 != want) {
-                g.h[i].sub2 = want;
-                changed = true;
-            }
+static int batch_mark_pending(lnt_batch *b, lnt_batch::Group &g) {
+    bool changed = false;
+    for (u32 i = 0; i < g.cap; i++) {
+        lnt_ctx *c = g.ctxs[i];
+        if (!c) continue;
+        c->pending = true;
+        c->pristine = false;
+        u32 want = c->prp ? 0u : 1u;
+        if (g.h[i].sub2 != want) {
+            g.h[i].sub2 = want;
+            changed = true;
         }
-        if (changed)
-            BHIPCHK(b, hipMemcpyAsync(g.d, g.h.data(), g.h.size() * sizeof(LntParams), hipMemcpyHostToDevice, b->stream),
-                    "hipMemcpy (batch parameters)");
+    }
+    return changed ? batch_upload(b, g) : LNT_OK;
+}
+
+// `step` iterations of group g on its stream.
+static int batch_group_run(lnt_batch *b, lnt_batch::Group &g, uint32_t step) {
+    int rc;
+    // the first launch reads the members' "-2" flags as they are; after it every member owes one
+    for (bool first = true; step; first = false) {
+        uint32_t done = 1;
+        if (g.pl.small) {  // the kernel loops over iterations; bounded launches keep each one short
+            done = std::min<uint32_t>(step, small_chunk(g.pl));
+            if (!lnt_launch_batch_small(g.pl, g.d, g.cap, done, g.ll, g.side))
+                return bfail(b, LNT_UNSUPPORTED, "no batched kernel for this shape");
+        } else if (!first && step >= GRAPH_ITERS) {
+            done = GRAPH_ITERS;
+            BHIPCHK(b, hipGraphLaunch(g.exec, g.side), "hipGraphLaunch");
+        } else if (!batch_group_step(g)) {
+            return bfail(b, LNT_UNSUPPORTED, "no batched kernel for this shape");
+        }
+        BHIPCHK(b, hipGetLastError(), "kernel launch");
+        step -= done;
+        if (first && (rc = batch_mark_pending(b, g))) return rc;
     }
     return LNT_OK;
 }
@@ -1278,32 +1290,27 @@ int lnt_batch_iterate(lnt_batch *b, uint32_t k) {
     int rc;
     if (!b->dirty) batch_refresh(b);
     if (b->dirty && (rc = batch_build(b))) return rc;
-    if (b->upload && (rc = batch_upload(b))) return rc;
-    // Members under a Gerbicz check count the squarings as checked iterations: the
-    // replays stop at each of their block ends for the block step on the member's stream.
-    // A batch of single-workgroup tests only runs `step` iterations in one launch per
-    // group (the kernel loops over iterations), without the graph.
-    bool all_small = true;
-    for (auto &g : b->groups) all_small = all_small && g.pl.small;
+    if (b->upload)
+        for (auto &g : b->groups)
+            if ((rc = batch_upload(b, g))) return rc;
+    b->upload = false;
+    // Members under a Gerbicz check count the squarings as checked iterations: the groups
+    // stop at each of their block ends for the block step on the member's stream.
     uint32_t left = k;
-    bool first = true;
     while (left) {
         uint32_t step = left;
         for (lnt_ctx *c : b->members)
             if (c->g.on) step = (uint32_t)std::min<uint64_t>(step, c->g.B - c->g.it % c->g.B);
-        if (all_small) {
-            for (auto &g : b->groups)
-                if (!lnt_launch_batch_small(g.pl, g.d, g.cap, step, g.ll, b->stream))
-                    return bfail(b, LNT_UNSUPPORTED, "no batched kernel for this shape");
-            BHIPCHK(b, hipGetLastError(), "kernel launch");
-            if (first && (rc = batch_mark_pending(b))) return rc;
-            first = false;
+        BHIPCHK(b, hipEventRecord(b->fork, b->stream), "hipEventRecord");
+        rc = LNT_OK;
+        for (auto &g : b->groups) {
+            BHIPCHK(b, hipStreamWaitEvent(g.side, b->fork, 0), "hipStreamWaitEvent");
+            if (rc == LNT_OK) rc = batch_group_run(b, g, step);
+            // joined on an error too: whatever was launched is waited for by the batch stream
+            BHIPCHK(b, hipEventRecord(g.join, g.side), "hipEventRecord");
+            BHIPCHK(b, hipStreamWaitEvent(b->stream, g.join, 0), "hipStreamWaitEvent");
         }
-        for (uint32_t i = 0; i < step && !all_small; i++) {
-            BHIPCHK(b, hipGraphLaunch(b->exec, b->stream), "hipGraphLaunch");
-            if (first && (rc = batch_mark_pending(b))) return rc;
-            first = false;
-        }
+        if (rc != LNT_OK) return rc;
         left -= step;
         // later work on a member's own stream starts after the batch's
         BHIPCHK(b, hipEventRecord(b->done, b->stream), "hipEventRecord");
@@ -1446,7 +1453,7 @@ extern "C" int lnt_iterate_static(uint32_t p, int mode, uint64_t *x, size_t n, u
     const LntParams P = params_of(pl, p, x, t);
     bool ok = true;
     if (pl.small) {
-        const uint32_t chunk = pl.n >= 2048 ? 256 : 1024;
+        const uint32_t chunk = small_chunk(pl);
         bool first = true;
         for (uint32_t left = k; left && ok;) {
             const uint32_t c = left < chunk ? left : chunk;

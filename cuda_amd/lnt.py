@@ -343,8 +343,8 @@ class LucasPRP:
 
 
 class Batch:
-    """Independent tests advanced together: one hipGraph launch per iteration for all
-    members (members of one shape share batched kernel launches)."""
+    """Independent tests advanced together: members of one shape share batched kernel
+    launches, and the shapes advance side by side."""
 
     def __init__(self, device: int = 0):
         self._lib = load()

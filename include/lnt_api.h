@@ -168,7 +168,8 @@ int lnt_iterate_static(uint32_t p, int mode, uint64_t *x, size_t n, uint32_t k, 
 
 /* ---- batches of independent tests (new: the reference runs one test per process) ----
  * Members keep their own residues; members of the same shape run as one batched launch
- * per kernel and one iteration of all members is a single hipGraph launch.  Work issued
+ * per kernel, and the shapes advance side by side on streams of their own, joined at the
+ * end of the call (and at every Gerbicz block end).  Work issued
  * on a member after lnt_batch_iterate runs after the batch's work.  A context belongs to
  * at most one batch; lnt_destroy takes it out of its batch. */
 typedef struct lnt_batch lnt_batch;
@@ -176,7 +177,7 @@ int lnt_batch_create(int device, lnt_batch **out);
 int lnt_batch_add(lnt_batch *batch, lnt_ctx *ctx);
 int lnt_batch_remove(lnt_batch *batch, lnt_ctx *ctx);
 int lnt_batch_size(const lnt_batch *batch);
-/* out[0] members, [1] kernel-shape groups, [2] iteration graphs captured so far (members
+/* out[0] members, [1] kernel-shape groups, [2] times the iteration graphs were captured (members
  * joining or leaving a group with free slots only rewrite its parameters).  cap >= 3. */
 int lnt_batch_stats(const lnt_batch *batch, uint64_t *out, int cap);
 /* Every member advances k iterations (asynchronous). */
