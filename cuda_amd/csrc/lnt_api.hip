@@ -607,6 +607,7 @@ static std::string describe(const Plan &pl) {
     } else {
         char row[64];
         if (pl.row3m) std::snprintf(row, sizeof row, "lnt_k_row3m<%u,%u,%u>", pl.row3m, pl.rBB, pl.rBC);
+        else if (pl.rowm) std::snprintf(row, sizeof row, "lnt_k_rowm<%u>", pl.rowm);
         else if (pl.row3 == 16) std::snprintf(row, sizeof row, "lnt_k_row16");
         else if (pl.row3) std::snprintf(row, sizeof row, "lnt_k_row3<%u,%u>", pl.row3, pl.G);
         else std::snprintf(row, sizeof row, "lnt_k_row<%u,%u>", pl.row.B1, pl.row.B2);
@@ -750,7 +751,7 @@ int lnt_tune(lnt_ctx *c, int loops) {
     std::vector<PlanOpts> opts;
     for (uint32_t lc = 7; lc <= 14; lc++)
         for (uint32_t K : {16u, 8u, 4u})
-            for (int r3 : {0, 1, 2})
+            for (int r3 : {-1, 0, 1, 2})
                 for (int c3 : {0, 1}) {
                     PlanOpts o;
                     o.lc = lc;
@@ -758,7 +759,8 @@ int lnt_tune(lnt_ctx *c, int loops) {
                     o.row3 = r3;
                     o.col3 = c3;
                     Plan tmp;
-                    if (make_plan(c->p, n, tmp, o).empty()) opts.push_back(o);
+                    if (!make_plan(c->p, n, tmp, o).empty()) continue;
+                    if (r3 >= 0 || tmp.rowm) opts.push_back(o);  // -1 elsewhere is one of the others
                 }
     std::vector<Cand> cands;
     // warm-up long enough to capture the candidate's iteration graph, so the timed loops

@@ -60,6 +60,7 @@ struct Plan {
     uint32_t row3 = 0;      // 3-phase rows: C = row3^3 (0: 2-phase rows)
     uint32_t row3m = 0;     // mixed-radix 3-phase rows: C = row3m * rBB * rBC (0: none)
     uint32_t rBB = 0, rBC = 0;
+    uint32_t rowm = 0;      // matrix-core rows of 256 * rowm words (256 .. 2048; 0: none)
     uint32_t col3 = 0;      // 3-phase columns: first radix BA (0: 2-phase columns)
     uint32_t cBB = 0, cBC = 0;  // 3-phase columns: second and third radix
     uint32_t M = 0;         // carry halo (compile-time), >= levels
@@ -72,7 +73,7 @@ struct Plan {
 inline bool same_kernels(const Plan &a, const Plan &b) {
     return a.small == b.small && a.small16 == b.small16 && a.n == b.n && a.C == b.C && a.R == b.R && a.row.B1 == b.row.B1 &&
            a.row.B2 == b.row.B2 && a.col.B1 == b.col.B1 && a.col.B2 == b.col.B2 && a.K == b.K && a.G == b.G &&
-           a.row3 == b.row3 && a.row3m == b.row3m && a.rBB == b.rBB && a.rBC == b.rBC && a.col3 == b.col3 &&
+           a.rowm == b.rowm && a.row3 == b.row3 && a.row3m == b.row3m && a.rBB == b.rBB && a.rBC == b.rBC && a.col3 == b.col3 &&
            a.cBB == b.cBB && a.cBC == b.cBC && a.M == b.M;
 }
 
@@ -133,11 +134,14 @@ inline bool digits_fit_31(uint32_t p, uint32_t n, uint32_t levels) {
 // Row/column split of a large residue: log2 C and log2 R.
 inline bool split_for(uint32_t log_n, uint32_t &lc, uint32_t &lr) {
     if (log_n < 13 || log_n > 26) return false;
-    // rows of 4096 words (3-phase row kernel) from n = 2^16 on: measured 1.2-2x faster than
-    // the square-ish splits with 2-phase rows of 256 .. 2048 words.  From 2^24 the rows
-    // are 8192 words (2^24: 0.550 against 0.581 ms per iteration with 4096 x 4096), and
-    // 16384 at 2^26 (mixed-radix 3-phase rows), over columns of at most 4096 words
-    lc = log_n >= 24 ? (log_n == 26 ? 14 : 13) : log_n >= 16 ? 12 : (log_n + 1) / 2;
+    // Small transforms are chains of latencies: 16-row columns are the cheapest (tile of 256
+    // words) with rows of up to 2048 words, then 64-row columns (us per squaring, against
+    // the next best split: 2^13 12.7 / 13.9, 2^14 13.3 / 14.2, 2^15 15.1 / 15.4, 2^16 16.1 / 17.2,
+    // 2^17 18.5 / 21.3, 2^18 23.0 / 25.4), 512 x 1024 at 2^19 (28.3 / 30.2).  From 2^20 rows of
+    // 4096 words; from 2^24 8192 words (0.550 against 0.581 ms with 4096 x 4096) and 16384 at
+    // 2^26 (mixed-radix 3-phase rows), over columns of at most 4096 words.
+    static const uint8_t lcs[] = {9, 10, 11, 10, 11, 12, 10};
+    lc = log_n >= 24 ? (log_n == 26 ? 14 : 13) : log_n >= 20 ? 12 : lcs[log_n - 13];
     lr = log_n - lc;
     return lr <= 12 && lr >= 4;
 }
@@ -146,7 +150,8 @@ inline bool split_for(uint32_t log_n, uint32_t &lc, uint32_t &lr) {
 struct PlanOpts {
     uint32_t lc = 0;    // log2 of the row length
     uint32_t K = 0;     // column tile width
-    int row3 = -1;      // 1: 3-phase rows when C is 512 or 4096, 0: 2-phase, -1: default
+    int row3 = -1;      // 1: 3-phase rows when C is 512 or 4096, 0: 2-phase, -1: default (on the
+                        // matrix cores from C = 256)
                         // (rows of 8192 and 16384 words are always 3-phase: 1 and 2
                         // select 32 or 16 words per thread)
     int col3 = -1;      // 1: 3-phase columns (R = 512 .. 4096), 0: 2-phase, -1: default
@@ -187,9 +192,10 @@ inline bool plan_consistent(const Plan &pl) {
     else if (pl.row3) row = (uint64_t)pl.row3 * pl.row3 * pl.row3;
     else row = (uint64_t)pl.row.B1 * pl.row.B2;
     if (row != pl.C) return false;
-    return pl.G && pl.R % pl.G == 0 && (!pl.row3m || pl.G == 1);
+    return pl.G && pl.R % pl.G == 0 && (!(pl.row3m || pl.rowm) || pl.G == 1);
 }
 
+    else if (pl.rowm) row = 256ull * pl.rowm;
 inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts opts);
 
 // Build the plan; returns an empty string on success, else the reason.  pl is rebuilt from
@@ -286,6 +292,9 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
 // Digit widths w_i = ceil(p(i+1)/n) - ceil(p i/n).
 inline void widths(uint32_t p, uint32_t n, std::vector<uint8_t> &w) {
     w.resize(n);
+    } else if (opts.row3 < 0 && pl.C >= 256) {
+        pl.rowm = pl.C / 256;
+        pl.G = 1;
     uint32_t L = ilog2(n);
     for (uint32_t i = 0; i < n; i++) {
         uint64_t e0 = ((uint64_t)p * i + n - 1) >> L, e1 = ((uint64_t)p * (i + 1) + n - 1) >> L;
@@ -321,7 +330,9 @@ inline void to_device_digits(const std::vector<uint8_t> &w, const uint64_t *d, u
 }
 
 // Device words (pre-carry signed values) -> canonical digits in [0, 2^w).  Returns true
-// if the value is 0 mod 2^p - 1.
+// if the value is 0 mod 2^p - 1.  d may be x (in place).
+// Runs of at least 2^17 digits are carried side by side on host threads, each from a zero
+// carry; the carries between the runs then ripple a few digits into the next one.
 inline bool to_canonical_digits(const std::vector<uint8_t> &w, const uint64_t *x, bool sub2,
                                 uint64_t *d) {
     const size_t n = w.size();

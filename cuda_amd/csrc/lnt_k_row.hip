@@ -1,9 +1,11 @@
 // Instantiations of the row kernels (row lengths 128 .. 16384).
 #include "lnt_launch.hpp"
 
-// lnt_k_row16.hip
+// lnt_k_row16.hip, lnt_k_rowm.hip
 bool lnt_launch_row16(const lnt::Plan &pl, const LntParams &P, hipStream_t s, int mode);
 bool lnt_launch_batch_row16(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s);
+bool lnt_launch_rowm(const lnt::Plan &pl, const LntParams &P, hipStream_t s, int mode);
+bool lnt_launch_batch_rowm(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s);
 
 template <int B1, int B2>
 static bool go_row(const lnt::Plan &pl, const LntParams &P, hipStream_t s, int mode) {
@@ -51,6 +53,7 @@ bool lnt_launch_row(const lnt::Plan &pl, const LntParams &P, hipStream_t s, int 
     if (pl.row3m) return false;
     if (pl.row3 == 16) return lnt_launch_row16(pl, P, s, mode);
     if (pl.row3 == 8) return go_row3<8, 4>(pl, P, s, mode);
+    if (pl.rowm) return lnt_launch_rowm(pl, P, s, mode);
 #define RW(b1, b2) if (pl.row.B1 == b1 && pl.row.B2 == b2) return go_row<b1, b2>(pl, P, s, mode);
     RW(16, 8) RW(16, 16) RW(32, 16) RW(32, 32) RW(64, 32) RW(64, 64)
 #undef RW
@@ -68,6 +71,7 @@ bool lnt_launch_batch_row(const lnt::Plan &pl, const LntParams *Ps, u32 count, h
 #undef R3M
     if (pl.row3m) return false;
     if (pl.row3 == 16) return lnt_launch_batch_row16(pl, Ps, count, s);
+    if (pl.rowm) return lnt_launch_batch_rowm(pl, Ps, count, s);
     if (pl.row3 == 8) {
         const u32 wgs = pl.R / 4;
         hipLaunchKernelGGL((lnt_kb_row3<8, 4>), dim3(wgs * count), dim3(256), 0, s, Ps, wgs);

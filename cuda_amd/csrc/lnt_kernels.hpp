@@ -795,6 +795,177 @@ LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
             const u64 so = base + (u64)I * BC;
             if (MODE == LNT_FORWARD) {
 #pragma unroll
+// ------------------------------------------------------------------ lines of 256 S words on the matrix cores
+// The transform of a line of L = 256 S words (S = 1, 2, 4, 8, 16) by S waves, four words per
+// thread: L = 16 * 16 * S with the 16-point DFTs of mdft.hpp in phases 1 and 2 and an S-point
+// one in phase 3 (S = 2, 4 in registers, 8 and 16 on the matrix cores).  With i = i1 + 16 S j,
+// i1 = a + S b; wave w, lane (q, n), id = 16 w + n:
+//   phase 1: DFT i1 = id over j -> k2, twiddle omega_L^(i1 k2)                       (twr)
+//   phase 2: DFT (k2, a) = (id / S, id mod S) over b -> kb, twiddle omega_16S^(a kb) (twr2)
+//   phase 3: DFTs (k2, kb) over a, all k2 of one wave; square (or the product modes)
+// and the inverse in reverse.  A wave keeps its k2 between phase 1 and the inverse phase 2: only
+// the exchanges around these wait for the other waves.  LDS words A + ... of the region: runs of 16
+// words 18 apart, so that they start 16-byte aligned, 16 neighbouring runs cover all banks and
+// the reads of adjacent word pairs are 128-bit.
+// lnt_line16 takes phase 1's inputs z (place e: i1 = id, j = lnt_m16_word(q, e)) and leaves the
+// inverse's outputs (place v: j = -lnt_m16_word(q, v) mod 16).  T holds the thread's twiddles
+// tw1, tw2, itw2, itw1 (loaded by line16_load_*; the before_* hooks may load them late).
+// Transform-domain words for MODE 1/2 at slot + v.
+template <int S>
+constexpr u32 lnt_line16_lds() { return 288 * S; }
+
+// a of this thread's phase-3 place v: S = 16 (w, n, -word(q, v)), S = 8 (2w + v / 2, n, -(2q + v % 2)),
+// S = 4 (4w + q, n, v), S = 2 (8w + 2q + v / 2, n, v % 2)
+template <int S>
+GL_HD constexpr int lnt_line16_a(int q, int v) {
+    return S == 16 ? lnt_m16_neg(q, v) : S == 8 ? (8 - 2 * q - (v & 1)) & 7 : S == 4 ? v : v & 1;
+}
+
+struct LntTw16 {
+    u64 tw1[4], tw2[4], itw2[4], itw1[4];
+};
+template <int S>
+LNT_KFN void line16_load_tw1(LntTw16 &T, const LntLane16 &L, const LntParams &P) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) T.tw1[e] = P.twr[16 * S * brev_v16(lnt_m16_word(L.q, e)) + L.id];
+}
+template <int S>
+LNT_KFN void line16_load_tw2(LntTw16 &T, const LntLane16 &L, const LntParams &P) {
+    if (S == 1) return;
+#pragma unroll
+    for (int e = 0; e < 4; e++) T.tw2[e] = P.twr2[S * brev_v16(lnt_m16_word(L.q, e)) + L.id % S];
+}
+template <int S>
+LNT_KFN void line16_load_itw2(LntTw16 &T, const LntLane16 &L, const LntParams &P) {
+    if (S == 1) return;
+#pragma unroll
+    for (int v = 0; v < 4; v++) T.itw2[v] = P.itwr2[S * brev_v16(L.n) + lnt_line16_a<S>(L.q, v)];
+}
+template <int S>
+LNT_KFN void line16_load_itw1(LntTw16 &T, const LntLane16 &L, const LntParams &P) {
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        T.itw1[v] = P.itwr[16 * S * brev_v16(L.id / S) + L.id % S + S * lnt_m16_neg(L.q, v)];
+}
+
+// Returns with z transformed, or (MODE_FORWARD) with the transform in y.  The region at A must be
+// free when phase 1 writes it (after z was read) and is free again after the next barrier.
+template <int S, int MODE, class H2, class HI2, class HI1>
+LNT_KFN void lnt_line16(u64 (&z)[4], const LntM16 &Mx, const LntM8 &M8, LView lds, u32 A, const LntLane16 &L, LntTw16 &T,
+                        const LntParams &P, u64 slot, H2 before_tw2, HI2 before_itw2, HI1 before_itw1) {
+    const int q = L.q, n = L.n, id = L.id;
+    const u32 t1 = A + (u32)(18 * (id % S) + id / S);  // place of i1 = id within a k2
+    const u32 own = A + (u32)(18 * id + 2 * q);        // this lane's words of run id
+    const u32 area = A + (u32)(288 * L.w);             // this wave's runs
+    // phase-3 layout of the wave's area: word (k2, kb, a)
+    auto p3 = [&](int k2l, int kb, int a) {
+        return area + (u32)(S == 16 ? 18 * kb + a : (16 * S + 2) * k2l + S * kb + a);
+    };
+    lnt_m16_dft(Mx, z);
+#pragma unroll
+    for (int v = 0; v < 4; v++) lds[(u32)(18 * S * lnt_m16_word(q, v)) + t1] = gl_mmul(z[v], T.tw1[v]);
+    before_tw2();
+    LNT_SYNC();
+    // phase 2
+#pragma unroll
+    for (int e = 0; e < 4; e++) z[e] = lds[own + lnt_m16_word(0, e)];
+    LNT_WAVE_SYNC();
+    lnt_m16_dft(Mx, z);
+    if (S > 1) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) lds[p3(n / S, lnt_m16_word(q, v), n % S)] = gl_mmul(z[v], T.tw2[v]);
+        if (MODE != LNT_FORWARD) before_itw2();
+        LNT_WAVE_SYNC();
+        // phase 3
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            z[v] = lds[S == 16  ? p3(0, n, 2 * q) + lnt_m16_word(0, v)
+                       : S == 8 ? p3(v / 2, n, 2 * q + v % 2)
+                       : S == 4 ? p3(q, n, v)
+                                : p3(2 * q + v / 2, n, v % 2)];
+        LNT_WAVE_SYNC();
+    }
+    auto phase3 = [&](bool inverse) {
+        if (S == 16) lnt_m16_dft(Mx, z);
+        if (S == 8) {
+            u64 h[2] = {z[0], z[1]}, g[2] = {z[2], z[3]};
+            lnt_m8_dft(M8, Mx, h);
+            lnt_m8_dft(M8, Mx, g);
+            z[0] = h[0], z[1] = h[1], z[2] = g[0], z[3] = g[1];
+        }
+        if (S == 4) inverse ? dft_inv<4>(z) : dft_fwd<4>(z);
+        if (S == 2) {
+            inverse ? dft_inv<2>(z) : dft_fwd<2>(z);
+            inverse ? dft_inv<2>(z + 2) : dft_fwd<2>(z + 2);
+        }
+    };
+    phase3(false);
+    // pointwise
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        if (MODE == LNT_FORWARD) P.y[slot + v] = z[v];
+        else z[v] = gl_mmul(z[v], MODE == LNT_MULTIPLY ? P.f[slot + v] : z[v]);
+    }
+    if (MODE == LNT_FORWARD) return;
+    if (S > 1) {
+        phase3(true);
+        before_itw1();
+        // inverse phase-2 twiddle; runs (k2, a) of words kb again
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int k2l = S == 16 ? 0 : S == 8 ? v / 2 : S == 4 ? q : 2 * q + v / 2;
+            lds[area + (u32)(18 * (S * k2l + lnt_line16_a<S>(q, v)) + n)] = gl_mmul(z[v], T.itw2[v]);
+        }
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int e = 0; e < 4; e++) z[e] = lds[own + lnt_m16_word(0, e)];
+        LNT_WAVE_SYNC();
+    }
+    // inverse phase 2: output place v is b = -k
+    lnt_m16_dft(Mx, z);
+#pragma unroll
+    for (int v = 0; v < 4; v++) lds[A + (u32)(18 * id + lnt_m16_neg(q, v))] = gl_mmul(z[v], T.itw1[v]);
+    LNT_SYNC();
+    // inverse phase 1
+#pragma unroll
+    for (int e = 0; e < 4; e++) z[e] = lds[(u32)(18 * S * lnt_m16_word(q, e)) + t1];
+    lnt_m16_dft(Mx, z);
+}
+
+// The row pass for rows of 256 S words (S <= 8), one row per workgroup of S waves: 4-step
+// twiddles around the line, all factors fetched at the start.  MODEs as in lnt_row_body; slots
+// base + 4 t + v.
+template <int S, int MODE = LNT_SQUARE>
+LNT_KFN void lnt_rowm_body(int tid, int bid, LView lds, const LntParams &P) {
+    static_assert(S <= 8, "16 waves have no registers for the factors: lnt_row16_body");
+    const u64 base = (u64)(256 * S) * (u64)bid;
+    const LntLane16 L = lnt_lane16(tid);
+    u64 z[4], t4[4];
+    LntTw16 T;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const u64 idx = base + L.id + 16 * S * lnt_m16_word(L.q, e);
+        z[e] = gl_mmul(P.y[idx], P.tw4[idx]);
+    }
+    line16_load_tw1<S>(T, L, P);
+    line16_load_tw2<S>(T, L, P);
+    if (MODE != LNT_FORWARD) {
+        line16_load_itw2<S>(T, L, P);
+        line16_load_itw1<S>(T, L, P);
+#pragma unroll
+        for (int v = 0; v < 4; v++) t4[v] = P.itw4[base + L.id + 16 * S * lnt_m16_neg(L.q, v)];
+    }
+    LntM16 Mx;
+    LntM8 M8;
+    lnt_m16_load(Mx, tid);
+    if (S == 8) lnt_m8_load(M8, Mx, tid);
+    auto loaded = [] {};
+    lnt_line16<S, MODE>(z, Mx, M8, lds, 0, L, T, P, base + 4 * (u64)tid, loaded, loaded, loaded);
+    if (MODE == LNT_FORWARD) return;
+#pragma unroll
+    for (int v = 0; v < 4; v++) P.y[base + L.id + 16 * S * lnt_m16_neg(L.q, v)] = gl_mmul(z[v], t4[v]);
+}
+
                 for (int i = 0; i < BC; i++) P.y[so + i] = e[i];
                 continue;
             }
@@ -948,102 +1119,63 @@ LNT_KFN void lnt_small_body(int tid, LView lds, const LntParams &P, u32 iters, b
 }
 
 // ------------------------------------------------------------------ small residues on the matrix cores
-// One workgroup of S waves runs `iters` iterations on n = 256 S words (S = 1, 2, 4, 8, 16), four
-// words per thread: n = 16 * 16 * S with the 16-point DFTs of mdft.hpp in phases 1 and 2 and an
-// S-point one in phase 3 (S = 2, 4 in registers, 8 and 16 on the matrix cores).  With
-// i = i1 + 16 S j, i1 = a + S b; wave w, lane (q, n), id = 16 w + n:
-//   phase 1: DFT i1 = id over j -> k2, twiddle omega_n^(i1 k2)                       (twr)
-//   phase 2: DFT (k2, a) = (id / S, id mod S) over b -> kb, twiddle omega_16S^(a kb) (twr2)
-//   phase 3: DFTs (k2, kb) over a, all k2 of one wave
-// One test is a chain of dependent steps on one compute unit, so what counts is its latency:
-// four words per thread put four times the waves of the former 16-word kernels to work on
-// it, a wave keeps its k2 from phase 2 to the inverse phase 2 (four barriers per iteration),
-// and up to S = 8 the factors of a thread's words stay in registers.  For n = 4096 that would
-// take more than the 128 registers of 16 waves: weights and twiddles are re-read (from the L2,
-// ahead of their use) and the unweights lie in LDS.
+// One workgroup of S waves runs `iters` iterations on n = 256 S words, a line of lnt_line16
+// between the carry and weights and the unweights.  One test is a chain of dependent steps on
+// one compute unit, so what counts is its latency: four words per thread put four times the
+// waves of the former 16-word kernels to work on it, an iteration has four barriers, and up to
+// S = 8 the factors of a thread's words stay in registers.  For n = 4096 that would take more
+// than the 128 registers of 16 waves: weights and twiddles are re-read (from the L2, ahead of
+// their use) and the unweights lie in LDS.
 // LDS: two regions, the residue (or its digits) in natural order in one while the other holds
-// the transform, runs of 16 words 18 apart as in the row kernel.  MODEs as above.
+// the transform.  MODEs as above.
 template <int S>
-constexpr u32 lnt_small16_region() { return 288 * S; }
-template <int S>
-constexpr u32 lnt_small16_lds() { return 2 * lnt_small16_region<S>() + (S == 16 ? 256 * S : 0); }
+constexpr u32 lnt_small16_lds() { return 2 * lnt_line16_lds<S>() + (S == 16 ? 256 * S : 0); }
 
 template <int S, int M, int MODE = LNT_SQUARE>
 LNT_KFN void lnt_small16_body(int tid, LView lds, const LntParams &P, u32 iters, bool sub2_first, bool ll) {
-    constexpr u32 N = 256 * S, L = 16 * S;
-    constexpr bool RES = S <= 8;                // factors live in registers
-    constexpr int KW = 16 / S;                  // k2 per wave
-    constexpr u32 U = 2 * lnt_small16_region<S>();  // unweights (S = 16)
-    const int w = LNT_UNIFORM(tid / 64);
-    int q = (tid % 64) / 16, n = tid % 16, id = 16 * w + n;
-    const u32 area = (u32)(288 * w);                // this wave's runs
-    // phase-3 layout of the wave's area: word (k2, kb, a)
-    auto p3 = [&](int k2l, int kb, int a) {
-        return area + (u32)(S == 16 ? 18 * kb + a : (16 * S + 2) * k2l + S * kb + a);
-    };
+    constexpr u32 N = 256 * S;
+    constexpr bool RES = S <= 8;                    // factors live in registers
+    constexpr u32 U = 2 * lnt_line16_lds<S>();      // unweights (S = 16)
+    LntLane16 L = lnt_lane16(tid);
     LntM16 Mx;
     LntM8 M8;
     lnt_m16_load(Mx, tid);
     if (S == 8) lnt_m8_load(M8, Mx, tid);
-    u64 wv[4], wb[4], uv[4], tw1[4], itw1[4], tw2[4], itw2[4];
-    const u64 r2 = gl_mul(GL_R, GL_R);
-    // phase-3 places of this thread: S = 16 (w, kb = n, a = -word(q, v)), S = 8 (2w + g, n, -(2q + v)),
-    // S = 4 (4w + q, n, v), S = 2 (8w + 2q + c, n, v)
-    auto p3a = [&](int v) { return S == 16 ? (16 - lnt_m16_word(q, v)) & 15 : S == 8 ? (8 - 2 * q - (v & 1)) & 7 : S == 4 ? v : v & 1; };
+    u64 wv[4], wb[4], uv[4];
+    LntTw16 T;
     auto load_w = [&]() {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const u32 i = (u32)id + L * lnt_m16_word(q, e);
+            const u32 i = (u32)(L.id + 16 * S * lnt_m16_word(L.q, e));
             wv[e] = P.w[2 * i];
             wb[e] = P.w[2 * i + 1];
         }
     };
-    auto load_tw1 = [&]() {
-#pragma unroll
-        for (int e = 0; e < 4; e++) tw1[e] = P.twr[L * brev_v16(lnt_m16_word(q, e)) + id];
-    };
-    auto load_tw2 = [&]() {
-        if (S == 1) return;
-#pragma unroll
-        for (int e = 0; e < 4; e++) tw2[e] = P.twr2[S * brev_v16(lnt_m16_word(q, e)) + id % S];
-    };
-    auto load_itw2 = [&]() {
-        if (S == 1) return;
-#pragma unroll
-        for (int v = 0; v < 4; v++) itw2[v] = P.itwr2[S * brev_v16(n) + p3a(v)];
-    };
-    auto load_itw1 = [&]() {
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            itw1[v] = P.itwr[L * brev_v16(id / S) + id % S + S * ((16 - lnt_m16_word(q, v)) & 15)];
-    };
     if (RES) {
         load_w();
-        load_tw1();
-        load_tw2();
-        load_itw2();
-        load_itw1();
+        line16_load_tw1<S>(T, L, P);
+        line16_load_tw2<S>(T, L, P);
+        line16_load_itw2<S>(T, L, P);
+        line16_load_itw1<S>(T, L, P);
     }
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         // unweight of output place v, times 2^128: one 2^64 for its Montgomery multiply and one
         // for the factor 2^-64 that the pointwise product leaves
-        const u32 i = (u32)id + L * ((16 - lnt_m16_word(q, v)) & 15);
+        const u32 i = (u32)(L.id + 16 * S * lnt_m16_neg(L.q, v));
         const u64 u = gl_mul(P.uw[i], r2);
         if (RES) uv[v] = u;
         else lds[U + i] = u;
     }
-    u32 A = 0, B = lnt_small16_region<S>();
+    u32 A = 0, B = lnt_line16_lds<S>();
 #pragma unroll
     for (int j = 0; j < 4; j++) lds[A + (u32)(tid + 64 * S * j)] = P.x[(u64)tid + 64 * S * j];
     LNT_SYNC();
     for (u32 it = 0; it < iters; it++) {
         if (!RES) {
             LNT_OPAQUE_LANE(tid);
-            n = tid % 16, q = (tid % 64) / 16, id = 16 * w + n;
+            L = lnt_lane16(tid);
         }
-        const u32 t1 = (u32)(18 * (id % S) + id / S);  // place of i1 = id within a k2 of the transform region
-        const u32 own = (u32)(18 * id + 2 * q);        // this lane's words of run id
         // carry of digits 4 tid .. 4 tid + 3 from the M pre-carry words before them on: A -> B
         {
             const u32 g0 = 4 * (u32)tid;
@@ -1059,89 +1191,22 @@ LNT_KFN void lnt_small16_body(int tid, LView lds, const LntParams &P, u32 iters,
         }
         if (!RES) {
             load_w();
-            load_tw1();
+            line16_load_tw1<S>(T, L, P);
         }
         LNT_SYNC();
         u64 z[4];
-        // phase 1: weight, DFT over j, twiddle: B -> A
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const u64 d = lds[B + (u32)id + L * lnt_m16_word(q, e)];
+            const u64 d = lds[B + (u32)(L.id + 16 * S * lnt_m16_word(L.q, e))];
             z[e] = P.bias ? gl_mul_biased((u32)d, wv[e], wb[e]) : gl_mul(d, wv[e]);
         }
-        lnt_m16_dft(Mx, z);
-#pragma unroll
-        for (int v = 0; v < 4; v++) lds[A + (u32)(18 * S * lnt_m16_word(q, v)) + t1] = gl_mmul(z[v], tw1[v]);
-        if (!RES) load_tw2();
-        LNT_SYNC();
-        // phase 2
-#pragma unroll
-        for (int e = 0; e < 4; e++) z[e] = lds[A + own + lnt_m16_word(0, e)];
-        LNT_WAVE_SYNC();
-        lnt_m16_dft(Mx, z);
-        if (S > 1) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) lds[A + p3(n / S, lnt_m16_word(q, v), n % S)] = gl_mmul(z[v], tw2[v]);
-            if (!RES && MODE != LNT_FORWARD) load_itw2();
-            LNT_WAVE_SYNC();
-            // phase 3
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                z[v] = lds[A + (S == 16  ? p3(0, n, 2 * q) + lnt_m16_word(0, v)
-                                : S == 8 ? p3(v / 2, n, 2 * q + v % 2)
-                                : S == 4 ? p3(q, n, v)
-                                         : p3(2 * q + v / 2, n, v % 2))];
-            LNT_WAVE_SYNC();
-        }
-        auto transform3 = [&](bool inverse) {
-            if (S == 16) lnt_m16_dft(Mx, z);
-            if (S == 8) {
-                u64 h[2] = {z[0], z[1]}, g[2] = {z[2], z[3]};
-                lnt_m8_dft(M8, Mx, h);
-                lnt_m8_dft(M8, Mx, g);
-                z[0] = h[0], z[1] = h[1], z[2] = g[0], z[3] = g[1];
-            }
-            if (S == 4) inverse ? dft_inv<4>(z) : dft_fwd<4>(z);
-            if (S == 2) {
-                inverse ? dft_inv<2>(z) : dft_fwd<2>(z);
-                inverse ? dft_inv<2>(z + 2) : dft_fwd<2>(z + 2);
-            }
-        };
-        transform3(false);
-        // pointwise
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            if (MODE == LNT_FORWARD) P.y[4 * (u64)tid + v] = z[v];
-            else z[v] = gl_mmul(z[v], MODE == LNT_MULTIPLY ? P.f[4 * (u64)tid + v] : z[v]);
-        }
+        lnt_line16<S, MODE>(
+            z, Mx, M8, lds, A, L, T, P, 4 * (u64)tid, [&]() { if (!RES) line16_load_tw2<S>(T, L, P); },
+            [&]() { if (!RES) line16_load_itw2<S>(T, L, P); }, [&]() { if (!RES) line16_load_itw1<S>(T, L, P); });
         if (MODE == LNT_FORWARD) return;
-        if (S > 1) {
-            transform3(true);
-            if (!RES) load_itw1();
-            // inverse phase-2 twiddle; runs (k2, a) of words kb again
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int k2l = S == 16 ? 0 : S == 8 ? v / 2 : S == 4 ? q : 2 * q + v / 2;
-                lds[A + area + (u32)(18 * (S * (k2l % KW) + p3a(v)) + n)] = gl_mmul(z[v], itw2[v]);
-            }
-            LNT_WAVE_SYNC();
-#pragma unroll
-            for (int e = 0; e < 4; e++) z[e] = lds[A + own + lnt_m16_word(0, e)];
-            LNT_WAVE_SYNC();
-        }
-        // inverse phase 2: output place v is b = -k
-        lnt_m16_dft(Mx, z);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            lds[A + (u32)(18 * id + ((16 - lnt_m16_word(q, v)) & 15))] = gl_mmul(z[v], itw1[v]);
-        LNT_SYNC();
-        // inverse phase 1, unweight: A -> B
-#pragma unroll
-        for (int e = 0; e < 4; e++) z[e] = lds[A + (u32)(18 * S * lnt_m16_word(q, e)) + t1];
-        lnt_m16_dft(Mx, z);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const u32 i = (u32)id + L * ((16 - lnt_m16_word(q, v)) & 15);
+            const u32 i = (u32)(L.id + 16 * S * lnt_m16_neg(L.q, v));
             lds[B + i] = gl_mmul(z[v], RES ? uv[v] : lds[U + i]);
         }
         LNT_SYNC();
@@ -1192,6 +1257,7 @@ GL_HD u64 lnt_tw4_3(u64 omega_n, u32 C, u32 BA, u32 BB, u32 BC, u64 idx) {
 // GL_R for the Montgomery multiply that applies it, one for the 2^-64 the square left.
 GL_HD u64 lnt_row_factor(u64 B, u64 m, u32 p, u32 n, u32 C, u32 slot) {
     const u64 v = gl_mul(gl_pow(B, lnt_wexp(p, n, (u64)C * (slot >> 1))), gl_mul(GL_R, GL_R));
+    const u64 r2 = gl_mul(GL_R, GL_R);
     return (slot & 1) ? gl_mul(v, m) : v;
 }
 // Weights: word i is half of the pair (w, -2^31 w) of slot i / 2 (gl_mul_biased takes both),
@@ -1214,3 +1280,4 @@ GL_HD u64 lnt_weight(u64 Bw, u32 p, u32 n, u32 i) {
     u32 r = (u32)((u64)p * i) & (n - 1);
     return gl_pow(Bw, (u64)(n - r));
 }
+        // weights from B, the line in A, unweights into B: the residue of the next iteration

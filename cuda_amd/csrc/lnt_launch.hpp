@@ -74,6 +74,13 @@ __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) 
     lnt_row3_body<B, G, MODE>(threadIdx.x, blockIdx.x, LView{smem, W}, P);
 }
 
+// rows of 256 S words on the matrix cores
+template <int S, int MODE>
+__global__ __launch_bounds__(64 * S) void lnt_k_rowm(LntParams P) {
+    __shared__ __align__(16) u64 smem[lnt_line16_lds<S>()];
+    lnt_rowm_body<S, MODE>(threadIdx.x, blockIdx.x, LView{smem, lnt_line16_lds<S>()}, P);
+}
+
 // 4096-word rows on the matrix cores
 template <int GW, int MODE>
 __global__ __launch_bounds__(1024 / GW) __attribute__((amdgpu_waves_per_eu(4))) void lnt_k_row16(LntParams P) {
@@ -185,6 +192,14 @@ __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) 
     const LntParams P = Ps[blockIdx.x / wgs];
     if (P.n == 0) return;  // an empty slot of the batch
     lnt_row3_body<B, G>(threadIdx.x, blockIdx.x % wgs, LView{smem, W}, P);
+}
+
+template <int S>
+__global__ __launch_bounds__(64 * S) void lnt_kb_rowm(const LntParams *__restrict__ Ps, u32 wgs) {
+    __shared__ __align__(16) u64 smem[lnt_line16_lds<S>()];
+    const LntParams P = Ps[blockIdx.x / wgs];
+    if (P.n == 0) return;  // an empty slot of the batch
+    lnt_rowm_body<S>(threadIdx.x, blockIdx.x % wgs, LView{smem, lnt_line16_lds<S>()}, P);
 }
 
 template <int GW>

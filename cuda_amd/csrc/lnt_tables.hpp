@@ -65,7 +65,8 @@ static TableSizes table_sizes(const Plan &pl) {
     t.n = pl.n;
     t.large = !pl.small;
     t.Lr = pl.small ? pl.n : pl.C;
-    t.L2 = pl.small16 > 1 ? 16 * pl.small16 : pl.row3m ? pl.rBB * pl.rBC : pl.row3 ? pl.row3 * pl.row3 : 0;
+    const u32 m16 = pl.small ? pl.small16 : pl.rowm;
+    t.L2 = m16 > 1 ? 16 * m16 : pl.row3m ? pl.rBB * pl.rBC : pl.row3 ? pl.row3 * pl.row3 : 0;
     t.R = pl.small ? 0 : pl.R;
     t.A = (!pl.small && pl.col3) ? pl.R / pl.col3 : 0;
     t.W = pl.small ? 2 * pl.n : 4 * pl.R;
@@ -94,9 +95,10 @@ static void fill_tables(const Plan &pl, u32 p, const TablePtrs &t, hipStream_t s
     const u32 Lr = z.Lr;
     u64 omr = gl_pow(554, (GL_P - 1) / Lr);
     // row line twiddles: first phase B1 x B2 (3-phase rows: row3 x row3^2, row3m x rBB rBC;
-    // one workgroup on the matrix cores: 16 x 16 small16)
-    const u32 rB1 = pl.small16 ? 16 : pl.row3m ? pl.row3m : pl.row3 ? pl.row3 : pl.row.B1;
-    const u32 rB2 = pl.small16 ? 16 * pl.small16
+    // lines on the matrix cores: 16 x 16 m16)
+    const u32 m16 = pl.small ? pl.small16 : pl.rowm;
+    const u32 rB1 = m16 ? 16 : pl.row3m ? pl.row3m : pl.row3 ? pl.row3 : pl.row.B1;
+    const u32 rB2 = m16        ? 16 * m16
                     : pl.row3m ? pl.rBB * pl.rBC
                     : pl.row3  ? pl.row3 * pl.row3
                                : pl.row.B2;
@@ -131,10 +133,10 @@ static void fill_tables(const Plan &pl, u32 p, const TablePtrs &t, hipStream_t s
         }
     }
     // second-phase row twiddles: a line of L2 = B2 words split (row3 x row3, rBB x rBC or
-    // 16 x small16)
+    // 16 x m16)
     if (z.L2) {
-        const u32 s1 = pl.small16 ? 16 : pl.row3m ? pl.rBB : pl.row3;
-        const u32 s2 = pl.small16 ? pl.small16 : pl.row3m ? pl.rBC : pl.row3;
+        const u32 s1 = m16 ? 16 : pl.row3m ? pl.rBB : pl.row3;
+        const u32 s2 = m16 ? m16 : pl.row3m ? pl.rBC : pl.row3;
         u64 om2 = gl_pow(554, (GL_P - 1) / z.L2);
         hipLaunchKernelGGL(lnt_k_line_tw, dim3((z.L2 + 255) / 256), dim3(256), 0, s, om2, s1, s2, z.L2, t.twr2);
         hipLaunchKernelGGL(lnt_k_line_tw, dim3((z.L2 + 255) / 256), dim3(256), 0, s, gl_inv(om2), s1, s2, z.L2,

@@ -267,3 +267,14 @@ LNT_KFN void lnt_m8_dft(const LntM8 &M, const LntM16 &M16, u64 (&x)[2]) {
     }
 }
 #endif
+
+// The lane's part in its workgroup's DFTs: wave w, lane (q, n), id = 16 w + n.
+struct LntLane16 {
+    int w, q, n, id;
+};
+LNT_KFN LntLane16 lnt_lane16(int tid) {
+    const int w = LNT_UNIFORM(tid / 64);
+    return LntLane16{w, (tid % 64) / 16, tid % 16, 16 * w + tid % 16};
+}
+// word of output place v of an inverse DFT
+GL_HD constexpr int lnt_m16_neg(int q, int v) { return (16 - lnt_m16_word(q, v)) & 15; }

@@ -80,13 +80,13 @@ extern "C" void *emu_create3(uint32_t p, uint32_t n, int prp, uint32_t lc, uint3
         for (uint32_t i = 0; i < 2 * pl.R; i++) e->uw[i] = lnt_row_factor(Binv, 2, p, n, pl.C, i);
     }
     widths(p, n, e->wid);
-    if (pl.small16) {
+    if (const uint32_t m16 = pl.small ? pl.small16 : pl.rowm) {
         Line l1, l2;
         l1.B1 = l2.B1 = 16;
-        l1.B2 = n / 16;
-        l2.B2 = pl.small16;
-        line_tables(n, l1, e->twr, e->itwr);
-        line_tables(16 * pl.small16, l2, e->twr2, e->itwr2);
+        l1.B2 = 16 * m16;
+        l2.B2 = m16;
+        line_tables(256 * m16, l1, e->twr, e->itwr);
+        line_tables(16 * m16, l2, e->twr2, e->itwr2);
     } else if (pl.row3m) {
         Line l1, l2;
         l1.B1 = pl.row3m;
@@ -297,6 +297,16 @@ static bool run_small(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mod
     if (pl.small16 == 16) return small16_any<16>(e, k, P, sub2, mode), true;
     if (pl.small16 == 8) return small16_any<8>(e, k, P, sub2, mode), true;
     if (pl.small16 == 4) return small16_any<4>(e, k, P, sub2, mode), true;
+template <int S>
+static void rowm_sq(Emu *e, const LntParams &P, int mode) {
+    for (uint32_t b = 0; b < e->pl.R; b++)
+        run_wg(64 * S, lnt_line16_lds<S>(), [&](int tid, LView L) {
+            if (mode == LNT_FORWARD) lnt_rowm_body<S, LNT_FORWARD>(tid, b, L, P);
+            else if (mode == LNT_MULTIPLY) lnt_rowm_body<S, LNT_MULTIPLY>(tid, b, L, P);
+            else lnt_rowm_body<S>(tid, b, L, P);
+        });
+}
+
     if (pl.small16 == 2) return small16_any<2>(e, k, P, sub2, mode), true;
     if (pl.small16 == 1) return small16_any<1>(e, k, P, sub2, mode), true;
 #define SM(b1, b2)                                                                          \
@@ -381,6 +391,10 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
 #undef C3I
     return ok;
 }
+    if (pl.rowm == 1) rowm_sq<1>(e, P, mode), ok = true;
+    if (pl.rowm == 2) rowm_sq<2>(e, P, mode), ok = true;
+    if (pl.rowm == 4) rowm_sq<4>(e, P, mode), ok = true;
+    if (pl.rowm == 8) rowm_sq<8>(e, P, mode), ok = true;
 
 extern "C" int emu_iterate(void *h, uint32_t k) {
     Emu *e = (Emu *)h;
