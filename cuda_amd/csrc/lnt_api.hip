@@ -297,11 +297,10 @@ static int copy_buf(lnt_ctx *c, u64 *dst, const u64 *src) {
 // Canonical digits of the residue in a device buffer (waits for the stream).
 static int canonical_of(lnt_ctx *c, const u64 *buf, bool pending, std::vector<uint64_t> &d) {
     const u32 n = c->pl.n;
-    std::vector<uint64_t> xd(n);
     d.resize(n);
-    HIPCHK(c, hipMemcpyAsync(xd.data(), buf, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpy (D2H)");
+    HIPCHK(c, hipMemcpyAsync(d.data(), buf, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpy (D2H)");
     HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    to_canonical_digits(c->wid, xd.data(), !c->prp && pending, d.data());
+    to_canonical_digits(c->wid, d.data(), !c->prp && pending, d.data());
     return LNT_OK;
 }
 
@@ -391,10 +390,10 @@ static int read_digits(lnt_ctx *c, uint64_t *d) {
         std::memcpy(d, c->set_digits.data(), (size_t)n * 8);
         return LNT_OK;
     }
-    std::vector<uint64_t> xd(n);
-    HIPCHK(c, hipMemcpyAsync(xd.data(), c->x, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpy (x)");
+    // copied to the caller's buffer and put in canonical digits there
+    HIPCHK(c, hipMemcpyAsync(d, c->x, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpy (x)");
     HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    bool zero = to_canonical_digits(c->wid, xd.data(), !c->prp && c->pending, d);
+    bool zero = to_canonical_digits(c->wid, d, !c->prp && c->pending, d);
     if (zero && c->prp && c->zero_ones)
         for (u32 i = 0; i < n; i++) d[i] = (1ull << c->wid[i]) - 1;
     return LNT_OK;
@@ -607,11 +606,14 @@ static std::string describe(const Plan &pl) {
     } else {
         char row[64];
         if (pl.row3m) std::snprintf(row, sizeof row, "lnt_k_row3m<%u,%u,%u>", pl.row3m, pl.rBB, pl.rBC);
-        else if (pl.rowm) std::snprintf(row, sizeof row, "lnt_k_rowm<%u>", pl.rowm);
         else if (pl.row3 == 16) std::snprintf(row, sizeof row, "lnt_k_row16");
+        else if (pl.rowm) std::snprintf(row, sizeof row, "lnt_k_rowm<%u>", pl.rowm);
         else if (pl.row3) std::snprintf(row, sizeof row, "lnt_k_row3<%u,%u>", pl.row3, pl.G);
         else std::snprintf(row, sizeof row, "lnt_k_row<%u,%u>", pl.row.B1, pl.row.B2);
-        if (pl.col3)
+        if (pl.colm)
+            std::snprintf(b, sizeof b, "LNT_2PASS_%ux%u;lnt_k_colm_fwd<%u>;%s;lnt_k_colm_inv<%u>", pl.R, pl.C, pl.colm,
+                          row, pl.colm);
+        else if (pl.col3)
             std::snprintf(b, sizeof b, "LNT_2PASS_%ux%u;lnt_k_col3_fwd<%u,%u,%u,%u>;%s;lnt_k_col3_inv<%u,%u,%u,%u>", pl.R,
                           pl.C, pl.col3, pl.cBB, pl.cBC, pl.K, row, pl.col3, pl.cBB, pl.cBC, pl.K);
         else
@@ -752,7 +754,7 @@ int lnt_tune(lnt_ctx *c, int loops) {
     for (uint32_t lc = 7; lc <= 14; lc++)
         for (uint32_t K : {16u, 8u, 4u})
             for (int r3 : {-1, 0, 1, 2})
-                for (int c3 : {0, 1}) {
+                for (int c3 : {-1, 0, 1}) {
                     PlanOpts o;
                     o.lc = lc;
                     o.K = K;
@@ -760,7 +762,8 @@ int lnt_tune(lnt_ctx *c, int loops) {
                     o.col3 = c3;
                     Plan tmp;
                     if (!make_plan(c->p, n, tmp, o).empty()) continue;
-                    if (r3 >= 0 || tmp.rowm) opts.push_back(o);  // -1 elsewhere is one of the others
+                    // -1 elsewhere is one of the others
+                    if ((r3 >= 0 || tmp.rowm) && (c3 >= 0 || tmp.colm)) opts.push_back(o);
                 }
     std::vector<Cand> cands;
     // warm-up long enough to capture the candidate's iteration graph, so the timed loops
@@ -914,18 +917,17 @@ static int gz_check(lnt_ctx *c, bool &passed) {
     int rc;
     // D is final for this check: read it back first and put it in canonical digits on a
     // host thread while the device runs the B squarings of E (the future's destructor
-    // waits for the thread on every return path, before xd and dd go away)
-    std::vector<uint64_t> xd(n), dd(n), de;
-    HIPCHK(c, hipMemcpyAsync(xd.data(), g.D.x, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpy (D2H)");
+    // waits for the thread on every return path, before dd goes away)
+    std::vector<uint64_t> dd(n), de;
+    HIPCHK(c, hipMemcpyAsync(dd.data(), g.D.x, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpy (D2H)");
     HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     const bool dsub2 = !c->prp && g.D.pending;
     std::future<bool> dconv;
     try {
-        dconv = std::async(std::launch::async, [c, &xd, &dd, dsub2] {
-            return to_canonical_digits(c->wid, xd.data(), dsub2, dd.data());
-        });
+        dconv = std::async(std::launch::async,
+                           [c, &dd, dsub2] { return to_canonical_digits(c->wid, dd.data(), dsub2, dd.data()); });
     } catch (const std::system_error &) {  // no thread available: convert here
-        to_canonical_digits(c->wid, xd.data(), dsub2, dd.data());
+        to_canonical_digits(c->wid, dd.data(), dsub2, dd.data());
     }
     if ((rc = copy_buf(c, g.E.x, g.Dprev.x))) return rc;
     g.E.pending = g.Dprev.pending;

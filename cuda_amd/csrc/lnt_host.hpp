@@ -2,10 +2,13 @@
 // conversions between the reference's canonical digits and the device representation.
 // Header-only; shared by the C ABI (lnt_api.hip) and the CPU emulation tests.
 #pragma once
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "gl64.hpp"
@@ -57,10 +60,11 @@ struct Plan {
     Line row, col;          // row line (also the small path's line), column line
     uint32_t K = 0;         // columns per column tile
     uint32_t G = 0;         // rows per row workgroup
+    uint32_t rowm = 0;      // matrix-core rows of 256 * rowm words (256 .. 2048; 0: none)
     uint32_t row3 = 0;      // 3-phase rows: C = row3^3 (0: 2-phase rows)
     uint32_t row3m = 0;     // mixed-radix 3-phase rows: C = row3m * rBB * rBC (0: none)
     uint32_t rBB = 0, rBC = 0;
-    uint32_t rowm = 0;      // matrix-core rows of 256 * rowm words (256 .. 2048; 0: none)
+    uint32_t colm = 0;      // matrix-core columns of 256 * colm words (256, 1024; 0: none)
     uint32_t col3 = 0;      // 3-phase columns: first radix BA (0: 2-phase columns)
     uint32_t cBB = 0, cBC = 0;  // 3-phase columns: second and third radix
     uint32_t M = 0;         // carry halo (compile-time), >= levels
@@ -73,8 +77,8 @@ struct Plan {
 inline bool same_kernels(const Plan &a, const Plan &b) {
     return a.small == b.small && a.small16 == b.small16 && a.n == b.n && a.C == b.C && a.R == b.R && a.row.B1 == b.row.B1 &&
            a.row.B2 == b.row.B2 && a.col.B1 == b.col.B1 && a.col.B2 == b.col.B2 && a.K == b.K && a.G == b.G &&
-           a.rowm == b.rowm && a.row3 == b.row3 && a.row3m == b.row3m && a.rBB == b.rBB && a.rBC == b.rBC && a.col3 == b.col3 &&
-           a.cBB == b.cBB && a.cBC == b.cBC && a.M == b.M;
+           a.rowm == b.rowm && a.row3 == b.row3 && a.row3m == b.row3m && a.rBB == b.rBB && a.rBC == b.rBC &&
+           a.colm == b.colm && a.col3 == b.col3 && a.cBB == b.cBB && a.cBC == b.cBC && a.M == b.M;
 }
 
 // Two plans order the transform domain the same way (the column tile width, rows per
@@ -137,10 +141,10 @@ inline bool split_for(uint32_t log_n, uint32_t &lc, uint32_t &lr) {
     // Small transforms are chains of latencies: 16-row columns are the cheapest (tile of 256
     // words) with rows of up to 2048 words, then 64-row columns (us per squaring, against
     // the next best split: 2^13 12.7 / 13.9, 2^14 13.3 / 14.2, 2^15 15.1 / 15.4, 2^16 16.1 / 17.2,
-    // 2^17 18.5 / 21.3, 2^18 23.0 / 25.4), 512 x 1024 at 2^19 (28.3 / 30.2).  From 2^20 rows of
-    // 4096 words; from 2^24 8192 words (0.550 against 0.581 ms with 4096 x 4096) and 16384 at
+    // 2^17 18.5 / 19.9), then 256-row columns (2^18 21.6 / 23.0, 2^19 25.1 / 28.2, 2^20 34.9 /
+    // 39.7).  From 2^20 rows of 4096 words; from 2^24 8192 words (0.550 against 0.581 ms with 4096 x 4096) and 16384 at
     // 2^26 (mixed-radix 3-phase rows), over columns of at most 4096 words.
-    static const uint8_t lcs[] = {9, 10, 11, 10, 11, 12, 10};
+    static const uint8_t lcs[] = {9, 10, 11, 10, 11, 10, 11};
     lc = log_n >= 24 ? (log_n == 26 ? 14 : 13) : log_n >= 20 ? 12 : lcs[log_n - 13];
     lr = log_n - lc;
     return lr <= 12 && lr >= 4;
@@ -154,7 +158,8 @@ struct PlanOpts {
                         // matrix cores from C = 256)
                         // (rows of 8192 and 16384 words are always 3-phase: 1 and 2
                         // select 32 or 16 words per thread)
-    int col3 = -1;      // 1: 3-phase columns (R = 512 .. 4096), 0: 2-phase, -1: default
+    int col3 = -1;      // 1: 3-phase columns (R = 512 .. 4096), 0: 2-phase, -1: default (on the
+                        // matrix cores for R = 256 and 1024)
 };
 
 // Column tile widths of the 3-phase column kernels.
@@ -184,18 +189,19 @@ inline bool plan_consistent(const Plan &pl) {
         return line == pl.n && pl.C == pl.n && pl.R == 1 && !pl.col3 && !pl.row3 && !pl.row3m;
     }
     if ((uint64_t)pl.R * pl.C != pl.n) return false;
-    const uint64_t col = pl.col3 ? (uint64_t)pl.col3 * pl.cBB * pl.cBC : (uint64_t)pl.col.B1 * pl.col.B2;
+    const uint64_t col = pl.colm ? 256ull * pl.colm : pl.col3 ? (uint64_t)pl.col3 * pl.cBB * pl.cBC : (uint64_t)pl.col.B1 * pl.col.B2;
     if (col != pl.R) return false;
-    if (!pl.K || pl.C % pl.K) return false;
+    if (!pl.K || pl.C % pl.K || (pl.colm && (pl.K != 16 || pl.col3 || (pl.colm != 1 && pl.colm != 4))))
+        return false;
     uint64_t row;
     if (pl.row3m) row = (uint64_t)pl.row3m * pl.rBB * pl.rBC;
     else if (pl.row3) row = (uint64_t)pl.row3 * pl.row3 * pl.row3;
+    else if (pl.rowm) row = 256ull * pl.rowm;
     else row = (uint64_t)pl.row.B1 * pl.row.B2;
     if (row != pl.C) return false;
     return pl.G && pl.R % pl.G == 0 && (!(pl.row3m || pl.rowm) || pl.G == 1);
 }
 
-    else if (pl.rowm) row = 256ull * pl.rowm;
 inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts opts);
 
 // Build the plan; returns an empty string on success, else the reason.  pl is rebuilt from
@@ -248,8 +254,12 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
     pl.row = line_for(lc);
     pl.col = line_for(lr);
     pl.K = pl.R >= 4096 ? 4 : pl.R >= 2048 ? 8 : 16;
-    // 3-phase columns by default for R >= 512 (measured faster there)
-    const int col3 = opts.col3 >= 0 ? opts.col3 : (pl.R >= 512 ? 1 : 0);
+    // matrix-core columns by default for R = 256 and 1024 (forward / inverse pass at 2^20 9.3 / 6.6
+    // us against 12.6 / 8.9 with the 2-phase kernels, at 2^22 33.9 / 22.0 against 34.7 / 23.9 with the
+    // 3-phase ones); 3-phase columns for 512 (as 16 x 16 x 2 with 16 waves 15.2 / 9.5 us at 2^19
+    // against 10.5 / 6.9) and above 1024
+    if (opts.col3 < 0 && (pl.R == 256 || pl.R == 1024) && (opts.K == 0 || opts.K == 16)) pl.colm = pl.R / 256;
+    const int col3 = pl.colm ? 0 : opts.col3 >= 0 ? opts.col3 : (pl.R >= 512 ? 1 : 0);
     if (col3 == 1) {
         if (pl.R < 512 || pl.R > 4096) return "3-phase columns need R = 512 .. 4096";
         pl.col3 = pl.R >= 1024 ? 16 : 8;
@@ -264,6 +274,7 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
         if (!(pl.col3 ? col3_tile_ok(pl.R, opts.K) : col_tile_ok(pl.R, opts.K))) return "unsupported column tile";
         pl.K = opts.K;
     }
+    if (pl.colm) pl.K = 16;
     pl.G = 64 / pl.row.B2;
     // 3-phase rows by default at C = 4096 (measured faster than the 2-phase rows there)
     if (pl.C > 4096) {
@@ -285,6 +296,9 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
         if (pl.C != 4096 && pl.C != 512) return "3-phase rows need C = 512 or 4096";
         pl.row3 = pl.C == 4096 ? 16 : 8;
         pl.G = pl.C == 4096 ? 1 : 4;
+    } else if (opts.row3 < 0 && pl.C >= 256) {
+        pl.rowm = pl.C / 256;
+        pl.G = 1;
     }
     return "";
 }
@@ -292,9 +306,6 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
 // Digit widths w_i = ceil(p(i+1)/n) - ceil(p i/n).
 inline void widths(uint32_t p, uint32_t n, std::vector<uint8_t> &w) {
     w.resize(n);
-    } else if (opts.row3 < 0 && pl.C >= 256) {
-        pl.rowm = pl.C / 256;
-        pl.G = 1;
     uint32_t L = ilog2(n);
     for (uint32_t i = 0; i < n; i++) {
         uint64_t e0 = ((uint64_t)p * i + n - 1) >> L, e1 = ((uint64_t)p * (i + 1) + n - 1) >> L;
@@ -336,27 +347,48 @@ inline void to_device_digits(const std::vector<uint8_t> &w, const uint64_t *d, u
 inline bool to_canonical_digits(const std::vector<uint8_t> &w, const uint64_t *x, bool sub2,
                                 uint64_t *d) {
     const size_t n = w.size();
-    std::vector<int64_t> v(n);
-    for (size_t i = 0; i < n; i++) v[i] = gl_to_i64(x[i]);
-    if (sub2) v[0] -= 2;
-    i128 carry = 0;
-    bool first = true;
-    for (int pass = 0; pass < 1000; pass++) {
-        size_t i = 0;
-        for (; i < n; i++) {
-            i128 t = (first ? (i128)v[i] : (i128)d[i]) + carry;
-            int wi = w[i];
-            i128 q = t >> wi;  // floor
-            d[i] = (uint64_t)(t - (q << wi));
-            carry = q;
-            if (!first && carry == 0) break;
+    const size_t T = std::max<size_t>(1, std::min<size_t>(8, n >> 17));
+    int64_t carry[8] = {};  // into run k
+    auto run = [&](size_t k) {
+        int64_t c = 0;
+        for (size_t i = n * k / T; i < n * (k + 1) / T; i++) {
+            int64_t v = gl_to_i64(x[i]);
+            if (sub2 && i == 0) v -= 2;
+            const int wi = w[i];
+            const int64_t mask = ((int64_t)1 << wi) - 1;
+            const int64_t t = (v & mask) + c;  // the sum of the whole words might not fit 64 bits
+            d[i] = (uint64_t)(t & mask);
+            c = (v >> wi) + (t >> wi);
         }
-        first = false;
-        if (carry == 0) break;
+        carry[(k + 1) % T] = c;
+    };
+    std::thread th[8];
+    for (size_t k = 1; k < T; k++) {
+        try {
+            th[k] = std::thread(run, k);
+        } catch (const std::system_error &) {  // no thread available
+            run(k);
+        }
+    }
+    run(0);
+    for (size_t k = 1; k < T; k++)
+        if (th[k].joinable()) th[k].join();
+    // (the carry out of digit n - 1 enters digit 0: 2^p = 1)
+    for (size_t k = 0, idle = 0; idle < T; k = (k + 1) % T) {
+        int64_t c = carry[k];
+        carry[k] = 0;
+        idle = c ? 0 : idle + 1;
+        for (size_t i = n * k / T; c && i < n * (k + 1) / T; i++) {
+            const int wi = w[i];
+            const int64_t t = (int64_t)d[i] + c;
+            d[i] = (uint64_t)(t & (((int64_t)1 << wi) - 1));
+            c = t >> wi;
+        }
+        carry[(k + 1) % T] += c;
     }
     // all-ones is 2^p - 1 = 0 (mod 2^p - 1): canonical 0
     bool all_ones = true, all_zero = true;
-    for (size_t i = 0; i < n; i++) {
+    for (size_t i = 0; i < n && (all_ones || all_zero); i++) {
         if (d[i] != (1ull << w[i]) - 1) all_ones = false;
         if (d[i] != 0) all_zero = false;
     }

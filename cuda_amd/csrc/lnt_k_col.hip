@@ -1,6 +1,12 @@
 // Instantiations of the column kernels (column lengths 64 .. 4096).
 #include "lnt_launch.hpp"
 
+// lnt_k_colm.hip
+bool lnt_launch_colm_fwd(const lnt::Plan &pl, const LntParams &P, bool sub2, hipStream_t s);
+bool lnt_launch_colm_inv(const lnt::Plan &pl, const LntParams &P, hipStream_t s);
+bool lnt_launch_batch_colm_fwd(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s);
+bool lnt_launch_batch_colm_inv(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s);
+
 template <int B1, int B2, int K>
 static bool go_col_fwd(const lnt::Plan &pl, const LntParams &P, bool sub2, hipStream_t s) {
     dim3 grid(pl.C / K), block(K * B2);
@@ -37,6 +43,7 @@ static bool go_col3_fwd(const lnt::Plan &pl, const LntParams &P, bool sub2, hipS
 
 bool lnt_launch_col_fwd(const lnt::Plan &pl, const LntParams &P, bool sub2, hipStream_t s) {
     if (!lnt::plan_consistent(pl)) return false;  // a kernel of another shape would run out of bounds
+    if (pl.colm) return lnt_launch_colm_fwd(pl, P, sub2, s);
     if (pl.col3) {
 #define C3F(ba, bb, bc, k) \
     if (pl.col3 == ba && pl.cBB == bb && pl.cBC == bc && pl.K == k) return go_col3_fwd<ba, bb, bc, k>(pl, P, sub2, s);
@@ -65,6 +72,7 @@ static bool go_col3_inv(const lnt::Plan &pl, const LntParams &P, hipStream_t s) 
 
 bool lnt_launch_col_inv(const lnt::Plan &pl, const LntParams &P, hipStream_t s) {
     if (!lnt::plan_consistent(pl)) return false;  // a kernel of another shape would run out of bounds
+    if (pl.colm) return lnt_launch_colm_inv(pl, P, s);
     if (pl.col3) {
 #define C3I(ba, bb, bc, k) \
     if (pl.col3 == ba && pl.cBB == bb && pl.cBC == bc && pl.K == k) return go_col3_inv<ba, bb, bc, k>(pl, P, s);
@@ -80,6 +88,7 @@ bool lnt_launch_col_inv(const lnt::Plan &pl, const LntParams &P, hipStream_t s) 
 
 bool lnt_launch_batch_col_fwd(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s) {
     if (!lnt::plan_consistent(pl)) return false;  // a kernel of another shape would run out of bounds
+    if (pl.colm) return lnt_launch_batch_colm_fwd(pl, Ps, count, s);
     if (pl.col3) {
 #define C3F(ba, bb, bc, k)                                                                                 \
     if (pl.col3 == ba && pl.cBB == bb && pl.cBC == bc && pl.K == k) {                                      \
@@ -110,6 +119,7 @@ bool lnt_launch_batch_col_fwd(const lnt::Plan &pl, const LntParams *Ps, u32 coun
 
 bool lnt_launch_batch_col_inv(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s) {
     if (!lnt::plan_consistent(pl)) return false;  // a kernel of another shape would run out of bounds
+    if (pl.colm) return lnt_launch_batch_colm_inv(pl, Ps, count, s);
     if (pl.col3) {
 #define C3I(ba, bb, bc, k)                                                                                \
     if (pl.col3 == ba && pl.cBB == bb && pl.cBC == bc && pl.K == k) {                                     \

@@ -121,6 +121,30 @@ GL_HD void lnt_carry_run(int64_t (&v)[M + K], u32 p, u32 log_n, u64 g0, u32 leve
     }
 }
 
+// Carry of one piece of a 16-digit run staged in LDS: PR neighbouring threads of one wave share
+// the run, thread s takes its digits [s PK, s PK + PK).  row0 is the LDS word of the run's first
+// digit, digit g0 of the residue; h holds the M words before the run (for s = 0).  The digits
+// go back to LDS as d + 2^31 for the biased weight multiply, else field-encoded.
+template <int M, int PK, int PR>
+LNT_KFN void lnt_carry_piece(LView lds, u32 row0, int s, const u64 (&h)[M], const LntParams &P, u64 g0, bool sub2) {
+    int64_t v[M + PK];
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const int at = PK * s - M + j;  // negative: before the run
+        u64 x = h[j];
+        if (PR > 1 && s) x = (PK < M && at < 0) ? P.x[(g0 + P.n + at) & (P.n - 1)] : lds[row0 + (u32)at];
+        v[j] = gl_to_i64(x);
+    }
+#pragma unroll
+    for (int j = 0; j < PK; j++) v[M + j] = gl_to_i64(lds[row0 + (u32)(PK * s + j)]);
+    LNT_WAVE_SYNC();  // every word read before any is overwritten
+    lnt_carry_run<M, PK>(v, P.p, P.log_n, g0 + PK * s, P.levels, sub2);
+#pragma unroll
+    for (int j = 0; j < PK; j++)
+        lds[row0 + (u32)(PK * s + j)] =
+            P.bias ? (u64)(u32)(v[M + j] + (int64_t(1) << 31)) : gl_from_i64(v[M + j]);
+}
+
 constexpr int LNT_PAD = 1;
 
 // ------------------------------------------------------------------ column forward
@@ -466,6 +490,154 @@ LNT_KFN void lnt_col3_inv_body(int tid, int bid, LView lds, const LntParams &P) 
     }
 }
 
+// ------------------------------------------------------------------ columns on the matrix cores
+// Columns of R = 256 S words (S = 1, 4), 16 adjacent columns per workgroup of 16 waves,
+// 4 S words per thread: the 16 columns of a tile are the 16 DFTs of a matrix instruction, so
+// lane (q, n) works on column c0 + n throughout.  With row r = a1 + 16 S j, a1 = a + S b:
+//   phase 1: group a1 = S w + g of wave w: DFT over j -> k2, twiddle omega_R^(a1 k2)         (twc)
+//   phase 2: group (k2 = w, a = g): DFT over b -> kb, twiddle omega_16S^(a kb)               (twc2)
+//   phase 3: S-point DFTs over a = g, in registers -> k3 (bit-reversed)
+// Frequency k2 + 16 (kb + 16 k3) goes to slot (16 k2 + kb) S + k3, where lnt_tw4_m puts its 4-step
+// twiddle.  Every DFT writes the LDS words that it read, so only the exchange between phases 1
+// and 2 and the hand-over of the carried digits wait for other waves.  LDS word (row r, column
+// n) at RS r + n; RS keeps the words of neighbouring lane groups (2 S rows apart in phase 2) on
+// the two halves of the banks.
+template <int S>
+struct LntColM {
+    static constexpr int R = 256 * S, L = 16 * S;
+    static constexpr int RS = S == 1 ? 24 : 18;
+    static constexpr u32 LDS = (u32)(R * RS);
+};
+
+template <int S, int M>
+LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, bool sub2) {
+    using Z = LntColM<S>;
+    constexpr int RS = Z::RS, L = Z::L;
+    constexpr int PR = 4 / S, PK = 4 * S;  // carry: threads per row, digits per thread
+    const LntLane16 T = lnt_lane16(tid);
+    const int q = T.q, n = T.n, w = T.w;
+    const u64 C = P.C, c0 = (u64)bid * 16;
+    // the tile, 16 columns of a row by 16 lanes; row r's M digits before it by the thread of
+    // its first piece
+    {
+        u64 a[PK], h[M];
+#pragma unroll
+        for (int i = 0; i < PK; i++) a[i] = P.x[c0 + n + C * (u64)(tid / 16 + 64 * i)];
+        const u64 g0 = C * (u64)(tid / PR) + c0;
+#pragma unroll
+        for (int j = 0; j < M; j++) h[j] = tid % PR == 0 ? P.x[(g0 + P.n - M + j) & (P.n - 1)] : 0;
+#pragma unroll
+        for (int i = 0; i < PK; i++) lds[(u32)(RS * (tid / 16 + 64 * i) + n)] = a[i];
+        LNT_SYNC();
+        // carry + (-2): PR neighbouring threads per row run of 16 digits
+        lnt_carry_piece<M, PK, PR>(lds, (u32)(RS * (tid / PR)), tid % PR, h, P, g0, sub2);
+    }
+    LntM16 Mx;
+    lnt_m16_load(Mx, tid);
+    const u32 ec = lnt_wexp(P.p, P.n, c0 + n), mC = 0u - P.p * P.C;  // weight slot parameters
+    LNT_SYNC();
+    // phase 1 with the weights
+#pragma unroll 1
+    for (int a1 = S * w; a1 < S * w + S; a1++) {
+        u64 z[4], tw[4];
+        const u32 at = (u32)(RS * a1 + n);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int j = lnt_m16_word(q, e);
+            const u32 sl = lnt_wslot(ec, mC, P.n, (u32)(a1 + L * j));
+            const u64 d = lds[at + (u32)(RS * L * j)];
+            z[e] = P.bias ? gl_mul_biased((u32)d, P.w[2 * sl], P.w[2 * sl + 1]) : gl_mul(d, P.w[2 * sl]);
+            tw[e] = P.twc[L * brev_v16(j) + a1];
+        }
+        lnt_m16_dft(Mx, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) lds[at + (u32)(RS * L * lnt_m16_word(q, v))] = gl_mmul(z[v], tw[v]);
+    }
+    LNT_SYNC();
+    // phase 2 (S = 1: the last); with S > 1 its words go through this lane's own LDS places to phase 3
+#pragma unroll 1
+    for (int g = 0; g < S; g++) {
+        u64 z[4];
+        const u32 at = (u32)(RS * (L * w + g) + n);
+#pragma unroll
+        for (int e = 0; e < 4; e++) z[e] = lds[at + (u32)(RS * S * lnt_m16_word(q, e))];
+        lnt_m16_dft(Mx, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int kb = lnt_m16_word(q, v);
+            if (S == 1) P.y[c0 + n + C * (u64)(16 * w + kb)] = z[v];
+            else lds[at + (u32)(RS * S * kb)] = gl_mmul(z[v], P.twc2[S * brev_v16(kb) + g]);
+        }
+    }
+    if (S == 1) return;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int kb = lnt_m16_word(q, v);
+        u64 t[S];
+#pragma unroll
+        for (int g = 0; g < S; g++) t[g] = lds[(u32)(RS * (L * w + g + S * kb) + n)];
+        dft_fwd<S>(t);
+#pragma unroll
+        for (int g = 0; g < S; g++) P.y[c0 + n + C * (u64)((16 * w + kb) * S + brev_c<S>(g))] = t[g];
+    }
+}
+
+template <int S>
+LNT_KFN void lnt_colm_inv_body(int tid, int bid, LView lds, const LntParams &P) {
+    using Z = LntColM<S>;
+    constexpr int RS = Z::RS, L = Z::L;
+    const LntLane16 T = lnt_lane16(tid);
+    const int q = T.q, n = T.n, w = T.w;
+    const u64 C = P.C, c = (u64)bid * 16 + n;
+    // phase 3 inverse over k3 and the inverse phase-2 twiddle, into this lane's own LDS places
+    if (S > 1) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int kb = lnt_m16_word(q, v);
+            u64 t[S];
+#pragma unroll
+            for (int g = 0; g < S; g++) t[g] = P.y[c + C * (u64)((16 * w + kb) * S + brev_c<S>(g))];
+            dft_inv<S>(t);
+#pragma unroll
+            for (int g = 0; g < S; g++)
+                lds[(u32)(RS * (L * w + g + S * kb) + n)] = gl_mmul(t[g], P.itwc2[S * brev_v16(kb) + g]);
+        }
+    }
+    LntM16 Mx;
+    lnt_m16_load(Mx, tid);
+    // phase 2 inverse: output place v is b = -lnt_m16_word(q, v)
+#pragma unroll 1
+    for (int g = 0; g < S; g++) {
+        u64 z[4], tw[4];
+        const u32 at = (u32)(RS * (L * w + g) + n);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int kb = lnt_m16_word(q, e);
+            z[e] = S == 1 ? P.y[c + C * (u64)(16 * w + kb)] : lds[at + (u32)(RS * S * kb)];
+            tw[e] = P.itwc[L * brev_v16(w) + g + S * lnt_m16_neg(q, e)];
+        }
+        LNT_WAVE_SYNC();
+        lnt_m16_dft(Mx, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) lds[at + (u32)(RS * S * lnt_m16_neg(q, v))] = gl_mmul(z[v], tw[v]);
+    }
+    const u32 ec = lnt_wexp(P.p, P.n, c), mC = 0u - P.p * P.C;  // weight slot parameters
+    LNT_SYNC();
+    // phase 1 inverse, unweight, store
+#pragma unroll 1
+    for (int a1 = S * w; a1 < S * w + S; a1++) {
+        u64 y[4], uv[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            y[e] = lds[(u32)(RS * (L * lnt_m16_word(q, e) + a1) + n)];
+            uv[e] = P.uw[lnt_wslot(ec, mC, P.n, (u32)(a1 + L * lnt_m16_neg(q, e)))];
+        }
+        lnt_m16_dft(Mx, y);
+#pragma unroll
+        for (int v = 0; v < 4; v++) P.x[c + C * (u64)(a1 + L * lnt_m16_neg(q, v))] = gl_mmul(y[v], uv[v]);
+    }
+}
+
 // ------------------------------------------------------------------ row pass
 // grid: R / G workgroups, block: G * B2 threads (G rows per workgroup).
 // LDS words: G * B1 * (B2 + PAD).
@@ -627,174 +799,6 @@ LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
     for (int j = 0; j < B; j++) P.y[base + t + (u64)T * j] = gl_mmul(a[j], iv[MODE == LNT_FORWARD ? 0 : j]);
 }
 
-// ------------------------------------------------------------------ 4096-word rows on the matrix cores
-// The row pass for C = 4096 = 16^3 with the 16-point DFTs of mdft.hpp: one row per workgroup
-// of W = 16 / GW waves, GW groups of 16 DFTs per wave and phase (4 GW words per thread).  With
-// i = i1 + 256 j, i1 = a + 16 b; group h = GW w + g of wave w, lane (q, n):
-//   phase 1: DFTs i1 = 16 h + n over j -> k2, twiddle omega_C^(i1 k2)     (twr)
-//   phase 2: DFTs (k2 = h, a = n) over b -> kb, twiddle omega_256^(a kb)  (twr2)
-//   phase 3: DFTs (k2 = h, kb = n) over a; square (or the product modes); the inverse takes
-//            the result as it lies.
-// A wave keeps its k2 between phase 1 and the inverse phase 2, so only the exchanges around
-// these wait for the other waves.  LDS word (row r of 16 words, x) at 18 r + x: runs of 16 words
-// start 16-byte aligned and 16 neighbouring runs cover all 64 banks, so the reads of adjacent
-// word pairs are 128-bit and free of conflicts.  Transform-domain slot for MODE 1/2: base + 4 GW t + 4 g + place.
-constexpr u32 LNT_ROW16_LDS = 256 * 18;
-template <int GW, int MODE = LNT_SQUARE>
-LNT_KFN void lnt_row16_body(int tid, int bid, LView lds, const LntParams &P) {
-    const int w = LNT_UNIFORM(tid / 64), q = (tid % 64) / 16, n = tid % 16;
-    const u64 base = (u64)4096 * (u64)bid;
-    LntM16 M;
-    u64 z[4], tw[4];
-    // phase 1
-#pragma unroll 1
-    for (int h = GW * w; h < GW * w + GW; h++) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int k = lnt_m16_word(q, e);
-            const u64 idx = base + 16 * h + n + 256 * k;
-            z[e] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
-            tw[e] = P.twr[256 * brev_v16(k) + 16 * h + n];
-        }
-        if (h == GW * w) lnt_m16_load(M, tid);
-        lnt_m16_dft(M, z);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            lds[(u32)(288 * lnt_m16_word(q, v) + 18 * n + h)] = gl_mmul(z[v], tw[v]);
-    }
-    LNT_SYNC();
-    // phases 2 and 3, the pointwise step and their inverses
-#pragma unroll 1
-    for (int h = GW * w; h < GW * w + GW; h++) {
-        const u32 row = (u32)(288 * h), own = row + (u32)(18 * n + 2 * q);  // this lane's words of run n
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            z[e] = lds[own + lnt_m16_word(0, e)];
-            tw[e] = P.twr2[16 * brev_v16(lnt_m16_word(q, e)) + n];
-        }
-        lnt_m16_dft(M, z);
-        LNT_WAVE_SYNC();
-#pragma unroll
-        for (int v = 0; v < 4; v++) lds[(u32)(row + 18 * lnt_m16_word(q, v) + n)] = gl_mmul(z[v], tw[v]);
-        LNT_WAVE_SYNC();
-#pragma unroll
-        for (int e = 0; e < 4; e++) z[e] = lds[own + lnt_m16_word(0, e)];
-        if (MODE != LNT_FORWARD) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) tw[v] = P.itwr2[16 * brev_v16(n) + ((16 - lnt_m16_word(q, v)) & 15)];
-        }
-        lnt_m16_dft(M, z);
-        LNT_WAVE_SYNC();
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const u64 slot = base + 4 * GW * (u64)tid + 4 * (h - GW * w) + v;
-            if (MODE == LNT_FORWARD) P.y[slot] = z[v];
-            else z[v] = gl_mmul(z[v], MODE == LNT_MULTIPLY ? P.f[slot] : z[v]);
-        }
-        if (MODE == LNT_FORWARD) continue;
-        lnt_m16_dft(M, z);  // inverse phase 3: output place v is the word -k
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            lds[(u32)(row + 18 * ((16 - lnt_m16_word(q, v)) & 15) + n)] = gl_mmul(z[v], tw[v]);
-        LNT_WAVE_SYNC();
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            z[e] = lds[own + lnt_m16_word(0, e)];
-            tw[e] = P.itwr[256 * brev_v16(h) + n + 16 * ((16 - lnt_m16_word(q, e)) & 15)];
-        }
-        lnt_m16_dft(M, z);  // inverse phase 2
-        LNT_WAVE_SYNC();
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            lds[(u32)(row + 18 * n + ((16 - lnt_m16_word(q, v)) & 15))] = gl_mmul(z[v], tw[v]);
-    }
-    if (MODE == LNT_FORWARD) return;
-    LNT_SYNC();
-    // inverse phase 1, inverse 4-step twiddle, store
-#pragma unroll 1
-    for (int h = GW * w; h < GW * w + GW; h++) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            z[e] = lds[(u32)(288 * lnt_m16_word(q, e) + 18 * n + h)];
-            tw[e] = P.itw4[base + 16 * h + n + 256 * ((16 - lnt_m16_word(q, e)) & 15)];
-        }
-        lnt_m16_dft(M, z);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            P.y[base + 16 * h + n + 256 * ((16 - lnt_m16_word(q, v)) & 15)] = gl_mmul(z[v], tw[v]);
-    }
-}
-
-// ------------------------------------------------------------------ mixed-radix 3-phase rows
-// Rows of C = BA * BB * BC words (8192 = 32*16*16 or 16*32*16, 16384 = 32*32*16 or
-// 16*32*32), one row per workgroup of A = BB * BC threads holding BA words each.  The
-// phases are those of the 3-phase columns (phase 1 over j of words t + A j; phase 2 items
-// (k1, u), BA * BC of them; phase 3 items (k1, k2), BA * BB of them), with the 4-step
-// twiddles at load and store and the square (or product) in the middle.  The phase-2
-// twiddle is applied where phase 3 reads (and its inverse where inverse phase 3 writes).
-// With BA = 16 a phase may have fewer items than threads (the rest wait at the barrier):
-// 16 words per thread keep the register count low enough for twice the waves of BA = 32.
-// LDS word of (k1, a = u + BC v): k1 * RS + v * (BC + 1) + u (padded runs).
-template <int BA, int BB, int BC>
-struct LntRow3m {
-    static constexpr int A = BB * BC, C = BA * A;
-    static constexpr int N2 = BA * BC, N3 = BA * BB;  // phase 2 / phase 3 items
-    static constexpr int Q2 = (N2 + A - 1) / A, Q3 = (N3 + A - 1) / A;  // items per thread
-    static constexpr int RS = BB * (BC + 1) + 1;
-    static constexpr u32 LDS = (u32)(BA * RS);
-    static_assert(N2 % A == 0 || A % N2 == 0, "phase 2 items");
-    static_assert(N3 % A == 0 || A % N3 == 0, "phase 3 items");
-};
-
-template <int BA, int BB, int BC, int MODE = LNT_SQUARE>
-LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
-    using S = LntRow3m<BA, BB, BC>;
-    constexpr int A = S::A, RS = S::RS, N2 = S::N2, N3 = S::N3, Q2 = S::Q2, Q3 = S::Q3;
-    const int t = tid;
-    const u64 base = (u64)P.C * (u64)bid;
-    auto pos = [](int k1, int a) { return (u32)(k1 * RS + (a / BC) * (BC + 1) + a % BC); };
-    u64 a[BA];
-#pragma unroll
-    for (int j = 0; j < BA; j++) {
-        const u64 idx = base + t + (u64)A * j;
-        a[j] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
-    }
-    // phase 1
-    dft_fwd<BA>(a);
-#pragma unroll
-    for (int rho = 1; rho < BA; rho++) a[rho] = gl_mmul(a[rho], P.twr[(u64)rho * A + t]);
-#pragma unroll
-    for (int rho = 0; rho < BA; rho++) lds[pos(brev_c<BA>(rho), t)] = a[rho];
-    LNT_SYNC();
-    // phase 2 (each item rewrites exactly the LDS words it read)
-#pragma unroll
-    for (int q = 0; q < Q2; q++) {
-        const int I = q * A + t, k1 = I / BC, u = I % BC;
-        if (N2 >= A || I < N2) {
-            u64 b[BB];
-#pragma unroll
-            for (int v = 0; v < BB; v++) b[v] = lds[pos(k1, u + BC * v)];
-            dft_fwd<BB>(b);
-#pragma unroll
-            for (int rho = 0; rho < BB; rho++) lds[pos(k1, u + BC * brev_c<BB>(rho))] = b[rho];
-        }
-    }
-    LNT_SYNC();
-    // phase 3 (with the phase-2 twiddle w_A^(u k2) at the read, where every thread has an
-    // item: phase 2 keeps only its DFT registers live), the pointwise step, inverse phase 3
-    // and the inverse phase-2 twiddle.  Item q of thread t: slots (q * A + t) * BC + rho.
-#pragma unroll
-    for (int q = 0; q < Q3; q++) {
-        const int I = q * A + t, k1 = I / BB, k2 = I % BB;
-        if (N3 >= A || I < N3) {
-            const u64 tb = (u64)brev_c<BB>(k2) * BC;  // twr2 row of k2
-            u64 e[BC];
-#pragma unroll
-            for (int u = 0; u < BC; u++) e[u] = gl_mmul(lds[pos(k1, u + BC * k2)], P.twr2[tb + u]);
-            dft_fwd<BC>(e);
-            const u64 so = base + (u64)I * BC;
-            if (MODE == LNT_FORWARD) {
-#pragma unroll
 // ------------------------------------------------------------------ lines of 256 S words on the matrix cores
 // The transform of a line of L = 256 S words (S = 1, 2, 4, 8, 16) by S waves, four words per
 // thread: L = 16 * 16 * S with the 16-point DFTs of mdft.hpp in phases 1 and 2 and an S-point
@@ -966,6 +970,174 @@ LNT_KFN void lnt_rowm_body(int tid, int bid, LView lds, const LntParams &P) {
     for (int v = 0; v < 4; v++) P.y[base + L.id + 16 * S * lnt_m16_neg(L.q, v)] = gl_mmul(z[v], t4[v]);
 }
 
+// ------------------------------------------------------------------ 4096-word rows on the matrix cores
+// The row pass for C = 4096 = 16^3 with the 16-point DFTs of mdft.hpp: one row per workgroup
+// of W = 16 / GW waves, GW groups of 16 DFTs per wave and phase (4 GW words per thread).  With
+// i = i1 + 256 j, i1 = a + 16 b; group h = GW w + g of wave w, lane (q, n):
+//   phase 1: DFTs i1 = 16 h + n over j -> k2, twiddle omega_C^(i1 k2)     (twr)
+//   phase 2: DFTs (k2 = h, a = n) over b -> kb, twiddle omega_256^(a kb)  (twr2)
+//   phase 3: DFTs (k2 = h, kb = n) over a; square (or the product modes); the inverse takes
+//            the result as it lies.
+// A wave keeps its k2 between phase 1 and the inverse phase 2, so only the exchanges around
+// these wait for the other waves.  LDS word (row r of 16 words, x) at 18 r + x: runs of 16 words
+// start 16-byte aligned and 16 neighbouring runs cover all 64 banks, so the reads of adjacent
+// word pairs are 128-bit and free of conflicts.  Transform-domain slot for MODE 1/2: base + 4 GW t + 4 g + place.
+constexpr u32 LNT_ROW16_LDS = 256 * 18;
+template <int GW, int MODE = LNT_SQUARE>
+LNT_KFN void lnt_row16_body(int tid, int bid, LView lds, const LntParams &P) {
+    const int w = LNT_UNIFORM(tid / 64), q = (tid % 64) / 16, n = tid % 16;
+    const u64 base = (u64)4096 * (u64)bid;
+    LntM16 M;
+    u64 z[4], tw[4];
+    // phase 1
+#pragma unroll 1
+    for (int h = GW * w; h < GW * w + GW; h++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int k = lnt_m16_word(q, e);
+            const u64 idx = base + 16 * h + n + 256 * k;
+            z[e] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
+            tw[e] = P.twr[256 * brev_v16(k) + 16 * h + n];
+        }
+        if (h == GW * w) lnt_m16_load(M, tid);
+        lnt_m16_dft(M, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[(u32)(288 * lnt_m16_word(q, v) + 18 * n + h)] = gl_mmul(z[v], tw[v]);
+    }
+    LNT_SYNC();
+    // phases 2 and 3, the pointwise step and their inverses
+#pragma unroll 1
+    for (int h = GW * w; h < GW * w + GW; h++) {
+        const u32 row = (u32)(288 * h), own = row + (u32)(18 * n + 2 * q);  // this lane's words of run n
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            z[e] = lds[own + lnt_m16_word(0, e)];
+            tw[e] = P.twr2[16 * brev_v16(lnt_m16_word(q, e)) + n];
+        }
+        lnt_m16_dft(M, z);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 4; v++) lds[(u32)(row + 18 * lnt_m16_word(q, v) + n)] = gl_mmul(z[v], tw[v]);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int e = 0; e < 4; e++) z[e] = lds[own + lnt_m16_word(0, e)];
+        if (MODE != LNT_FORWARD) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) tw[v] = P.itwr2[16 * brev_v16(n) + ((16 - lnt_m16_word(q, v)) & 15)];
+        }
+        lnt_m16_dft(M, z);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const u64 slot = base + 4 * GW * (u64)tid + 4 * (h - GW * w) + v;
+            if (MODE == LNT_FORWARD) P.y[slot] = z[v];
+            else z[v] = gl_mmul(z[v], MODE == LNT_MULTIPLY ? P.f[slot] : z[v]);
+        }
+        if (MODE == LNT_FORWARD) continue;
+        lnt_m16_dft(M, z);  // inverse phase 3: output place v is the word -k
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[(u32)(row + 18 * ((16 - lnt_m16_word(q, v)) & 15) + n)] = gl_mmul(z[v], tw[v]);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            z[e] = lds[own + lnt_m16_word(0, e)];
+            tw[e] = P.itwr[256 * brev_v16(h) + n + 16 * ((16 - lnt_m16_word(q, e)) & 15)];
+        }
+        lnt_m16_dft(M, z);  // inverse phase 2
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            lds[(u32)(row + 18 * n + ((16 - lnt_m16_word(q, v)) & 15))] = gl_mmul(z[v], tw[v]);
+    }
+    if (MODE == LNT_FORWARD) return;
+    LNT_SYNC();
+    // inverse phase 1, inverse 4-step twiddle, store
+#pragma unroll 1
+    for (int h = GW * w; h < GW * w + GW; h++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            z[e] = lds[(u32)(288 * lnt_m16_word(q, e) + 18 * n + h)];
+            tw[e] = P.itw4[base + 16 * h + n + 256 * ((16 - lnt_m16_word(q, e)) & 15)];
+        }
+        lnt_m16_dft(M, z);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            P.y[base + 16 * h + n + 256 * ((16 - lnt_m16_word(q, v)) & 15)] = gl_mmul(z[v], tw[v]);
+    }
+}
+
+// ------------------------------------------------------------------ mixed-radix 3-phase rows
+// Rows of C = BA * BB * BC words (8192 = 32*16*16 or 16*32*16, 16384 = 32*32*16 or
+// 16*32*32), one row per workgroup of A = BB * BC threads holding BA words each.  The
+// phases are those of the 3-phase columns (phase 1 over j of words t + A j; phase 2 items
+// (k1, u), BA * BC of them; phase 3 items (k1, k2), BA * BB of them), with the 4-step
+// twiddles at load and store and the square (or product) in the middle.  The phase-2
+// twiddle is applied where phase 3 reads (and its inverse where inverse phase 3 writes).
+// With BA = 16 a phase may have fewer items than threads (the rest wait at the barrier):
+// 16 words per thread keep the register count low enough for twice the waves of BA = 32.
+// LDS word of (k1, a = u + BC v): k1 * RS + v * (BC + 1) + u (padded runs).
+template <int BA, int BB, int BC>
+struct LntRow3m {
+    static constexpr int A = BB * BC, C = BA * A;
+    static constexpr int N2 = BA * BC, N3 = BA * BB;  // phase 2 / phase 3 items
+    static constexpr int Q2 = (N2 + A - 1) / A, Q3 = (N3 + A - 1) / A;  // items per thread
+    static constexpr int RS = BB * (BC + 1) + 1;
+    static constexpr u32 LDS = (u32)(BA * RS);
+    static_assert(N2 % A == 0 || A % N2 == 0, "phase 2 items");
+    static_assert(N3 % A == 0 || A % N3 == 0, "phase 3 items");
+};
+
+template <int BA, int BB, int BC, int MODE = LNT_SQUARE>
+LNT_KFN void lnt_row3m_body(int tid, int bid, LView lds, const LntParams &P) {
+    using S = LntRow3m<BA, BB, BC>;
+    constexpr int A = S::A, RS = S::RS, N2 = S::N2, N3 = S::N3, Q2 = S::Q2, Q3 = S::Q3;
+    const int t = tid;
+    const u64 base = (u64)P.C * (u64)bid;
+    auto pos = [](int k1, int a) { return (u32)(k1 * RS + (a / BC) * (BC + 1) + a % BC); };
+    u64 a[BA];
+#pragma unroll
+    for (int j = 0; j < BA; j++) {
+        const u64 idx = base + t + (u64)A * j;
+        a[j] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
+    }
+    // phase 1
+    dft_fwd<BA>(a);
+#pragma unroll
+    for (int rho = 1; rho < BA; rho++) a[rho] = gl_mmul(a[rho], P.twr[(u64)rho * A + t]);
+#pragma unroll
+    for (int rho = 0; rho < BA; rho++) lds[pos(brev_c<BA>(rho), t)] = a[rho];
+    LNT_SYNC();
+    // phase 2 (each item rewrites exactly the LDS words it read)
+#pragma unroll
+    for (int q = 0; q < Q2; q++) {
+        const int I = q * A + t, k1 = I / BC, u = I % BC;
+        if (N2 >= A || I < N2) {
+            u64 b[BB];
+#pragma unroll
+            for (int v = 0; v < BB; v++) b[v] = lds[pos(k1, u + BC * v)];
+            dft_fwd<BB>(b);
+#pragma unroll
+            for (int rho = 0; rho < BB; rho++) lds[pos(k1, u + BC * brev_c<BB>(rho))] = b[rho];
+        }
+    }
+    LNT_SYNC();
+    // phase 3 (with the phase-2 twiddle w_A^(u k2) at the read, where every thread has an
+    // item: phase 2 keeps only its DFT registers live), the pointwise step, inverse phase 3
+    // and the inverse phase-2 twiddle.  Item q of thread t: slots (q * A + t) * BC + rho.
+#pragma unroll
+    for (int q = 0; q < Q3; q++) {
+        const int I = q * A + t, k1 = I / BB, k2 = I % BB;
+        if (N3 >= A || I < N3) {
+            const u64 tb = (u64)brev_c<BB>(k2) * BC;  // twr2 row of k2
+            u64 e[BC];
+#pragma unroll
+            for (int u = 0; u < BC; u++) e[u] = gl_mmul(lds[pos(k1, u + BC * k2)], P.twr2[tb + u]);
+            dft_fwd<BC>(e);
+            const u64 so = base + (u64)I * BC;
+            if (MODE == LNT_FORWARD) {
+#pragma unroll
                 for (int i = 0; i < BC; i++) P.y[so + i] = e[i];
                 continue;
             }
@@ -1158,6 +1330,7 @@ LNT_KFN void lnt_small16_body(int tid, LView lds, const LntParams &P, u32 iters,
         line16_load_itw2<S>(T, L, P);
         line16_load_itw1<S>(T, L, P);
     }
+    const u64 r2 = gl_mul(GL_R, GL_R);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         // unweight of output place v, times 2^128: one 2^64 for its Montgomery multiply and one
@@ -1194,6 +1367,7 @@ LNT_KFN void lnt_small16_body(int tid, LView lds, const LntParams &P, u32 iters,
             line16_load_tw1<S>(T, L, P);
         }
         LNT_SYNC();
+        // weights from B, the line in A, unweights into B: the residue of the next iteration
         u64 z[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -1252,12 +1426,19 @@ GL_HD u64 lnt_tw4_3(u64 omega_n, u32 C, u32 BA, u32 BB, u32 BC, u64 idx) {
     return gl_mul(gl_pow(omega_n, (u64)c * kcol), GL_R);
 }
 
+// 4-step twiddle of a matrix-core column (256 S words): slot (16 k2 + kb) S + k3 holds frequency
+// k2 + 16 (kb + 16 k3).
+GL_HD u64 lnt_tw4_m(u64 omega_n, u32 C, u32 S, u64 idx) {
+    const u32 c = (u32)(idx % C), s = (u32)(idx / C);
+    const u32 k2 = s / (16 * S), kb = s / S % 16, k3 = s % S;
+    return gl_mul(gl_pow(omega_n, (u64)c * (k2 + 16 * (kb + 16 * k3))), GL_R);
+}
+
 // Large-path weight tables (the factorisation at lnt_wexp), row slots 2r + h.
 // Unweights: B^f_r (B the inverse weight base), times m = 2 when h = 1, times GL_R^2: one
 // GL_R for the Montgomery multiply that applies it, one for the 2^-64 the square left.
 GL_HD u64 lnt_row_factor(u64 B, u64 m, u32 p, u32 n, u32 C, u32 slot) {
     const u64 v = gl_mul(gl_pow(B, lnt_wexp(p, n, (u64)C * (slot >> 1))), gl_mul(GL_R, GL_R));
-    const u64 r2 = gl_mul(GL_R, GL_R);
     return (slot & 1) ? gl_mul(v, m) : v;
 }
 // Weights: word i is half of the pair (w, -2^31 w) of slot i / 2 (gl_mul_biased takes both),
@@ -1280,4 +1461,3 @@ GL_HD u64 lnt_weight(u64 Bw, u32 p, u32 n, u32 i) {
     u32 r = (u32)((u64)p * i) & (n - 1);
     return gl_pow(Bw, (u64)(n - r));
 }
-        // weights from B, the line in A, unweights into B: the residue of the next iteration

@@ -74,6 +74,19 @@ __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) 
     lnt_row3_body<B, G, MODE>(threadIdx.x, blockIdx.x, LView{smem, W}, P);
 }
 
+// columns of 256 S words on the matrix cores
+template <int S, int M>
+__global__ __launch_bounds__(1024) void lnt_k_colm_fwd(LntParams P, int sub2) {
+    __shared__ __align__(16) u64 smem[LntColM<S>::LDS];
+    lnt_colm_fwd_body<S, M>(threadIdx.x, lnt_xcd_bid(blockIdx.x, gridDim.x), LView{smem, LntColM<S>::LDS}, P, sub2 != 0);
+}
+
+template <int S>
+__global__ __launch_bounds__(1024) void lnt_k_colm_inv(LntParams P) {
+    __shared__ __align__(16) u64 smem[LntColM<S>::LDS];
+    lnt_colm_inv_body<S>(threadIdx.x, lnt_xcd_bid(blockIdx.x, gridDim.x), LView{smem, LntColM<S>::LDS}, P);
+}
+
 // rows of 256 S words on the matrix cores
 template <int S, int MODE>
 __global__ __launch_bounds__(64 * S) void lnt_k_rowm(LntParams P) {
@@ -192,6 +205,25 @@ __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) 
     const LntParams P = Ps[blockIdx.x / wgs];
     if (P.n == 0) return;  // an empty slot of the batch
     lnt_row3_body<B, G>(threadIdx.x, blockIdx.x % wgs, LView{smem, W}, P);
+}
+
+// (members interleaved as in lnt_kb_col_fwd)
+template <int S, int M>
+__global__ __launch_bounds__(1024) void lnt_kb_colm_fwd(const LntParams *__restrict__ Ps, u32 wgs) {
+    __shared__ __align__(16) u64 smem[LntColM<S>::LDS];
+    const u32 b = lnt_xcd_bid(blockIdx.x, gridDim.x), slots = gridDim.x / wgs;
+    const LntParams P = Ps[b % slots];
+    if (P.n == 0) return;  // an empty slot of the batch
+    lnt_colm_fwd_body<S, M>(threadIdx.x, b / slots, LView{smem, LntColM<S>::LDS}, P, P.sub2 != 0);
+}
+
+template <int S>
+__global__ __launch_bounds__(1024) void lnt_kb_colm_inv(const LntParams *__restrict__ Ps, u32 wgs) {
+    __shared__ __align__(16) u64 smem[LntColM<S>::LDS];
+    const u32 b = lnt_xcd_bid(blockIdx.x, gridDim.x), slots = gridDim.x / wgs;
+    const LntParams P = Ps[b % slots];
+    if (P.n == 0) return;  // an empty slot of the batch
+    lnt_colm_inv_body<S>(threadIdx.x, b / slots, LView{smem, LntColM<S>::LDS}, P);
 }
 
 template <int S>

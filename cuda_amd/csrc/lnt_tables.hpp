@@ -49,6 +49,12 @@ static __global__ void lnt_k_tw4_3(u64 om, u32 C, u32 BA, u32 BB, u32 BC, u32 n,
     tw[i] = gl_mul(lnt_tw4_3(om, C, BA, BB, BC, i), lnt_col_factor(B, s, p, n, C, i));
 }
 
+static __global__ void lnt_k_tw4_m(u64 om, u32 C, u32 S, u32 n, u64 B, u64 s, u32 p, u64 *tw) {
+    u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    tw[i] = gl_mul(lnt_tw4_m(om, C, S, i), lnt_col_factor(B, s, p, n, C, i));
+}
+
 template <class T>
 static GView<T> view(T *p, u64 n) {
     return GView<T>{p, n};
@@ -68,7 +74,7 @@ static TableSizes table_sizes(const Plan &pl) {
     const u32 m16 = pl.small ? pl.small16 : pl.rowm;
     t.L2 = m16 > 1 ? 16 * m16 : pl.row3m ? pl.rBB * pl.rBC : pl.row3 ? pl.row3 * pl.row3 : 0;
     t.R = pl.small ? 0 : pl.R;
-    t.A = (!pl.small && pl.col3) ? pl.R / pl.col3 : 0;
+    t.A = pl.small ? 0 : pl.colm ? 16 * pl.colm : pl.col3 ? pl.R / pl.col3 : 0;
     t.W = pl.small ? 2 * pl.n : 4 * pl.R;
     t.Wu = pl.small ? pl.n : 2 * pl.R;
     return t;
@@ -107,7 +113,18 @@ static void fill_tables(const Plan &pl, u32 p, const TablePtrs &t, hipStream_t s
     if (z.large) {
         u64 omc = gl_pow(554, (GL_P - 1) / pl.R);
         u64 omn = gl_pow(554, (GL_P - 1) / n);
-        if (pl.col3) {
+        if (pl.colm) {
+            // phase 1 (16 x 16 S line) and phase 2 (16 x S line) twiddles
+            const u32 A = z.A, S = pl.colm;
+            const u64 oma = gl_pow(554, (GL_P - 1) / A);
+            const dim3 gR((pl.R + 255) / 256), gA((A + 255) / 256), gn((n + 255) / 256), blk(256);
+            hipLaunchKernelGGL(lnt_k_line_tw, gR, blk, 0, s, omc, 16u, A, pl.R, t.twc);
+            hipLaunchKernelGGL(lnt_k_line_tw, gR, blk, 0, s, gl_inv(omc), 16u, A, pl.R, t.itwc);
+            hipLaunchKernelGGL(lnt_k_line_tw, gA, blk, 0, s, oma, 16u, S, A, t.twc2);
+            hipLaunchKernelGGL(lnt_k_line_tw, gA, blk, 0, s, gl_inv(oma), 16u, S, A, t.itwc2);
+            hipLaunchKernelGGL(lnt_k_tw4_m, gn, blk, 0, s, omn, pl.C, S, n, Bw, (u64)1, p, t.tw4);
+            hipLaunchKernelGGL(lnt_k_tw4_m, gn, blk, 0, s, gl_inv(omn), pl.C, S, n, Binv, ninv, p, t.itw4);
+        } else if (pl.col3) {
             // phase 1 (BA x A line) and phase 2 (BB x BC line) twiddles, 3-phase slot order
             const u32 A = z.A;
             hipLaunchKernelGGL(lnt_k_line_tw, dim3((pl.R + 255) / 256), dim3(256), 0, s, omc, pl.col3, A, pl.R, t.twc);

@@ -109,7 +109,21 @@ extern "C" void *emu_create3(uint32_t p, uint32_t n, int prp, uint32_t lc, uint3
     }
     e->twc2.assign(1, 1);
     e->itwc2.assign(1, 1);
-    if (!pl.small && pl.col3) {
+    if (!pl.small && pl.colm) {
+        Line l1, l2;
+        l1.B1 = l2.B1 = 16;
+        l1.B2 = 16 * pl.colm;
+        l2.B2 = pl.colm;
+        line_tables(pl.R, l1, e->twc, e->itwc);
+        line_tables(16 * pl.colm, l2, e->twc2, e->itwc2);
+        e->tw4.resize(n);
+        e->itw4.resize(n);
+        u64 om = gl_pow(554, (GL_P - 1) / n), iom = gl_inv(om);
+        for (uint64_t i = 0; i < n; i++) {
+            e->tw4[i] = gl_mul(lnt_tw4_m(om, pl.C, pl.colm, i), lnt_col_factor(Bw, 1, p, n, pl.C, i));
+            e->itw4[i] = gl_mul(lnt_tw4_m(iom, pl.C, pl.colm, i), lnt_col_factor(Binv, ninv, p, n, pl.C, i));
+        }
+    } else if (!pl.small && pl.col3) {
         Line l1, l2;
         l1.B1 = pl.col3;
         l1.B2 = pl.R / pl.col3;
@@ -246,6 +260,21 @@ static void col3_inv(Emu *e, const LntParams &P) {
                [&](int tid, LView L) { lnt_col3_inv_body<BA, BB, BC, K>(tid, b, L, P); });
 }
 
+template <int S>
+static void colm_fwd(Emu *e, bool sub2, const LntParams &P) {
+    for (uint32_t b = 0; b < e->pl.C / 16; b++)
+        run_wg(1024, LntColM<S>::LDS, [&](int tid, LView L) {
+            if (e->pl.M == 4) lnt_colm_fwd_body<S, 4>(tid, b, L, P, sub2);
+            else lnt_colm_fwd_body<S, 8>(tid, b, L, P, sub2);
+        });
+}
+
+template <int S>
+static void colm_inv(Emu *e, const LntParams &P) {
+    for (uint32_t b = 0; b < e->pl.C / 16; b++)
+        run_wg(1024, LntColM<S>::LDS, [&](int tid, LView L) { lnt_colm_inv_body<S>(tid, b, L, P); });
+}
+
 template <int B, int G>
 static void row3_sq(Emu *e, const LntParams &P, int mode) {
     const Plan &pl = e->pl;
@@ -265,6 +294,16 @@ static void row16_sq(Emu *e, const LntParams &P, int mode) {
             if (mode == LNT_FORWARD) lnt_row16_body<GW, LNT_FORWARD>(tid, b, L, P);
             else if (mode == LNT_MULTIPLY) lnt_row16_body<GW, LNT_MULTIPLY>(tid, b, L, P);
             else lnt_row16_body<GW>(tid, b, L, P);
+        });
+}
+
+template <int S>
+static void rowm_sq(Emu *e, const LntParams &P, int mode) {
+    for (uint32_t b = 0; b < e->pl.R; b++)
+        run_wg(64 * S, lnt_line16_lds<S>(), [&](int tid, LView L) {
+            if (mode == LNT_FORWARD) lnt_rowm_body<S, LNT_FORWARD>(tid, b, L, P);
+            else if (mode == LNT_MULTIPLY) lnt_rowm_body<S, LNT_MULTIPLY>(tid, b, L, P);
+            else lnt_rowm_body<S>(tid, b, L, P);
         });
 }
 
@@ -297,16 +336,6 @@ static bool run_small(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mod
     if (pl.small16 == 16) return small16_any<16>(e, k, P, sub2, mode), true;
     if (pl.small16 == 8) return small16_any<8>(e, k, P, sub2, mode), true;
     if (pl.small16 == 4) return small16_any<4>(e, k, P, sub2, mode), true;
-template <int S>
-static void rowm_sq(Emu *e, const LntParams &P, int mode) {
-    for (uint32_t b = 0; b < e->pl.R; b++)
-        run_wg(64 * S, lnt_line16_lds<S>(), [&](int tid, LView L) {
-            if (mode == LNT_FORWARD) lnt_rowm_body<S, LNT_FORWARD>(tid, b, L, P);
-            else if (mode == LNT_MULTIPLY) lnt_rowm_body<S, LNT_MULTIPLY>(tid, b, L, P);
-            else lnt_rowm_body<S>(tid, b, L, P);
-        });
-}
-
     if (pl.small16 == 2) return small16_any<2>(e, k, P, sub2, mode), true;
     if (pl.small16 == 1) return small16_any<1>(e, k, P, sub2, mode), true;
 #define SM(b1, b2)                                                                          \
@@ -336,6 +365,8 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
         if (pl.M == 4) col_fwd<b1, b2, k, 4>(e, sub2, P); else col_fwd<b1, b2, k, 8>(e, sub2, P); \
         ok = true;                                                               \
     }
+    if (pl.colm == 1) colm_fwd<1>(e, sub2, P), ok = true;
+    if (pl.colm == 4) colm_fwd<4>(e, sub2, P), ok = true;
     if (!pl.col3) {
         CF(4, 4, 16) CF(8, 4, 16) CF(8, 8, 16) CF(16, 8, 16) CF(16, 16, 16) CF(32, 16, 16) CF(32, 32, 16)
         CF(32, 32, 8) CF(64, 32, 8) CF(64, 32, 4) CF(64, 64, 4)
@@ -359,6 +390,10 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
     if (pl.row3m == 16 && pl.rBB == 32 && pl.rBC == 32) row3m_sq<16, 32, 32>(e, P, mode), ok = true;
     if (pl.row3 == 16) (e->wide_rows ? row16_sq<1>(e, P, mode) : row16_sq<4>(e, P, mode)), ok = true;
     if (pl.row3 == 8) row3_sq<8, 4>(e, P, mode), ok = true;
+    if (pl.rowm == 1) rowm_sq<1>(e, P, mode), ok = true;
+    if (pl.rowm == 2) rowm_sq<2>(e, P, mode), ok = true;
+    if (pl.rowm == 4) rowm_sq<4>(e, P, mode), ok = true;
+    if (pl.rowm == 8) rowm_sq<8>(e, P, mode), ok = true;
 #define RW(b1, b2)                                                        \
     if (!ok && !pl.row3m && pl.row.B1 == b1 && pl.row.B2 == b2) {                      \
         row_sq<b1, b2, 64 / b2>(e, P, mode);                              \
@@ -374,6 +409,8 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
         col_inv<b1, b2, k>(e, P);                                               \
         ok = true;                                                              \
     }
+    if (pl.colm == 1) colm_inv<1>(e, P), ok = true;
+    if (pl.colm == 4) colm_inv<4>(e, P), ok = true;
     if (!pl.col3) {
         CI(4, 4, 16) CI(8, 4, 16) CI(8, 8, 16) CI(16, 8, 16) CI(16, 16, 16) CI(32, 16, 16) CI(32, 32, 16)
         CI(32, 32, 8) CI(64, 32, 8) CI(64, 32, 4) CI(64, 64, 4)
@@ -391,10 +428,6 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
 #undef C3I
     return ok;
 }
-    if (pl.rowm == 1) rowm_sq<1>(e, P, mode), ok = true;
-    if (pl.rowm == 2) rowm_sq<2>(e, P, mode), ok = true;
-    if (pl.rowm == 4) rowm_sq<4>(e, P, mode), ok = true;
-    if (pl.rowm == 8) rowm_sq<8>(e, P, mode), ok = true;
 
 extern "C" int emu_iterate(void *h, uint32_t k) {
     Emu *e = (Emu *)h;

@@ -120,6 +120,41 @@ def test_emulated_3phase_columns_match_oracle(p, n, lc, K):
     assert e.digits() == o.digits()
 
 
+@pytest.mark.parametrize("p,n,lc,prp", [
+    (1000003, 65536, 8, False), (262147, 65536, 8, False),   # 256-row columns; 8 halo digits
+    (4000037, 262144, 8, True), (1048583, 262144, 8, True),  # 1024-row columns
+    (132049, 8192, 9, True), (250007, 16384, 10, False), (400009, 32768, 11, True),  # rows of 512, 1024, 2048
+])
+def test_emulated_matrix_core_columns_and_rows_match_oracle(p, n, lc, prp):
+    """Columns and rows of 256 S words on the matrix cores (256-word rows under 256- and
+    1024-row columns), with 4 and with 8 carry halo digits."""
+    rnd = random.Random(p + n)
+    o = OracleTest(p, n, prp)
+    d = [rnd.getrandbits(wi) for wi in o.widths()]
+    o.set_digits(d)
+    e = Emu(p, n, prp, lc)
+    e.set_digits(d)
+    o.iterate(2)
+    e.iterate(2)
+    assert e.digits() == o.digits()
+
+
+@pytest.mark.parametrize("p,n", [(2063, 512), (9689, 512), (4099, 1024), (19937, 1024), (8209, 2048), (44497, 2048),
+                                 (16411, 4096)])
+def test_emulated_one_workgroup_lines_match_oracle(p, n):
+    """n = 256 S in one workgroup with few (8 halo digits, field-encoded digits) and with
+    the usual bits per digit."""
+    rnd = random.Random(p)
+    o = OracleTest(p, n, False)
+    d = [rnd.getrandbits(wi) for wi in o.widths()]
+    o.set_digits(d)
+    e = Emu(p, n)
+    e.set_digits(d)
+    o.iterate(3)
+    e.iterate(3)
+    assert e.digits() == o.digits()
+
+
 def test_emulated_wide_4096_word_rows_match_oracle():
     """4096-word rows on the matrix cores by 16 waves of one DFT group each (the CASES run them
     by four waves): squarings, then a product through the forward and multiply modes."""
