@@ -599,7 +599,9 @@ uint32_t lnt_length(const lnt_ctx *c) { return c ? c->pl.n : 0; }
 
 static std::string describe(const Plan &pl) {
     char b[320];
-    if (pl.small && pl.small16) {
+    if (pl.small && pl.tiny) {
+        std::snprintf(b, sizeof b, "LNT_1WG;lnt_k_tiny<%u>", pl.n / 8);
+    } else if (pl.small && pl.small16) {
         std::snprintf(b, sizeof b, "LNT_1WG;lnt_k_small16<%u>", pl.small16);
     } else if (pl.small) {
         std::snprintf(b, sizeof b, "LNT_1WG;lnt_k_small<%u,%u>", pl.row.B1, pl.row.B2);

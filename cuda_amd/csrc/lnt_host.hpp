@@ -55,6 +55,7 @@ inline Line line_for(uint32_t a) {
 struct Plan {
     bool small = false;     // single-workgroup path (n <= 4096)
     uint32_t small16 = 0;   // its matrix-core kernel: n = 256 * small16 (0: the 2-phase kernel)
+    bool tiny = false;      // n = 64 or 128: the one-wave matrix-core kernel (tables of the 2-phase one)
     uint32_t n = 0, log_n = 0;
     uint32_t C = 0, R = 0;  // large path: row length, row count
     Line row, col;          // row line (also the small path's line), column line
@@ -75,7 +76,7 @@ struct Plan {
 // Two plans run the same kernel instantiations over the same table layouts (only the
 // exponent-dependent carry level count may differ).
 inline bool same_kernels(const Plan &a, const Plan &b) {
-    return a.small == b.small && a.small16 == b.small16 && a.n == b.n && a.C == b.C && a.R == b.R && a.row.B1 == b.row.B1 &&
+    return a.small == b.small && a.small16 == b.small16 && a.tiny == b.tiny && a.n == b.n && a.C == b.C && a.R == b.R && a.row.B1 == b.row.B1 &&
            a.row.B2 == b.row.B2 && a.col.B1 == b.col.B1 && a.col.B2 == b.col.B2 && a.K == b.K && a.G == b.G &&
            a.rowm == b.rowm && a.row3 == b.row3 && a.row3m == b.row3m && a.rBB == b.rBB && a.rBC == b.rBC &&
            a.colm == b.colm && a.col3 == b.col3 && a.cBB == b.cBB && a.cBC == b.cBC && a.M == b.M;
@@ -186,6 +187,7 @@ inline bool plan_consistent(const Plan &pl) {
     if (pl.levels < 1 || pl.levels > pl.M || (pl.M != 4 && pl.M != 8)) return false;
     if (pl.small) {
         const uint64_t line = pl.small16 ? 256ull * pl.small16 : (uint64_t)pl.row.B1 * pl.row.B2;
+        if (pl.tiny && (pl.small16 || (pl.n != 64 && pl.n != 128))) return false;
         return line == pl.n && pl.C == pl.n && pl.R == 1 && !pl.col3 && !pl.row3 && !pl.row3m;
     }
     if ((uint64_t)pl.R * pl.C != pl.n) return false;
@@ -226,8 +228,8 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
     if (pl.levels == 0) return "NTT length too small for this exponent (convolution would overflow)";
     pl.bias = digits_fit_31(p, (uint32_t)n, pl.levels);
     pl.M = pl.levels <= 4 ? 4 : 8;
-    // n <= 4096 runs in one workgroup: from n = 256 on the matrix cores (n = 256 * S with S
-    // waves), below, or when row3 = 0 asks for it, with the 2-phase kernel (at n = 2048 that
+    // n <= 4096 runs in one workgroup: from n = 64 on the matrix cores (from 256 as n = 256 * S
+    // with S waves), below, or when row3 = 0 asks for it, with the 2-phase kernel (at n = 2048 that
     // holds 64 words in each of 32 threads, 121 us per iteration, so row3 = 0 takes the
     // row/column path there).  A row length may also be asked for at n = 2048 and 4096.
     if (pl.log_n <= 10 || (pl.log_n <= 12 && !force_lc && !(pl.log_n == 11 && opts.row3 == 0))) {
@@ -236,6 +238,7 @@ inline std::string make_plan_fields(uint32_t p, uint64_t n, Plan &pl, PlanOpts o
         pl.C = pl.n;
         pl.R = 1;
         if (opts.row3 != 0 && pl.n >= 256) pl.small16 = pl.n / 256;
+        pl.tiny = opts.row3 != 0 && (pl.n == 64 || pl.n == 128);
         return "";
     }
     uint32_t lc, lr;

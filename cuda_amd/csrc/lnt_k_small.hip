@@ -28,7 +28,7 @@ bool lnt_launch_batch_small16(const lnt::Plan &pl, const LntParams *Ps, u32 coun
 bool lnt_launch_small(const lnt::Plan &pl, const LntParams &P, u32 iters, bool sub2_first, bool ll, hipStream_t s,
                       int mode) {
     if (!lnt::plan_consistent(pl)) return false;  // a kernel of another shape would run out of bounds
-    if (pl.small16) return lnt_launch_small16(pl, P, iters, sub2_first, ll, s, mode);
+    if (pl.small16 || pl.tiny) return lnt_launch_small16(pl, P, iters, sub2_first, ll, s, mode);
 #define SM(b1, b2) if (pl.row.B1 == b1 && pl.row.B2 == b2) return go_small<b1, b2>(pl, P, iters, sub2_first, ll, s, mode);
     SM(4, 2) SM(4, 4) SM(8, 4) SM(8, 8) SM(16, 8) SM(16, 16) SM(32, 16) SM(32, 32) SM(64, 32) SM(64, 64)
 #undef SM
@@ -47,7 +47,7 @@ static bool go_batch_small(const lnt::Plan &pl, const LntParams *Ps, u32 count, 
 
 bool lnt_launch_batch_small(const lnt::Plan &pl, const LntParams *Ps, u32 count, u32 iters, bool ll, hipStream_t s) {
     if (!lnt::plan_consistent(pl)) return false;  // a kernel of another shape would run out of bounds
-    if (pl.small16) return lnt_launch_batch_small16(pl, Ps, count, iters, ll, s);
+    if (pl.small16 || pl.tiny) return lnt_launch_batch_small16(pl, Ps, count, iters, ll, s);
 #define SM(b1, b2) if (pl.row.B1 == b1 && pl.row.B2 == b2) return go_batch_small<b1, b2>(pl, Ps, count, iters, ll, s);
     SM(4, 2) SM(4, 4) SM(8, 4) SM(8, 8) SM(16, 8) SM(16, 16) SM(32, 16) SM(32, 32) SM(64, 32) SM(64, 64)
 #undef SM

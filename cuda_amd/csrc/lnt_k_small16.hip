@@ -1,8 +1,8 @@
-// The single-workgroup kernels on the matrix cores, n = 256 .. 4096.
+// The single-workgroup kernels on the matrix cores, n = 64 .. 4096.
 //
 // One test on one compute unit is bound by the latency of its dependent steps.  Microseconds
 // per squaring against the register-DFT kernels before (8, 16 or 64 words per thread; n = 2048
-// as three launches): n = 256 2.6 / 17.1, 512 3.3 / 7.2, 1024 3.5 / 40.8, 2048 4.7 / 21.9,
+// as three launches): n = 64 1.3 / 7.7, 128 2.0 / 16.4, 256 2.6 / 17.1, 512 3.3 / 7.2, 1024 3.5 / 40.8, 2048 4.7 / 21.9,
 // 4096 9.4 / 24.6.  Built with the max-ilp machine scheduler (-amdgpu-sched-strategy=max-ilp,
 // set for this file in the Makefile): with at most four waves per SIMD nothing else hides the
 // wait states of the carry chains (n = 256 .. 2048 2.8, 3.6, 4.1, 4.8 us without, 4096 equal).
@@ -21,8 +21,36 @@ static void go_small16_m(const LntParams &P, u32 iters, bool sub2_first, bool ll
         hipLaunchKernelGGL((lnt_k_small16<S, M, LNT_SQUARE>), grid, block, 0, s, P, iters, (int)sub2_first, (int)ll);
 }
 
+template <int N1, int M>
+static void go_tiny_m(const LntParams &P, u32 iters, bool sub2_first, bool ll, hipStream_t s, int mode) {
+    if (mode == LNT_FORWARD)
+        hipLaunchKernelGGL((lnt_k_tiny<N1, M, LNT_FORWARD>), dim3(1), dim3(64), 0, s, P, 1u, (int)sub2_first, (int)ll);
+    else if (mode == LNT_MULTIPLY)
+        hipLaunchKernelGGL((lnt_k_tiny<N1, M, LNT_MULTIPLY>), dim3(1), dim3(64), 0, s, P, 1u, (int)sub2_first, (int)ll);
+    else
+        hipLaunchKernelGGL((lnt_k_tiny<N1, M, LNT_SQUARE>), dim3(1), dim3(64), 0, s, P, iters, (int)sub2_first,
+                           (int)ll);
+}
+
+template <int N1>
+static bool go_tiny(const lnt::Plan &pl, const LntParams &P, u32 iters, bool sub2_first, bool ll, hipStream_t s,
+                    int mode) {
+    if (pl.M == 4) go_tiny_m<N1, 4>(P, iters, sub2_first, ll, s, mode);
+    else go_tiny_m<N1, 8>(P, iters, sub2_first, ll, s, mode);
+    return true;
+}
+
+template <int N1>
+static bool go_batch_tiny(const lnt::Plan &pl, const LntParams *Ps, u32 count, u32 iters, bool ll, hipStream_t s) {
+    if (pl.M == 4) hipLaunchKernelGGL((lnt_kb_tiny<N1, 4>), dim3(count), dim3(64), 0, s, Ps, iters, (int)ll);
+    else hipLaunchKernelGGL((lnt_kb_tiny<N1, 8>), dim3(count), dim3(64), 0, s, Ps, iters, (int)ll);
+    return true;
+}
+
 bool lnt_launch_small16(const lnt::Plan &pl, const LntParams &P, u32 iters, bool sub2_first, bool ll, hipStream_t s,
                         int mode) {
+    if (pl.tiny && pl.n == 64) return go_tiny<8>(pl, P, iters, sub2_first, ll, s, mode);
+    if (pl.tiny && pl.n == 128) return go_tiny<16>(pl, P, iters, sub2_first, ll, s, mode);
     if (pl.n != 256 * pl.small16) return false;
 #define SM(S)                                                                 \
     if (pl.small16 == S) {                                                    \
@@ -36,6 +64,8 @@ bool lnt_launch_small16(const lnt::Plan &pl, const LntParams &P, u32 iters, bool
 }
 
 bool lnt_launch_batch_small16(const lnt::Plan &pl, const LntParams *Ps, u32 count, u32 iters, bool ll, hipStream_t s) {
+    if (pl.tiny && pl.n == 64) return go_batch_tiny<8>(pl, Ps, count, iters, ll, s);
+    if (pl.tiny && pl.n == 128) return go_batch_tiny<16>(pl, Ps, count, iters, ll, s);
     if (pl.n != 256 * pl.small16) return false;
 #define SM(S)                                                                                                     \
     if (pl.small16 == S) {                                                                                        \

@@ -167,7 +167,8 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     constexpr int RP = B1 / B2;
     constexpr int S = B2 + LNT_PAD;
     constexpr int KS = lnt_col_ks<B1, B2, K>();
-    constexpr int RT = (RR + T - 1) / T;  // carry rows per thread (the last may be idle)
+    constexpr int RT = (RR + T - 1) / T;  // carry rows per thread
+    constexpr int PR = RR < T ? T / RR : 1;  // carry: threads per row where rows are fewer than threads
     const u64 C = P.C;
     const u64 n = P.n;
     const u64 c0 = (u64)bid * K;
@@ -186,10 +187,11 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     if (HP) {
 #pragma unroll
         for (int q = 0; q < RT; q++) {
-            const u64 g0 = C * (u64)(tid + T * q) + c0;
+            const u64 g0 = C * (u64)(tid / PR + T * q) + c0;
 #pragma unroll
             for (int j = 0; j < M; j++)
-                h[HP ? q : 0][j] = (tid + T * q < RR) ? P.x[(g0 + n - M + j) & (n - 1)] : 0;
+                h[HP ? q : 0][j] =
+                    (tid / PR + T * q < RR && tid % PR == 0) ? P.x[(g0 + n - M + j) & (n - 1)] : 0;
         }
     }
     if (PF) {
@@ -200,9 +202,15 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     for (int j = 0; j < B1; j++) lds[(u32)((t + B2 * j) * KS + cl)] = a[j];
     LNT_SYNC();
 
-    // 1. carry + (-2): one thread per row run of K digits (plus the M halo digits)
+    // 1. carry + (-2): one thread per row run of K digits (plus the M halo digits), or PR
+    //    threads per run where there are more threads than rows (16 to 64 rows: the carry is
+    //    a quarter to a half of the chain that these short kernels are)
+    if constexpr (PR > 1) {
+        static_assert(HP && K == 16, "the halo words are prefetched");
+        lnt_carry_piece<M, K / PR, PR>(lds, (u32)(tid / PR * KS), tid % PR, h[0], P, C * (u64)(tid / PR) + c0, sub2);
+    }
 #pragma unroll
-    for (int q = 0; q < RT; q++) {
+    for (int q = 0; q < (PR > 1 ? 0 : RT); q++) {
         const int r = tid + T * q;
         if (r >= RR) break;
         int64_t v[M + K];
@@ -1288,6 +1296,114 @@ LNT_KFN void lnt_small_body(int tid, LView lds, const LntParams &P, u32 iters, b
     }
 #pragma unroll
     for (int j = 0; j < B1; j++) P.x[(u64)t + B2 * j] = lds[(u32)(t + B2 * j)];
+}
+
+// ------------------------------------------------------------------ n = 64 and 128 in one wave
+// n = N1 * 8 words (N1 = 8, 16) in one wave with N1-point DFTs over j (i = i1 + 8 j) and 8-point
+// DFTs over i1, both on the matrix cores.  Phase 1 has eight DFTs, so the lanes n >= 8 repeat
+// those of n - 8 and write nothing.  One wave needs no barrier, and all factors stay in registers.
+// Tables as for the 2-phase kernel (line N1 x 8).  LDS: n words in natural order, then the
+// transform, word (k2, i1) at 10 k2 + i1.  MODEs as above.
+template <int N1>
+constexpr u32 lnt_tiny_lds() { return 8 * N1 + 10 * N1; }
+
+template <int N1, int M, int MODE = LNT_SQUARE>
+LNT_KFN void lnt_tiny_body(int tid, LView lds, const LntParams &P, u32 iters, bool sub2_first, bool ll) {
+    constexpr u32 N = 8 * N1, Z = N;
+    constexpr int W1 = N1 / 4;  // phase-1 words per lane
+    constexpr int PK = N / 64;  // digits per thread in the carry
+    const int q = tid / 16, n = tid % 16, c = n & 7, k2 = N1 == 16 ? n : c;
+    const bool act = n < 8, act2 = N1 == 16 || act;
+    // phase-1 input j / output k2 at place e, and the inverse's output j at place v
+    auto word = [&](int e) { return N1 == 16 ? lnt_m16_word(q, e) : 2 * q + e; };
+    auto neg = [&](int e) { return (N1 - word(e)) & (N1 - 1); };
+    LntM16 Mx;
+    LntM8 M8;
+    lnt_m16_load(Mx, tid);
+    lnt_m8_load(M8, Mx, tid);
+    u64 wv[W1], wb[W1], tw[W1], uv[W1], itw[2];
+    const u64 r2 = gl_mul(GL_R, GL_R);
+#pragma unroll
+    for (int e = 0; e < W1; e++) {
+        const u32 i = (u32)(c + 8 * word(e));
+        wv[e] = P.w[2 * i];
+        wb[e] = P.w[2 * i + 1];
+        tw[e] = P.twr[8 * (N1 == 16 ? brev_v16(word(e)) : brev_v16(word(e)) >> 1) + c];
+        uv[e] = gl_mul(P.uw[c + 8 * neg(e)], r2);  // (the 2^128 as in lnt_small16_body)
+    }
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+        itw[v] = P.itwr[8 * (N1 == 16 ? brev_v16(k2) : brev_v16(k2) >> 1) + ((8 - 2 * q - v) & 7)];
+    auto dft1 = [&](u64 (&z)[4]) {
+        if (N1 == 16) lnt_m16_dft(Mx, z);
+        else {
+            u64 h[2] = {z[0], z[1]};
+            lnt_m8_dft(M8, Mx, h);
+            z[0] = h[0], z[1] = h[1];
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < PK; j++) lds[(u32)(tid + 64 * j)] = P.x[(u64)tid + 64 * j];
+    LNT_WAVE_SYNC();
+    for (u32 it = 0; it < iters; it++) {
+        {
+            const u32 g0 = PK * (u32)tid;
+            int64_t v[M + PK];
+#pragma unroll
+            for (int j = 0; j < M + PK; j++) v[j] = gl_to_i64(lds[(g0 + N - M + j) & (N - 1)]);
+            LNT_WAVE_SYNC();  // every word read before any is overwritten
+            lnt_carry_run<M, PK>(v, P.p, P.log_n, g0, P.levels, it == 0 ? sub2_first : ll);
+#pragma unroll
+            for (int j = 0; j < PK; j++)
+                lds[g0 + j] = P.bias ? (u64)(u32)(v[M + j] + (int64_t(1) << 31)) : gl_from_i64(v[M + j]);
+        }
+        LNT_WAVE_SYNC();
+        u64 z[4] = {}, g[2];
+#pragma unroll
+        for (int e = 0; e < W1; e++) {
+            const u64 d = lds[(u32)(c + 8 * word(e))];
+            z[e] = P.bias ? gl_mul_biased((u32)d, wv[e], wb[e]) : gl_mul(d, wv[e]);
+        }
+        dft1(z);
+#pragma unroll
+        for (int v = 0; v < W1; v++) {
+            const u64 t = gl_mmul(z[v], tw[v]);
+            if (act) lds[Z + (u32)(10 * word(v) + c)] = t;
+        }
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 2; v++) g[v] = lds[Z + (u32)(10 * k2 + 2 * q + v)];
+        lnt_m8_dft(M8, Mx, g);
+        const u64 slot = 2 * (u64)(q * N1 + k2);
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            if (MODE == LNT_FORWARD) {
+                if (act2) P.y[slot + v] = g[v];
+            } else {
+                g[v] = gl_mmul(g[v], MODE == LNT_MULTIPLY ? P.f[slot + v] : g[v]);
+            }
+        }
+        if (MODE == LNT_FORWARD) return;
+        lnt_m8_dft(M8, Mx, g);
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            const u64 t = gl_mmul(g[v], itw[v]);
+            if (act2) lds[Z + (u32)(10 * k2 + ((8 - 2 * q - v) & 7))] = t;
+        }
+        LNT_WAVE_SYNC();
+#pragma unroll
+        for (int e = 0; e < W1; e++) z[e] = lds[Z + (u32)(10 * word(e) + c)];
+        dft1(z);
+#pragma unroll
+        for (int v = 0; v < W1; v++) {
+            const u64 t = gl_mmul(z[v], uv[v]);
+            if (act) lds[(u32)(c + 8 * neg(v))] = t;
+        }
+        LNT_WAVE_SYNC();
+    }
+#pragma unroll
+    for (int j = 0; j < PK; j++) P.x[(u64)tid + 64 * j] = lds[(u32)(tid + 64 * j)];
 }
 
 // ------------------------------------------------------------------ small residues on the matrix cores

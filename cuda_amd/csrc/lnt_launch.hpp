@@ -23,6 +23,12 @@ __global__ __launch_bounds__(B2 < 64 ? 64 : B2) void lnt_k_small(LntParams P, u3
     lnt_small_body<B1, B2, M, MODE>(threadIdx.x, LView{smem, W}, P, iters, sub2_first != 0, ll != 0);
 }
 
+template <int N1, int M, int MODE>
+__global__ __launch_bounds__(64) void lnt_k_tiny(LntParams P, u32 iters, int sub2_first, int ll) {
+    __shared__ __align__(16) u64 smem[lnt_tiny_lds<N1>()];
+    lnt_tiny_body<N1, M, MODE>(threadIdx.x, LView{smem, lnt_tiny_lds<N1>()}, P, iters, sub2_first != 0, ll != 0);
+}
+
 template <int S, int M, int MODE>
 __global__ __launch_bounds__(64 * S) void lnt_k_small16(LntParams P, u32 iters, int sub2_first, int ll) {
     constexpr u32 W = lnt_small16_lds<S>();
@@ -125,6 +131,14 @@ __global__ __launch_bounds__(B2 < 64 ? 64 : B2) void lnt_kb_small(const LntParam
     const LntParams P = Ps[blockIdx.x];
     if (P.n == 0) return;  // an empty slot of the batch
     lnt_small_body<B1, B2, M>(threadIdx.x, LView{smem, W}, P, iters, P.sub2 != 0, ll != 0);
+}
+
+template <int N1, int M>
+__global__ __launch_bounds__(64) void lnt_kb_tiny(const LntParams *__restrict__ Ps, u32 iters, int ll) {
+    __shared__ __align__(16) u64 smem[lnt_tiny_lds<N1>()];
+    const LntParams P = Ps[blockIdx.x];
+    if (P.n == 0) return;  // an empty slot of the batch
+    lnt_tiny_body<N1, M>(threadIdx.x, LView{smem, lnt_tiny_lds<N1>()}, P, iters, P.sub2 != 0, ll != 0);
 }
 
 template <int S, int M>

@@ -216,6 +216,23 @@ static void small16_iter(Emu *e, uint32_t k, const LntParams &P, bool sub2) {
            [&](int tid, LView L) { lnt_small16_body<S, M, MODE>(tid, L, P, k, sub2, !e->prp); });
 }
 
+template <int N1, int M, int MODE = LNT_SQUARE>
+static void tiny_iter(Emu *e, uint32_t k, const LntParams &P, bool sub2) {
+    run_wg(64, lnt_tiny_lds<N1>(), [&](int tid, LView L) { lnt_tiny_body<N1, M, MODE>(tid, L, P, k, sub2, !e->prp); });
+}
+
+template <int N1>
+static void tiny_any(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mode) {
+    if (mode == LNT_FORWARD) {
+        if (e->pl.M == 4) tiny_iter<N1, 4, LNT_FORWARD>(e, 1, P, sub2);
+        else tiny_iter<N1, 8, LNT_FORWARD>(e, 1, P, sub2);
+    } else if (mode == LNT_MULTIPLY) {
+        if (e->pl.M == 4) tiny_iter<N1, 4, LNT_MULTIPLY>(e, 1, P, sub2);
+        else tiny_iter<N1, 8, LNT_MULTIPLY>(e, 1, P, sub2);
+    } else if (e->pl.M == 4) tiny_iter<N1, 4>(e, k, P, sub2);
+    else tiny_iter<N1, 8>(e, k, P, sub2);
+}
+
 template <int S>
 static void small16_any(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mode) {
     if (mode == LNT_FORWARD) {
@@ -333,6 +350,8 @@ static void row_sq(Emu *e, const LntParams &P, int mode) {
 // Dispatch tables for the emulated sizes (a subset of the HIP build's).
 static bool run_small(Emu *e, uint32_t k, const LntParams &P, bool sub2, int mode = LNT_SQUARE) {
     const Plan &pl = e->pl;
+    if (pl.tiny && pl.n == 64) return tiny_any<8>(e, k, P, sub2, mode), true;
+    if (pl.tiny && pl.n == 128) return tiny_any<16>(e, k, P, sub2, mode), true;
     if (pl.small16 == 16) return small16_any<16>(e, k, P, sub2, mode), true;
     if (pl.small16 == 8) return small16_any<8>(e, k, P, sub2, mode), true;
     if (pl.small16 == 4) return small16_any<4>(e, k, P, sub2, mode), true;

@@ -139,11 +139,11 @@ def test_emulated_matrix_core_columns_and_rows_match_oracle(p, n, lc, prp):
     assert e.digits() == o.digits()
 
 
-@pytest.mark.parametrize("p,n", [(2063, 512), (9689, 512), (4099, 1024), (19937, 1024), (8209, 2048), (44497, 2048),
+@pytest.mark.parametrize("p,n", [(131, 64), (1279, 64), (263, 128), (2203, 128), (2063, 512), (9689, 512), (4099, 1024), (19937, 1024), (8209, 2048), (44497, 2048),
                                  (16411, 4096)])
 def test_emulated_one_workgroup_lines_match_oracle(p, n):
-    """n = 256 S in one workgroup with few (8 halo digits, field-encoded digits) and with
-    the usual bits per digit."""
+    """n = 64, 128 and 256 S in one workgroup with few (8 halo digits, field-encoded digits) and
+    with the usual bits per digit."""
     rnd = random.Random(p)
     o = OracleTest(p, n, False)
     d = [rnd.getrandbits(wi) for wi in o.widths()]
