@@ -102,8 +102,8 @@ def cpu_baseline(p: int, n: int, seconds: float, gpu_check):
 
 def batched_leg(seed: int, iters: int, chunk: int = 1000, tune_loops: int = 0):
     """The batched uneven workload: 64 LL tests, exponents log-uniform in [1M, 20M] from
-    splitmix64(seed), 10,000 iterations each; all advance together (one hipGraph launch per
-    iteration) versus the same tests one at a time on the plain path.  Both timings include
+    splitmix64(seed), 10,000 iterations each; all advance together (one lnt_batch_iterate
+    call per chunk) versus the same tests one at a time on the plain path.  Both timings include
     each test's set-up (tables) and its final res64 readout; with tune_loops each length is
     tuned once beforehand (untimed) and both sides run the tuned plans."""
     from cuda_amd import Batch, LucasPRP, secured_log2_length

@@ -143,8 +143,9 @@ inline bool split_for(uint32_t log_n, uint32_t &lc, uint32_t &lr) {
     // words) with rows of up to 2048 words, then 64-row columns (us per squaring, against
     // the next best split: 2^13 12.7 / 13.9, 2^14 13.3 / 14.2, 2^15 15.1 / 15.4, 2^16 16.1 / 17.2,
     // 2^17 18.5 / 19.9), then 256-row columns (2^18 21.6 / 23.0, 2^19 25.1 / 28.2, 2^20 34.9 /
-    // 39.7).  From 2^20 rows of 4096 words; from 2^24 8192 words (0.550 against 0.581 ms with 4096 x 4096) and 16384 at
-    // 2^26 (mixed-radix 3-phase rows), over columns of at most 4096 words.
+    // 39.7; since the columns load ahead of their use 11.2, 11.9, 13.3, 15.4, 17.2, 21.0 and, at 2^20, 33.8).
+    // From 2^20 rows of 4096 words; from 2^24 8192 words (0.550 against 0.581 ms with 4096 x 4096)
+    // and 16384 at 2^26 (mixed-radix 3-phase rows), over columns of at most 4096 words.
     static const uint8_t lcs[] = {9, 10, 11, 10, 11, 10, 11};
     lc = log_n >= 24 ? (log_n == 26 ? 14 : 13) : log_n >= 20 ? 12 : lcs[log_n - 13];
     lr = log_n - lc;

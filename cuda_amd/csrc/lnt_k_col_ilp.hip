@@ -1,5 +1,6 @@
-// The inverse column kernel of the 2^22 plan (lnt_k_col3_inv<16, 8, 8, 16>: 1024-word
-// columns, 16 columns per workgroup), compiled with the max-ilp machine scheduler
+// The 3-phase inverse column kernel of 1024-word columns in tiles of 16
+// (lnt_k_col3_inv<16, 8, 8, 16>; a plan or the tuner asks for it, the default there is the
+// matrix-core kernel), compiled with the max-ilp machine scheduler
 // (-amdgpu-sched-strategy=max-ilp, set for this file in the Makefile).  The scheduler
 // interleaves the carry-chain pairs of independent words so that the wait states between
 // a carry-out and its carry-in are filled with work: 1.0 us faster for this shape at

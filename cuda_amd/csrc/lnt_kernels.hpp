@@ -11,7 +11,8 @@
 //   phase 1: thread t < B2 holds words t + B2*j (j < B1), a B1-point register DFT,
 //            then the inter-block twiddle omega_L^(t * k2);
 //   phase 2: after an LDS transpose, B2-point register DFTs over t.
-//   Output X[B1*k1 + k2].  All roots of order <= 64 are powers of two, so the only
+//   Output X[B1*k1 + k2].  Lines of 256, 512, 1024, 2048 and 4096 words take 16-point DFTs on the
+//   matrix cores instead (mdft.hpp; bodies below).  All roots of order <= 64 are powers of two, so the only
 //   general twiddle inside a line is the one between the phases.  3-phase lines
 //   (rows of 16^3 words, columns of BA * BB * BC words) add one more phase and twiddle.
 // Large residues (n >= 2^13) are a 2-D split: C-word rows (contiguous) and R-word
@@ -181,7 +182,10 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     // Tables are prefetched into registers when a thread's line fits (B1 <= 32).
     // The halo digits are prefetched too when there are few of them per thread.
     constexpr bool PF = B1 <= 32, HP = RT * M <= 16;
-    u64 a[B1], wv[PF ? B1 : 1], h[HP ? RT : 1][M];
+    // short lines (latency-bound passes; registers to spare) fetch the weights' second halves and
+    // the twiddles too, here and in the inverse: squaring 2^15 13.85 -> 13.3 us, 2^17 18.1 -> 17.2
+    constexpr bool PT = B1 <= 8;
+    u64 a[B1], wv[PF ? B1 : 1], wb[PT ? B1 : 1], tw[PT ? B1 : 1], h[HP ? RT : 1][M];
 #pragma unroll
     for (int j = 0; j < B1; j++) a[j] = P.x[c + C * (u64)(t + B2 * j)];
     if (HP) {
@@ -196,7 +200,12 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     }
     if (PF) {
 #pragma unroll
-        for (int j = 0; j < B1; j++) wv[PF ? j : 0] = P.w[2 * lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j))];
+        for (int j = 0; j < B1; j++) {
+            const u32 sl = lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j));
+            wv[PF ? j : 0] = P.w[2 * sl];
+            if (PT) wb[PT ? j : 0] = P.w[2 * sl + 1];
+            if (PT) tw[PT ? j : 0] = P.twc[(u64)j * B2 + t];
+        }
     }
 #pragma unroll
     for (int j = 0; j < B1; j++) lds[(u32)((t + B2 * j) * KS + cl)] = a[j];
@@ -233,7 +242,7 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
         for (int j = 0; j < B1; j++) {
             const u32 sl = lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j));
             a[j] = gl_mul_biased((u32)lds[(u32)((t + B2 * j) * KS + cl)], PF ? wv[PF ? j : 0] : P.w[2 * sl],
-                                 P.w[2 * sl + 1]);
+                                 PT ? wb[PT ? j : 0] : P.w[2 * sl + 1]);
         }
     } else {
 #pragma unroll
@@ -244,7 +253,8 @@ LNT_KFN void lnt_col_fwd_body(int tid, int bid, LView lds, const LntParams &P, b
     dft_fwd<B1>(a);
     if (B2 > 1) {
 #pragma unroll
-        for (int rho = 1; rho < B1; rho++) a[rho] = gl_mmul(a[rho], P.twc[(u64)rho * B2 + t]);
+        for (int rho = 1; rho < B1; rho++)
+            a[rho] = gl_mmul(a[rho], PT ? tw[PT ? rho : 0] : P.twc[(u64)rho * B2 + t]);
     }
     LNT_SYNC();
 #pragma unroll
@@ -275,13 +285,17 @@ LNT_KFN void lnt_col_inv_body(int tid, int bid, LView lds, const LntParams &P) {
     const u64 c = (u64)bid * K + cl;
     const u32 ec = lnt_wexp(P.p, P.n, c), mC = 0u - P.p * P.C;  // weight slot parameters
     constexpr bool PF = B1 <= 32;  // prefetch the unweighting factors (fits when B1 <= 32)
-    u64 a[B1], uv[PF ? B1 : 1];
+    constexpr bool PT = B1 <= 8;   // and the twiddles of short lines
+    u64 a[B1], uv[PF ? B1 : 1], tw[PT ? B1 : 1];
     // (the inverse 4-step twiddle was applied by the row pass as it stored the row)
 #pragma unroll
     for (int i = 0; i < B1; i++) a[i] = P.y[c + C * ((u64)t * B1 + i)];
     if (PF) {
 #pragma unroll
-        for (int j = 0; j < B1; j++) uv[PF ? j : 0] = P.uw[lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j))];
+        for (int j = 0; j < B1; j++) {
+            uv[PF ? j : 0] = P.uw[lnt_wslot(ec, mC, P.n, (u32)(t + B2 * j))];
+            if (PT) tw[PT ? j : 0] = P.itwc[(u64)j * B2 + t];
+        }
     }
 #pragma unroll
     for (int q = 0; q < RP; q++) {
@@ -294,7 +308,7 @@ LNT_KFN void lnt_col_inv_body(int tid, int bid, LView lds, const LntParams &P) {
 #pragma unroll
     for (int rho = 0; rho < B1; rho++) {
         u64 v = lds[(u32)((brev_c<B1>(rho) * S + t) * K + cl)];
-        a[rho] = (B2 > 1 && rho > 0) ? gl_mmul(v, P.itwc[(u64)rho * B2 + t]) : v;
+        a[rho] = (B2 > 1 && rho > 0) ? gl_mmul(v, PT ? tw[PT ? rho : 0] : P.itwc[(u64)rho * B2 + t]) : v;
     }
     dft_inv<B1>(a);
 #pragma unroll
@@ -543,20 +557,30 @@ LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
     LntM16 Mx;
     lnt_m16_load(Mx, tid);
     const u32 ec = lnt_wexp(P.p, P.n, c0 + n), mC = 0u - P.p * P.C;  // weight slot parameters
+    // phase 1 with the weights, those of a group fetched before the barrier or the DFT ahead of it
+    // (S = 1 at 2^18: 8.4 -> 7.7 us; S = 4: no change)
+    u64 wv[4], wb[4];
+    auto fetch_w = [&](int a1) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const u32 sl = lnt_wslot(ec, mC, P.n, (u32)(a1 + L * lnt_m16_word(q, e)));
+            wv[e] = P.w[2 * sl];
+            wb[e] = P.w[2 * sl + 1];
+        }
+    };
+    fetch_w(S * w);
     LNT_SYNC();
-    // phase 1 with the weights
 #pragma unroll 1
     for (int a1 = S * w; a1 < S * w + S; a1++) {
         u64 z[4], tw[4];
         const u32 at = (u32)(RS * a1 + n);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int j = lnt_m16_word(q, e);
-            const u32 sl = lnt_wslot(ec, mC, P.n, (u32)(a1 + L * j));
-            const u64 d = lds[at + (u32)(RS * L * j)];
-            z[e] = P.bias ? gl_mul_biased((u32)d, P.w[2 * sl], P.w[2 * sl + 1]) : gl_mul(d, P.w[2 * sl]);
-            tw[e] = P.twc[L * brev_v16(j) + a1];
+            const u64 d = lds[at + (u32)(RS * L * lnt_m16_word(q, e))];
+            z[e] = P.bias ? gl_mul_biased((u32)d, wv[e], wb[e]) : gl_mul(d, wv[e]);
+            tw[e] = P.twc[L * brev_v16(lnt_m16_word(q, e)) + a1];
         }
+        if (S > 1 && a1 + 1 < S * w + S) fetch_w(a1 + 1);
         lnt_m16_dft(Mx, z);
 #pragma unroll
         for (int v = 0; v < 4; v++) lds[at + (u32)(RS * L * lnt_m16_word(q, v))] = gl_mmul(z[v], tw[v]);
@@ -724,9 +748,9 @@ LNT_KFN void lnt_row_body(int tid, int bid, LView lds, const LntParams &P) {
 // reverse.  Within the LDS row of k2 a word (r, a) sits at r * (B + 1) + a, so every
 // phase reads and writes conflict-free strides.  Transform-domain slot for MODE 1/2:
 // base + k2 * B^2 + kb * B + i (thread-contiguous).
+// Reached for B = 8 (rows of 512 words) when a plan or the tuner asks for 3-phase rows.
 // LDS layout: word (k2, a) of a row at k2 * RS + a with runs of B words, unpadded by default:
-// the phase-3 runs are then 16-byte aligned and pair into 128-bit LDS accesses (at n = 2^22
-// the unpadded 4096-word row ran 53 against 55 us with one pad word per run).
+// the phase-3 runs are then 16-byte aligned and pair into 128-bit LDS accesses.
 template <int B, int G, int MODE = LNT_SQUARE, int PAD = 0>
 LNT_KFN void lnt_row3_body(int tid, int bid, LView lds, const LntParams &P) {
     constexpr int T = B * B;        // threads per row
@@ -997,6 +1021,7 @@ LNT_KFN void lnt_row16_body(int tid, int bid, LView lds, const LntParams &P) {
     const u64 base = (u64)4096 * (u64)bid;
     LntM16 M;
     u64 z[4], tw[4];
+    if (GW > 1) lnt_m16_load(M, tid);  // ahead of the loads of phase 1 (94.4 -> 92.6 us per squaring at 2^22)
     // phase 1
 #pragma unroll 1
     for (int h = GW * w; h < GW * w + GW; h++) {
@@ -1007,7 +1032,7 @@ LNT_KFN void lnt_row16_body(int tid, int bid, LView lds, const LntParams &P) {
             z[e] = gl_mmul(P.y[idx], P.tw4[idx]);  // 4-step twiddle of the column pass
             tw[e] = P.twr[256 * brev_v16(k) + 16 * h + n];
         }
-        if (h == GW * w) lnt_m16_load(M, tid);
+        if (GW == 1) lnt_m16_load(M, tid);
         lnt_m16_dft(M, z);
 #pragma unroll
         for (int v = 0; v < 4; v++)

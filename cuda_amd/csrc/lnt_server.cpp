@@ -1,6 +1,6 @@
 // Serving loop over the C ABI (include/lnt_api.h): a scheduler thread admits submitted
 // tests while their device footprint fits the budget, advances the admitted tests in
-// batches (lnt_batch_*: one hipGraph launch per iteration of all members), lets arrivals
+// batches (lnt_batch_*: every kernel shape's members advance together), lets arrivals
 // join and finished tests leave between scheduling steps (continuous batching), and
 // queues each result with its submit / admit / done times.  All GPU work is issued from
 // the scheduler thread; lnt_server_submit and lnt_server_poll only touch the queues.

@@ -200,6 +200,26 @@ def test_interrupt_and_resume_equals_uninterrupted(tmp_path):
 
 
 @pytest.mark.gpu
+def test_interrupt_and_resume_of_a_longer_run(tmp_path):
+    """The interrupt and resume above for a run of a few seconds (M216091, n = 2^14: 216,089
+    squarings), which a one-second delay reaches in the middle."""
+    (tmp_path / "LucasNTT.ini").write_text("PerformanceLoops = 10\n")
+    p = subprocess.Popen([CLI, "216091"], cwd=tmp_path, stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True)
+    out = ""
+    while "From iteration" not in out:
+        out += p.stdout.readline()
+    time.sleep(1.0)
+    p.send_signal(signal.SIGINT)
+    out += p.communicate(timeout=300)[0]
+    assert "Interrupted = 1" in (tmp_path / "LucasNTT_results.txt").read_text(), out
+    assert (tmp_path / "LucasNTT_results.dat").exists()
+    r = run([], tmp_path)
+    assert "Previous residue successfully loaded!" in r.stdout, r.stdout
+    assert "M(216091) is prime!" in r.stdout
+
+
+@pytest.mark.gpu
 def test_tuning_persists_in_the_tune_file(tmp_path):
     """A run that tunes writes LucasNTT.tune; a later run without tuning reads it and ends
     on the same residue."""
