@@ -1,7 +1,16 @@
 // Columns of 256 and 1024 words on the matrix cores (the 1024-word ones take about as long as the
 // 3-phase kernels: with one tile per compute unit the load, the carry, the transform and the
 // store follow each other there, and only the transform got shorter).
+//
+// Batches with more tiles than compute units (a quarter of their slots counted) run the 256-word tiles
+// with 4 waves of four groups each, four tiles on a unit that work past each other's loads and
+// barriers, where one test takes 16 waves a tile: per squaring of all, 16 tests of 2^20 402 -> 334 us,
+// 13 of 2^18 94 -> 79, one test of 2^20 in eight slots 81 -> 62; with fewer tiles the 16 waves stay
+// ahead (6 tests of 2^18 53 against 63).
 #include "lnt_launch.hpp"
+
+// Compute units of an MI355X.
+static constexpr u32 COLM_UNITS = 256;
 
 bool lnt_launch_colm_fwd(const lnt::Plan &pl, const LntParams &P, bool sub2, hipStream_t s) {
     if (pl.R != 256 * pl.colm || pl.K != 16) return false;
@@ -33,14 +42,16 @@ bool lnt_launch_colm_inv(const lnt::Plan &pl, const LntParams &P, hipStream_t s)
 bool lnt_launch_batch_colm_fwd(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s) {
     if (pl.R != 256 * pl.colm || pl.K != 16) return false;
     const u32 wgs = pl.C / 16;
-    const dim3 grid(wgs * count), block(1024);
-#define CM(S)                                                                                \
-    if (pl.colm == S) {                                                                      \
-        if (pl.M == 4) hipLaunchKernelGGL((lnt_kb_colm_fwd<S, 4>), grid, block, 0, s, Ps, wgs); \
-        else hipLaunchKernelGGL((lnt_kb_colm_fwd<S, 8>), grid, block, 0, s, Ps, wgs);        \
-        return true;                                                                         \
+    const dim3 grid(wgs * count);
+#define CM(S, W)                                                                                         \
+    {                                                                                                    \
+        if (pl.M == 4) hipLaunchKernelGGL((lnt_kb_colm_fwd<S, 4, W>), grid, dim3(64 * W), 0, s, Ps, wgs); \
+        else hipLaunchKernelGGL((lnt_kb_colm_fwd<S, 8, W>), grid, dim3(64 * W), 0, s, Ps, wgs);          \
+        return true;                                                                                     \
     }
-    CM(1) CM(4)
+    if (pl.colm == 4) CM(4, 16)
+    if (pl.colm == 1 && wgs * (count / 4) > COLM_UNITS) CM(1, 4)
+    if (pl.colm == 1) CM(1, 16)
 #undef CM
     return false;
 }
@@ -48,13 +59,15 @@ bool lnt_launch_batch_colm_fwd(const lnt::Plan &pl, const LntParams *Ps, u32 cou
 bool lnt_launch_batch_colm_inv(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s) {
     if (pl.R != 256 * pl.colm || pl.K != 16) return false;
     const u32 wgs = pl.C / 16;
-    const dim3 grid(wgs * count), block(1024);
-#define CM(S)                                                              \
-    if (pl.colm == S) {                                                    \
-        hipLaunchKernelGGL(lnt_kb_colm_inv<S>, grid, block, 0, s, Ps, wgs); \
-        return true;                                                       \
+    const dim3 grid(wgs * count);
+#define CM(S, W)                                                                           \
+    {                                                                                      \
+        hipLaunchKernelGGL((lnt_kb_colm_inv<S, W>), grid, dim3(64 * W), 0, s, Ps, wgs);    \
+        return true;                                                                       \
     }
-    CM(1) CM(4)
+    if (pl.colm == 4) CM(4, 16)
+    if (pl.colm == 1 && wgs * (count / 4) > COLM_UNITS) CM(1, 4)
+    if (pl.colm == 1) CM(1, 16)
 #undef CM
     return false;
 }

@@ -524,18 +524,20 @@ LNT_KFN void lnt_col3_inv_body(int tid, int bid, LView lds, const LntParams &P) 
 // and 2 and the hand-over of the carried digits wait for other waves.  LDS word (row r, column
 // n) at RS r + n; RS keeps the words of neighbouring lane groups (2 S rows apart in phase 2) on
 // the two halves of the banks.
-template <int S>
+// W = 16 waves take S groups each (four times as many with W = 4, S = 1).
+template <int S, int W = 16>
 struct LntColM {
     static constexpr int R = 256 * S, L = 16 * S;
-    static constexpr int RS = S == 1 ? 24 : 18;
+    static constexpr int RS = S == 1 && W == 16 ? 24 : 18;
     static constexpr u32 LDS = (u32)(R * RS);
 };
 
-template <int S, int M>
+template <int S, int M, int W = 16>
 LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, bool sub2) {
-    using Z = LntColM<S>;
-    constexpr int RS = Z::RS, L = Z::L;
-    constexpr int PR = 4 / S, PK = 4 * S;  // carry: threads per row, digits per thread
+    static_assert(S == 1 || W == 16, "phase 3 takes the words of one k2 from the wave's own places");
+    using Z = LntColM<S, W>;
+    constexpr int RS = Z::RS, L = Z::L, G = 16 * S / W;
+    constexpr int PR = W / (4 * S), PK = 16 / PR;  // carry: threads per row, digits per thread
     const LntLane16 T = lnt_lane16(tid);
     const int q = T.q, n = T.n, w = T.w;
     const u64 C = P.C, c0 = (u64)bid * 16;
@@ -544,12 +546,12 @@ LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
     {
         u64 a[PK], h[M];
 #pragma unroll
-        for (int i = 0; i < PK; i++) a[i] = P.x[c0 + n + C * (u64)(tid / 16 + 64 * i)];
+        for (int i = 0; i < PK; i++) a[i] = P.x[c0 + n + C * (u64)(tid / 16 + 4 * W * i)];
         const u64 g0 = C * (u64)(tid / PR) + c0;
 #pragma unroll
         for (int j = 0; j < M; j++) h[j] = tid % PR == 0 ? P.x[(g0 + P.n - M + j) & (P.n - 1)] : 0;
 #pragma unroll
-        for (int i = 0; i < PK; i++) lds[(u32)(RS * (tid / 16 + 64 * i) + n)] = a[i];
+        for (int i = 0; i < PK; i++) lds[(u32)(RS * (tid / 16 + 4 * W * i) + n)] = a[i];
         LNT_SYNC();
         // carry + (-2): PR neighbouring threads per row run of 16 digits
         lnt_carry_piece<M, PK, PR>(lds, (u32)(RS * (tid / PR)), tid % PR, h, P, g0, sub2);
@@ -568,10 +570,10 @@ LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
             wb[e] = P.w[2 * sl + 1];
         }
     };
-    fetch_w(S * w);
+    fetch_w(G * w);
     LNT_SYNC();
 #pragma unroll 1
-    for (int a1 = S * w; a1 < S * w + S; a1++) {
+    for (int a1 = G * w; a1 < G * w + G; a1++) {
         u64 z[4], tw[4];
         const u32 at = (u32)(RS * a1 + n);
 #pragma unroll
@@ -580,7 +582,7 @@ LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
             z[e] = P.bias ? gl_mul_biased((u32)d, wv[e], wb[e]) : gl_mul(d, wv[e]);
             tw[e] = P.twc[L * brev_v16(lnt_m16_word(q, e)) + a1];
         }
-        if (S > 1 && a1 + 1 < S * w + S) fetch_w(a1 + 1);
+        if (G > 1 && a1 + 1 < G * w + G) fetch_w(a1 + 1);
         lnt_m16_dft(Mx, z);
 #pragma unroll
         for (int v = 0; v < 4; v++) lds[at + (u32)(RS * L * lnt_m16_word(q, v))] = gl_mmul(z[v], tw[v]);
@@ -588,16 +590,17 @@ LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
     LNT_SYNC();
     // phase 2 (S = 1: the last); with S > 1 its words go through this lane's own LDS places to phase 3
 #pragma unroll 1
-    for (int g = 0; g < S; g++) {
+    for (int i = 0; i < G; i++) {
+        const int k2 = S == 1 ? G * w + i : w, g = S == 1 ? 0 : i;
         u64 z[4];
-        const u32 at = (u32)(RS * (L * w + g) + n);
+        const u32 at = (u32)(RS * (L * k2 + g) + n);
 #pragma unroll
         for (int e = 0; e < 4; e++) z[e] = lds[at + (u32)(RS * S * lnt_m16_word(q, e))];
         lnt_m16_dft(Mx, z);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int kb = lnt_m16_word(q, v);
-            if (S == 1) P.y[c0 + n + C * (u64)(16 * w + kb)] = z[v];
+            if (S == 1) P.y[c0 + n + C * (u64)(16 * k2 + kb)] = z[v];
             else lds[at + (u32)(RS * S * kb)] = gl_mmul(z[v], P.twc2[S * brev_v16(kb) + g]);
         }
     }
@@ -614,10 +617,11 @@ LNT_KFN void lnt_colm_fwd_body(int tid, int bid, LView lds, const LntParams &P, 
     }
 }
 
-template <int S>
+template <int S, int W = 16>
 LNT_KFN void lnt_colm_inv_body(int tid, int bid, LView lds, const LntParams &P) {
-    using Z = LntColM<S>;
-    constexpr int RS = Z::RS, L = Z::L;
+    static_assert(S == 1 || W == 16, "phase 3 leaves the words of one k2 in the wave's own places");
+    using Z = LntColM<S, W>;
+    constexpr int RS = Z::RS, L = Z::L, G = 16 * S / W;
     const LntLane16 T = lnt_lane16(tid);
     const int q = T.q, n = T.n, w = T.w;
     const u64 C = P.C, c = (u64)bid * 16 + n;
@@ -639,14 +643,15 @@ LNT_KFN void lnt_colm_inv_body(int tid, int bid, LView lds, const LntParams &P) 
     lnt_m16_load(Mx, tid);
     // phase 2 inverse: output place v is b = -lnt_m16_word(q, v)
 #pragma unroll 1
-    for (int g = 0; g < S; g++) {
+    for (int i = 0; i < G; i++) {
+        const int k2 = S == 1 ? G * w + i : w, g = S == 1 ? 0 : i;
         u64 z[4], tw[4];
-        const u32 at = (u32)(RS * (L * w + g) + n);
+        const u32 at = (u32)(RS * (L * k2 + g) + n);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int kb = lnt_m16_word(q, e);
-            z[e] = S == 1 ? P.y[c + C * (u64)(16 * w + kb)] : lds[at + (u32)(RS * S * kb)];
-            tw[e] = P.itwc[L * brev_v16(w) + g + S * lnt_m16_neg(q, e)];
+            z[e] = S == 1 ? P.y[c + C * (u64)(16 * k2 + kb)] : lds[at + (u32)(RS * S * kb)];
+            tw[e] = P.itwc[L * brev_v16(k2) + g + S * lnt_m16_neg(q, e)];
         }
         LNT_WAVE_SYNC();
         lnt_m16_dft(Mx, z);
@@ -657,7 +662,7 @@ LNT_KFN void lnt_colm_inv_body(int tid, int bid, LView lds, const LntParams &P) 
     LNT_SYNC();
     // phase 1 inverse, unweight, store
 #pragma unroll 1
-    for (int a1 = S * w; a1 < S * w + S; a1++) {
+    for (int a1 = G * w; a1 < G * w + G; a1++) {
         u64 y[4], uv[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -966,6 +971,43 @@ LNT_KFN void lnt_line16(u64 (&z)[4], const LntM16 &Mx, const LntM8 &M8, LView ld
 #pragma unroll
     for (int e = 0; e < 4; e++) z[e] = lds[(u32)(18 * S * lnt_m16_word(q, e)) + t1];
     lnt_m16_dft(Mx, z);
+}
+
+// ROWS rows per workgroup, one after the other, for launches that fill the chip: the DFT matrix is
+// loaded once, the factors are read where they are used, which keeps to the 128 registers of
+// four waves per SIMD, and consecutive rows take turns on two LDS regions, so that a row's first
+// exchange need not wait for the last reads of the row before.
+template <int S, int ROWS>
+LNT_KFN void lnt_rowm_rows_body(int tid, int bid, LView lds, const LntParams &P) {
+    LntM16 Mx;
+    LntM8 M8;
+    lnt_m16_load(Mx, tid);
+    if (S == 8) lnt_m8_load(M8, Mx, tid);
+#pragma unroll 1
+    for (int r = 0; r < ROWS; r++) {
+        LNT_OPAQUE_LANE(tid);
+        const LntLane16 L = lnt_lane16(tid);
+        const u64 base = (u64)(256 * S) * ((u64)bid * ROWS + r);
+        u64 z[4], t4[4];
+        LntTw16 T;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const u64 idx = base + L.id + 16 * S * lnt_m16_word(L.q, e);
+            z[e] = gl_mmul(P.y[idx], P.tw4[idx]);
+        }
+        line16_load_tw1<S>(T, L, P);
+        auto last = [&]() {
+            line16_load_itw1<S>(T, L, P);
+#pragma unroll
+            for (int v = 0; v < 4; v++) t4[v] = P.itw4[base + L.id + 16 * S * lnt_m16_neg(L.q, v)];
+        };
+        lnt_line16<S, LNT_SQUARE>(
+            z, Mx, M8, lds, (u32)((r & 1) * lnt_line16_lds<S>()), L, T, P, 0,
+            [&]() { S > 1 ? line16_load_tw2<S>(T, L, P) : last(); },
+            [&]() { line16_load_itw2<S>(T, L, P); }, last);
+#pragma unroll
+        for (int v = 0; v < 4; v++) P.y[base + L.id + 16 * S * lnt_m16_neg(L.q, v)] = gl_mmul(z[v], t4[v]);
+    }
 }
 
 // The row pass for rows of 256 S words (S <= 8), one row per workgroup of S waves: 4-step

@@ -222,22 +222,24 @@ __global__ __launch_bounds__(G * B * B) __attribute__((amdgpu_waves_per_eu(4))) 
 }
 
 // (members interleaved as in lnt_kb_col_fwd)
-template <int S, int M>
-__global__ __launch_bounds__(1024) void lnt_kb_colm_fwd(const LntParams *__restrict__ Ps, u32 wgs) {
-    __shared__ __align__(16) u64 smem[LntColM<S>::LDS];
+template <int S, int M, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void lnt_kb_colm_fwd(
+    const LntParams *__restrict__ Ps, u32 wgs) {
+    __shared__ __align__(16) u64 smem[LntColM<S, W>::LDS];
     const u32 b = lnt_xcd_bid(blockIdx.x, gridDim.x), slots = gridDim.x / wgs;
     const LntParams P = Ps[b % slots];
     if (P.n == 0) return;  // an empty slot of the batch
-    lnt_colm_fwd_body<S, M>(threadIdx.x, b / slots, LView{smem, LntColM<S>::LDS}, P, P.sub2 != 0);
+    lnt_colm_fwd_body<S, M, W>(threadIdx.x, b / slots, LView{smem, LntColM<S, W>::LDS}, P, P.sub2 != 0);
 }
 
-template <int S>
-__global__ __launch_bounds__(1024) void lnt_kb_colm_inv(const LntParams *__restrict__ Ps, u32 wgs) {
-    __shared__ __align__(16) u64 smem[LntColM<S>::LDS];
+template <int S, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void lnt_kb_colm_inv(
+    const LntParams *__restrict__ Ps, u32 wgs) {
+    __shared__ __align__(16) u64 smem[LntColM<S, W>::LDS];
     const u32 b = lnt_xcd_bid(blockIdx.x, gridDim.x), slots = gridDim.x / wgs;
     const LntParams P = Ps[b % slots];
     if (P.n == 0) return;  // an empty slot of the batch
-    lnt_colm_inv_body<S>(threadIdx.x, b / slots, LView{smem, LntColM<S>::LDS}, P);
+    lnt_colm_inv_body<S, W>(threadIdx.x, b / slots, LView{smem, LntColM<S, W>::LDS}, P);
 }
 
 template <int S>
@@ -246,6 +248,16 @@ __global__ __launch_bounds__(64 * S) void lnt_kb_rowm(const LntParams *__restric
     const LntParams P = Ps[blockIdx.x / wgs];
     if (P.n == 0) return;  // an empty slot of the batch
     lnt_rowm_body<S>(threadIdx.x, blockIdx.x % wgs, LView{smem, lnt_line16_lds<S>()}, P);
+}
+
+template <int S, int ROWS>
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4))) void lnt_kb_rowm_rows(
+    const LntParams *__restrict__ Ps, u32 wgs) {
+    constexpr u32 LDS = 2 * lnt_line16_lds<S>();
+    __shared__ __align__(16) u64 smem[LDS];
+    const LntParams P = Ps[blockIdx.x / wgs];
+    if (P.n == 0) return;  // an empty slot of the batch
+    lnt_rowm_rows_body<S, ROWS>(threadIdx.x, blockIdx.x % wgs, LView{smem, LDS}, P);
 }
 
 template <int GW>

@@ -22,6 +22,7 @@ struct Emu {
     uint32_t p;
     bool prp, pending;
     bool wide_rows = false;  // 4096-word rows with 16 waves instead of four
+    bool batch_forms = false;  // the forms that batches launch: 4-wave column tiles, four rows per workgroup
     std::vector<uint64_t> x, y, f, w, uw, tw4, itw4, twr, itwr, twr2, itwr2, twc, itwc, twc2, itwc2;
     std::vector<uint8_t> wid;
     LntParams P;
@@ -277,19 +278,19 @@ static void col3_inv(Emu *e, const LntParams &P) {
                [&](int tid, LView L) { lnt_col3_inv_body<BA, BB, BC, K>(tid, b, L, P); });
 }
 
-template <int S>
+template <int S, int W = 16>
 static void colm_fwd(Emu *e, bool sub2, const LntParams &P) {
     for (uint32_t b = 0; b < e->pl.C / 16; b++)
-        run_wg(1024, LntColM<S>::LDS, [&](int tid, LView L) {
-            if (e->pl.M == 4) lnt_colm_fwd_body<S, 4>(tid, b, L, P, sub2);
-            else lnt_colm_fwd_body<S, 8>(tid, b, L, P, sub2);
+        run_wg(64 * W, LntColM<S, W>::LDS, [&](int tid, LView L) {
+            if (e->pl.M == 4) lnt_colm_fwd_body<S, 4, W>(tid, b, L, P, sub2);
+            else lnt_colm_fwd_body<S, 8, W>(tid, b, L, P, sub2);
         });
 }
 
-template <int S>
+template <int S, int W = 16>
 static void colm_inv(Emu *e, const LntParams &P) {
     for (uint32_t b = 0; b < e->pl.C / 16; b++)
-        run_wg(1024, LntColM<S>::LDS, [&](int tid, LView L) { lnt_colm_inv_body<S>(tid, b, L, P); });
+        run_wg(64 * W, LntColM<S, W>::LDS, [&](int tid, LView L) { lnt_colm_inv_body<S, W>(tid, b, L, P); });
 }
 
 template <int B, int G>
@@ -312,6 +313,12 @@ static void row16_sq(Emu *e, const LntParams &P, int mode) {
             else if (mode == LNT_MULTIPLY) lnt_row16_body<GW, LNT_MULTIPLY>(tid, b, L, P);
             else lnt_row16_body<GW>(tid, b, L, P);
         });
+}
+
+template <int S>
+static void rowm_rows(Emu *e, const LntParams &P) {
+    for (uint32_t b = 0; b < e->pl.R / 4; b++)
+        run_wg(64 * S, 2 * lnt_line16_lds<S>(), [&](int tid, LView L) { lnt_rowm_rows_body<S, 4>(tid, b, L, P); });
 }
 
 template <int S>
@@ -384,7 +391,7 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
         if (pl.M == 4) col_fwd<b1, b2, k, 4>(e, sub2, P); else col_fwd<b1, b2, k, 8>(e, sub2, P); \
         ok = true;                                                               \
     }
-    if (pl.colm == 1) colm_fwd<1>(e, sub2, P), ok = true;
+    if (pl.colm == 1) (e->batch_forms ? colm_fwd<1, 4>(e, sub2, P) : colm_fwd<1>(e, sub2, P)), ok = true;
     if (pl.colm == 4) colm_fwd<4>(e, sub2, P), ok = true;
     if (!pl.col3) {
         CF(4, 4, 16) CF(8, 4, 16) CF(8, 8, 16) CF(16, 8, 16) CF(16, 16, 16) CF(32, 16, 16) CF(32, 32, 16)
@@ -412,7 +419,7 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
     if (pl.rowm == 1) rowm_sq<1>(e, P, mode), ok = true;
     if (pl.rowm == 2) rowm_sq<2>(e, P, mode), ok = true;
     if (pl.rowm == 4) rowm_sq<4>(e, P, mode), ok = true;
-    if (pl.rowm == 8) rowm_sq<8>(e, P, mode), ok = true;
+    if (pl.rowm == 8) (e->batch_forms && mode == LNT_SQUARE ? rowm_rows<8>(e, P) : rowm_sq<8>(e, P, mode)), ok = true;
 #define RW(b1, b2)                                                        \
     if (!ok && !pl.row3m && pl.row.B1 == b1 && pl.row.B2 == b2) {                      \
         row_sq<b1, b2, 64 / b2>(e, P, mode);                              \
@@ -428,7 +435,7 @@ static bool run_large_once(Emu *e, bool sub2, const LntParams &P, int mode = LNT
         col_inv<b1, b2, k>(e, P);                                               \
         ok = true;                                                              \
     }
-    if (pl.colm == 1) colm_inv<1>(e, P), ok = true;
+    if (pl.colm == 1) (e->batch_forms ? colm_inv<1, 4>(e, P) : colm_inv<1>(e, P)), ok = true;
     if (pl.colm == 4) colm_inv<4>(e, P), ok = true;
     if (!pl.col3) {
         CI(4, 4, 16) CI(8, 4, 16) CI(8, 8, 16) CI(16, 8, 16) CI(16, 16, 16) CI(32, 16, 16) CI(32, 32, 16)
@@ -482,6 +489,7 @@ extern "C" void emu_set_digits(void *h, const uint64_t *d) {
     e->pending = false;
 }
 
+extern "C" void emu_batch_forms(void *h, int on) { ((Emu *)h)->batch_forms = on != 0; }
 extern "C" void emu_wide_rows(void *h, int on) { ((Emu *)h)->wide_rows = on != 0; }
 extern "C" uint32_t emu_levels(void *h) { return ((Emu *)h)->pl.levels; }
 extern "C" uint32_t emu_secured(uint32_t p) { return secured_log2_length(p); }

@@ -179,6 +179,24 @@ def test_emulated_wide_4096_word_rows_match_oracle():
     assert e.digits() == o.digits()
 
 
+@pytest.mark.parametrize("p,n,lc", [(400009, 32768, 7), (131101, 32768, 7),  # 256-row columns; 8 halo digits
+                                    (400009, 32768, 11), (1000003, 131072, 11)])  # rows of 2048: 16 and 64
+def test_emulated_batch_forms_match_oracle(p, n, lc):
+    """The kernel forms that only batches launch: 256-word columns with four waves per tile and
+    2048-word rows four to a workgroup (two LDS regions in turn)."""
+    rnd = random.Random(p + n + lc)
+    L = emu()
+    L.emu_batch_forms.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    o, e = OracleTest(p, n, False), Emu(p, n, False, lc)
+    L.emu_batch_forms(e.h, 1)
+    d = [rnd.getrandbits(wi) for wi in o.widths()]
+    o.set_digits(d)
+    e.set_digits(d)
+    o.iterate(2)
+    e.iterate(2)
+    assert e.digits() == o.digits()
+
+
 @pytest.mark.parametrize("p,n", [(9689, 512), (86243, 4096)])
 def test_emulated_orbit_matches_gmp(p, n):
     g = golden(p, "LL")

@@ -233,3 +233,25 @@ def test_membership_changes_reuse_the_graph():
     for t, s, what in ((a, sa, "left"), (b, sb, "stayed"), (d, sd, "joined"), (c, sc, "new shape")):
         assert t.get_digits() == s.get_digits(), what
     batch.close()
+
+
+@pytest.mark.parametrize("ps", [[8000009 + 2 * i for i in range(6)],  # 2^19: 2048-word rows four to a workgroup
+                                [1048583, 4000037, 4000039],          # 2^18: 256-word columns, 8 and 4 halo digits
+                                [16000057]])                          # 2^20
+def test_batch_kernel_forms_match_solo(ps):
+    """The kernel forms that only batches launch leave the residues of the plain path's."""
+    say("batch forms", ps)
+    n = max(1 << cuda_amd.secured_log2_length(p) for p in ps)
+    batch = cuda_amd.Batch()
+    members, solo = ([cuda_amd.LucasPRP(p, n) for p in ps] for _ in range(2))
+    for t in members:
+        batch.add(t)
+    for k in (3, 40):
+        batch.iterate(k)
+        batch.sync()
+        for t, s in zip(members, solo):
+            s.iterate(k)
+            assert t.get_digits() == s.get_digits(), (t.p, k)
+    batch.close()
+    for t in members + solo:
+        t.close()
