@@ -186,17 +186,40 @@ def test_interrupt_and_resume_equals_uninterrupted(tmp_path):
     out = ""
     while "From iteration" not in out:
         out += p.stdout.readline()
-    time.sleep(1.0)
+    time.sleep(0.1)  # the whole run takes about 0.8 s
     p.send_signal(signal.SIGINT)
     out += p.communicate(timeout=300)[0]
-    stats = (tmp_path / "LucasNTT_results.txt").read_text()
-    if "Interrupted = 1" not in stats:
-        pytest.skip("the run finished before the interrupt arrived")
+    assert "Interrupted = 1" in (tmp_path / "LucasNTT_results.txt").read_text(), out
     assert (tmp_path / "LucasNTT_results.dat").exists()
     r = run([], tmp_path)
     assert "Previous residue successfully loaded!" in r.stdout, r.stdout
     assert "M(86243) is prime!" in r.stdout
     assert not (tmp_path / "LucasNTT_results.dat").exists()  # LoadResidue removes the dump
+
+
+@pytest.mark.gpu
+def test_interrupt_between_dumps_of_a_one_workgroup_run(tmp_path):
+    """The same where each dump waits for the squarings before it, so that the interrupt ends
+    the run in its middle: the dumped residue is the oracle's at that iteration."""
+    (tmp_path / "LucasNTT.ini").write_text("PerformanceLoops = 0\nDumpIterations = 1000\n")
+    p = subprocess.Popen([CLI, "86243"], cwd=tmp_path, stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True)
+    out = ""
+    while "From iteration" not in out:
+        out += p.stdout.readline()
+    time.sleep(0.1)
+    p.send_signal(signal.SIGINT)
+    out += p.communicate(timeout=300)[0]
+    stats = dict(l.split(" = ", 1) for l in (tmp_path / "LucasNTT_results.txt").read_text().splitlines()
+                 if " = " in l)
+    done = int(stats["currentIteration"]) - 1
+    assert stats["Interrupted"] == "1" and 0 < done < 86241, (stats, out)
+    o = OracleTest(86243, 4096)
+    o.iterate(done)
+    assert [int(l, 16) for l in (tmp_path / "LucasNTT_results.dat").read_text().splitlines()] == o.digits()
+    r = run([], tmp_path)
+    assert "Previous residue successfully loaded!" in r.stdout, r.stdout
+    assert "M(86243) is prime!" in r.stdout
 
 
 @pytest.mark.gpu
