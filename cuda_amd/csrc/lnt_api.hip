@@ -1055,6 +1055,7 @@ struct lnt_batch {
         hipEvent_t join = nullptr;
         hipGraph_t graph = nullptr;  // GRAPH_ITERS iterations (not for single-workgroup tests)
         hipGraphExec_t exec = nullptr;
+        uint32_t ran = 0;  // iterations of the present step launched so far
     };
     std::vector<Group> groups;
     hipEvent_t fork = nullptr;
@@ -1215,6 +1216,7 @@ static int batch_group_run(lnt_batch *b, lnt_batch::Group &g, uint32_t step) {
         }
         BHIPCHK(b, hipGetLastError(), "kernel launch");
         step -= done;
+        g.ran += done;
         if (first && (rc = batch_mark_pending(b, g))) return rc;
     }
     return LNT_OK;
@@ -1302,35 +1304,42 @@ int lnt_batch_iterate(lnt_batch *b, uint32_t k) {
     b->upload = false;
     // Members under a Gerbicz check count the squarings as checked iterations: the groups
     // stop at each of their block ends for the block step on the member's stream.
-    uint32_t left = k;
-    while (left) {
+    rc = LNT_OK;
+    for (uint32_t left = k; left && rc == LNT_OK;) {
         uint32_t step = left;
         for (lnt_ctx *c : b->members)
             if (c->g.on) step = (uint32_t)std::min<uint64_t>(step, c->g.B - c->g.it % c->g.B);
-        BHIPCHK(b, hipEventRecord(b->fork, b->stream), "hipEventRecord");
-        rc = LNT_OK;
+        for (auto &g : b->groups) g.ran = 0;
+        // the first error ends the call, after what was launched by then is accounted for: the
+        // batch stream waits for it, later work on a member's own stream starts after it, and
+        // checked members count their squarings
+        auto hip = [&](hipError_t e, const char *what) {
+            if (e != hipSuccess && rc == LNT_OK)
+                rc = bfail(b, LNT_DEVICE_ERROR, std::string(what) + " (" + hipGetErrorString(e) + ")");
+        };
+        hip(hipEventRecord(b->fork, b->stream), "hipEventRecord");
         for (auto &g : b->groups) {
-            BHIPCHK(b, hipStreamWaitEvent(g.side, b->fork, 0), "hipStreamWaitEvent");
+            hip(hipStreamWaitEvent(g.side, b->fork, 0), "hipStreamWaitEvent");
             if (rc == LNT_OK) rc = batch_group_run(b, g, step);
-            // joined on an error too: whatever was launched is waited for by the batch stream
-            BHIPCHK(b, hipEventRecord(g.join, g.side), "hipEventRecord");
-            BHIPCHK(b, hipStreamWaitEvent(b->stream, g.join, 0), "hipStreamWaitEvent");
+            hip(hipEventRecord(g.join, g.side), "hipEventRecord");
+            hip(hipStreamWaitEvent(b->stream, g.join, 0), "hipStreamWaitEvent");
         }
-        if (rc != LNT_OK) return rc;
         left -= step;
-        // later work on a member's own stream starts after the batch's
-        BHIPCHK(b, hipEventRecord(b->done, b->stream), "hipEventRecord");
-        for (lnt_ctx *c : b->members) BHIPCHK(b, hipStreamWaitEvent(c->stream, b->done, 0), "hipStreamWaitEvent");
-        for (lnt_ctx *c : b->members) {
-            if (!c->g.on) continue;
-            c->g.it += step;
-            if (c->g.it % c->g.B) continue;
-            if ((rc = gz_block_end(c))) return bfail(b, rc, std::string("member p=") + std::to_string(c->p) + ": " + c->err);
-            BHIPCHK(b, hipEventRecord(c->ev_gz, c->stream), "hipEventRecord");
-            BHIPCHK(b, hipStreamWaitEvent(b->stream, c->ev_gz, 0), "hipStreamWaitEvent");
-        }
+        hip(hipEventRecord(b->done, b->stream), "hipEventRecord");
+        for (lnt_ctx *c : b->members) hip(hipStreamWaitEvent(c->stream, b->done, 0), "hipStreamWaitEvent");
+        for (auto &g : b->groups)
+            for (lnt_ctx *c : g.ctxs) {
+                if (!c || !c->g.on || !g.ran) continue;
+                c->g.it += g.ran;
+                if (c->g.it % c->g.B) continue;
+                const int rg = gz_block_end(c);
+                if (rg != LNT_OK && rc == LNT_OK)
+                    rc = bfail(b, rg, std::string("member p=") + std::to_string(c->p) + ": " + c->err);
+                hip(hipEventRecord(c->ev_gz, c->stream), "hipEventRecord");
+                hip(hipStreamWaitEvent(b->stream, c->ev_gz, 0), "hipStreamWaitEvent");
+            }
     }
-    return LNT_OK;
+    return rc;
 }
 
 int lnt_batch_sync(lnt_batch *b, float *elapsed_ms) {

@@ -1,0 +1,93 @@
+"""Which HIP calls the engine makes, and in which order (no GPU needed): liblnt.so runs on a HIP
+runtime without a device (tests/emu/fake_hip.cpp) that writes the calls to a log."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+from helpers import HERE, ROOT
+
+FAKE_SRC = os.path.join(HERE, "emu", "fake_hip.cpp")
+FAKE_SO = os.path.join(HERE, "emu", "_build", "libfakehip.so")
+
+PRELUDE = """
+import ctypes, json, sys
+fake = ctypes.CDLL(%r, ctypes.RTLD_GLOBAL)  # ahead of the HIP runtime that liblnt.so names
+fake.fake_log.restype = ctypes.c_char_p
+sys.path.insert(0, %r)
+import cuda_amd
+
+def log():
+    return [l.split() for l in fake.fake_log().decode().splitlines()]
+
+def stream_of(t):  # the context was the last to make calls
+    return log()[-1][1]
+"""
+
+
+@pytest.fixture(scope="module")
+def fake():
+    """Runs a script on the fake runtime; its last line of output is JSON."""
+    if not os.path.exists(FAKE_SO) or os.path.getmtime(FAKE_SRC) > os.path.getmtime(FAKE_SO):
+        os.makedirs(os.path.dirname(FAKE_SO), exist_ok=True)
+        tmp = f"{FAKE_SO}.{os.getpid()}.tmp"
+        subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", "-o", tmp, FAKE_SRC], check=True)
+        os.replace(tmp, FAKE_SO)
+
+    def run(script, **env):
+        r = subprocess.run([sys.executable, "-c", PRELUDE % (FAKE_SO, ROOT) + script], capture_output=True,
+                           text=True, timeout=300, env={**os.environ, **env})
+        assert r.returncode == 0, r.stdout + r.stderr
+        return json.loads(r.stdout.splitlines()[-1])
+    return run
+
+
+def ordered_before(log):
+    """Per stream, the launches that work enqueued on it now comes after: those of the stream
+    itself, of the streams that it waits for, and what the host waited for."""
+    seen, events, host, launches = {}, {}, set(), []
+    for i, (op, stream, *arg) in enumerate(log):
+        s = seen.setdefault(stream, set())
+        s |= host
+        if op in ("launch", "graph"):
+            s.add(i)
+            launches.append((i, stream))
+        elif op == "record":
+            events[arg[0]] = set(s)
+        elif op == "wait":
+            s |= events.get(arg[0], set())
+        elif op == "sync":
+            host |= s
+    return seen, launches
+
+
+@pytest.mark.parametrize("block", [1000, 40])
+def test_failed_batch_step_is_joined_and_counted(fake, block):
+    """A batch step whose second group fails: the members' streams wait for what the first group
+    launched, and a checked member of it counts those squarings, the end of a block included."""
+    got = fake("""
+block = %d
+a = cuda_amd.LucasPRP(1000003, prp=True); sa = stream_of(a)
+b = cuda_amd.LucasPRP(2000003, prp=True); sb = stream_of(b)
+a.gerbicz_begin(block, 1)
+batch = cuda_amd.Batch()
+batch.add(a); batch.add(b)
+batch.iterate(40)
+fake.fake_clear()
+fake.fake_fail(b"graph", 3)  # the first of the second group
+try:
+    batch.iterate(40)
+    failed = False
+except cuda_amd.LntError:
+    failed = True
+print(json.dumps(dict(log=log(), sa=sa, sb=sb, failed=failed, st=a.gerbicz_stats())))
+""" % block)
+    assert got["failed"]
+    seen, launches = ordered_before(got["log"])
+    of_groups = {i for i, s in launches if s not in (got["sa"], got["sb"])}
+    assert len(of_groups) >= 10
+    assert of_groups <= seen[got["sa"]] and of_groups <= seen[got["sb"]]
+    assert got["st"]["iteration"] == 80 and got["st"]["checks"] == (2 if block == 40 else 0)
