@@ -1034,7 +1034,8 @@ int lnt_gerbicz_stats(lnt_ctx *c, uint64_t *out, int cap) {
 // stream of its own, single-workgroup groups as one launch that loops over them, the others
 // as replays of a captured graph of GRAPH_ITERS iterations and the remainder one by one.
 // (Stepping all groups together, one graph launch per iteration with the groups as its
-// branches, spent 97 us per iteration on 24 tests of 2^11 .. 2^14 words.)
+// branches, spent 97 us per iteration on 24 tests of 2^11 .. 2^14 words; only short steps are
+// run so, see batch_short.)
 
 struct lnt_batch {
     int device = 0;
@@ -1060,9 +1061,12 @@ struct lnt_batch {
     std::vector<Group> groups;
     hipEvent_t fork = nullptr;
     hipEvent_t done = nullptr;  // end of the last batch_iterate: members' streams wait on it
-    bool dirty = true;      // the groups or their capacities changed: capture new graphs
+    hipGraph_t graph = nullptr;  // one iteration of every group (for short steps)
+    hipGraphExec_t exec = nullptr;
+    bool again = false;     // these groups have made a short step
+    bool dirty = true;      // the groups or their capacities changed: new groups and graphs
     bool upload = false;    // parameters changed: copy them to the device before the next step
-    uint64_t captures = 0;  // times the groups' graphs were captured
+    uint64_t captures = 0;  // times the groups were formed, whose steps capture their graphs
     std::string err;
 };
 
@@ -1084,6 +1088,12 @@ static int bfail(lnt_batch *b, int code, const std::string &m) {
 static bool same_group(const Plan &a, const Plan &b) { return same_kernels(a, b); }
 
 static void batch_release(lnt_batch *b) {
+    if (b->stream) (void)hipStreamSynchronize(b->stream);
+    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->exec = nullptr;
+    b->graph = nullptr;
+    b->again = false;
     for (auto &g : b->groups) {
         if (g.side) (void)hipStreamSynchronize(g.side);
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -1095,9 +1105,9 @@ static void batch_release(lnt_batch *b) {
     b->groups.clear();
 }
 
-// Launch one iteration of the row/column group g on its stream (all cap slots; empty ones
-// return at once).
+// Launch one iteration of group g on its stream (all cap slots; empty ones return at once).
 static bool batch_group_step(lnt_batch::Group &g) {
+    if (g.pl.small) return lnt_launch_batch_small(g.pl, g.d, g.cap, 1, g.ll, g.side);
     return lnt_launch_batch_col_fwd(g.pl, g.d, g.cap, g.side) && lnt_launch_batch_row(g.pl, g.d, g.cap, g.side) &&
            lnt_launch_batch_col_inv(g.pl, g.d, g.cap, g.side);
 }
@@ -1116,7 +1126,8 @@ static lnt_batch::Group *group_of(lnt_batch *b, const lnt_ctx *c) {
 }
 
 // Groups for the current members, each with room to grow (at least 8 slots, a power of
-// two, at least twice its members), their parameters, streams and captured graphs.
+// two, at least twice its members), their parameters and streams.  The first step that
+// replays a graph captures it.
 static int batch_build(lnt_batch *b) {
     batch_release(b);
     for (lnt_ctx *c : b->members) {
@@ -1140,13 +1151,6 @@ static int batch_build(lnt_batch *b) {
         BHIPCHK(b, hipMalloc(&g.d, g.h.size() * sizeof(LntParams)), "hipMalloc (batch parameters)");
         BHIPCHK(b, hipStreamCreateWithFlags(&g.side, hipStreamNonBlocking), "hipStreamCreate");
         BHIPCHK(b, hipEventCreateWithFlags(&g.join, hipEventDisableTiming), "hipEventCreate");
-        if (g.pl.small) continue;
-        BHIPCHK(b, hipStreamBeginCapture(g.side, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-        bool ok = true;
-        for (uint32_t i = 0; i < GRAPH_ITERS && ok; i++) ok = batch_group_step(g);
-        hipError_t ec = hipStreamEndCapture(g.side, &g.graph);
-        if (!ok || ec != hipSuccess) return bfail(b, LNT_DEVICE_ERROR, "batch graph capture failed");
-        BHIPCHK(b, hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
     b->dirty = false;
     b->upload = true;
@@ -1154,9 +1158,37 @@ static int batch_build(lnt_batch *b) {
     return LNT_OK;
 }
 
-// Copy group g's parameter slots to the device, in the order of its stream.
-static int batch_upload(lnt_batch *b, lnt_batch::Group &g) {
-    BHIPCHK(b, hipMemcpyAsync(g.d, g.h.data(), g.h.size() * sizeof(LntParams), hipMemcpyHostToDevice, g.side),
+// Captures GRAPH_ITERS iterations of group g.
+static int batch_capture_group(lnt_batch *b, lnt_batch::Group &g) {
+    if (g.graph) (void)hipGraphDestroy(g.graph);  // of an instantiation that failed
+    g.graph = nullptr;
+    BHIPCHK(b, hipStreamBeginCapture(g.side, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    bool ok = true;
+    for (uint32_t i = 0; i < GRAPH_ITERS && ok; i++) ok = batch_group_step(g);
+    hipError_t ec = hipStreamEndCapture(g.side, &g.graph);
+    if (!ok || ec != hipSuccess) return bfail(b, LNT_DEVICE_ERROR, "batch graph capture failed");
+    BHIPCHK(b, hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0), "hipGraphInstantiate");
+    return LNT_OK;
+}
+
+// Captures one iteration of every group, each a branch off the batch stream.
+static int batch_capture_all(lnt_batch *b) {
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->graph = nullptr;
+    BHIPCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    bool ok = hipEventRecord(b->fork, b->stream) == hipSuccess;
+    for (auto &g : b->groups)
+        ok = ok && hipStreamWaitEvent(g.side, b->fork, 0) == hipSuccess && batch_group_step(g) &&
+             hipEventRecord(g.join, g.side) == hipSuccess && hipStreamWaitEvent(b->stream, g.join, 0) == hipSuccess;
+    hipError_t ec = hipStreamEndCapture(b->stream, &b->graph);
+    if (!ok || ec != hipSuccess) return bfail(b, LNT_DEVICE_ERROR, "batch graph capture failed");
+    BHIPCHK(b, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0), "hipGraphInstantiate");
+    return LNT_OK;
+}
+
+// Copy group g's parameter slots to the device, in the order of stream s.
+static int batch_upload(lnt_batch *b, lnt_batch::Group &g, hipStream_t s) {
+    BHIPCHK(b, hipMemcpyAsync(g.d, g.h.data(), g.h.size() * sizeof(LntParams), hipMemcpyHostToDevice, s),
             "hipMemcpy (batch parameters)");
     return LNT_OK;
 }
@@ -1182,7 +1214,7 @@ static void batch_refresh(lnt_batch *b) {
 }
 
 // After an iteration every LL member owes its "-2": refresh the flags where they changed.
-static int batch_mark_pending(lnt_batch *b, lnt_batch::Group &g) {
+static int batch_mark_pending(lnt_batch *b, lnt_batch::Group &g, hipStream_t s) {
     bool changed = false;
     for (u32 i = 0; i < g.cap; i++) {
         lnt_ctx *c = g.ctxs[i];
@@ -1195,21 +1227,55 @@ static int batch_mark_pending(lnt_batch *b, lnt_batch::Group &g) {
             changed = true;
         }
     }
-    return changed ? batch_upload(b, g) : LNT_OK;
+    return changed ? batch_upload(b, g, s) : LNT_OK;
+}
+
+// Steps that launch the graph of all groups for each iteration.  One iteration on the groups'
+// own streams pays for forking and joining them: per call, graph against streams, 41 / 61 us
+// with one test of 2^16, 48 / 69 with four, 73 / 88 with two shapes, 147 / 185 with four, 246 / 322
+// with eight.  Over several iterations the streams are ahead (two shapes, four iterations: 215 /
+// 190) until the host is behind with their launches: eight shapes take 409 / 519, 574 / 689 and
+// 741 / 872 us for two, three and four, six 295 / 303, 416 / 401 and 546 / 493.
+// The first such step of new groups takes the streams: capturing (0.1 to 0.5 ms) pays from the
+// second on.
+static bool batch_short(lnt_batch *b, uint32_t step) {
+    if (step != 1 && (step > 4 || b->groups.size() <= 6)) return false;
+    const bool again = b->again;
+    b->again = true;
+    return again;
+}
+
+// `step` iterations of every group on the batch stream.
+static int batch_run_short(lnt_batch *b, uint32_t step) {
+    int rc;
+    if (!b->exec && (rc = batch_capture_all(b))) return rc;
+    for (; step; step--) {
+        BHIPCHK(b, hipGraphLaunch(b->exec, b->stream), "hipGraphLaunch");
+        for (auto &g : b->groups) g.ran++;
+        for (auto &g : b->groups)
+            if ((rc = batch_mark_pending(b, g, b->stream))) return rc;
+    }
+    return LNT_OK;
 }
 
 // `step` iterations of group g on its stream.
 static int batch_group_run(lnt_batch *b, lnt_batch::Group &g, uint32_t step) {
     int rc;
-    // the first launch reads the members' "-2" flags as they are; after it every member owes one
-    for (bool first = true; step; first = false) {
+    // the first launch reads the members' "-2" flags as they are, after it every member owes one:
+    // one iteration goes ahead of the graph's where that changes a flag
+    // (a step of GRAPH_ITERS: the launches of a few groups keep ahead of the device, one test of 2^16
+    // takes 365 us and a replay 388, 24 tests in four groups 726 / 801; with six shapes it is 1725 / 1368)
+    bool steady = step > GRAPH_ITERS || b->groups.size() > 4;
+    for (u32 i = 0; i < g.cap; i++) steady = steady && (!g.ctxs[i] || g.h[i].sub2 == (g.ll ? 1u : 0u));
+    for (; step; steady = true) {
         uint32_t done = 1;
         if (g.pl.small) {  // the kernel loops over iterations; bounded launches keep each one short
             done = std::min<uint32_t>(step, small_chunk(g.pl));
             if (!lnt_launch_batch_small(g.pl, g.d, g.cap, done, g.ll, g.side))
                 return bfail(b, LNT_UNSUPPORTED, "no batched kernel for this shape");
-        } else if (!first && step >= GRAPH_ITERS) {
+        } else if (steady && step >= GRAPH_ITERS) {
             done = GRAPH_ITERS;
+            if (!g.exec && (rc = batch_capture_group(b, g))) return rc;
             BHIPCHK(b, hipGraphLaunch(g.exec, g.side), "hipGraphLaunch");
         } else if (!batch_group_step(g)) {
             return bfail(b, LNT_UNSUPPORTED, "no batched kernel for this shape");
@@ -1217,7 +1283,7 @@ static int batch_group_run(lnt_batch *b, lnt_batch::Group &g, uint32_t step) {
         BHIPCHK(b, hipGetLastError(), "kernel launch");
         step -= done;
         g.ran += done;
-        if (first && (rc = batch_mark_pending(b, g))) return rc;
+        if ((rc = batch_mark_pending(b, g, g.side))) return rc;
     }
     return LNT_OK;
 }
@@ -1300,7 +1366,7 @@ int lnt_batch_iterate(lnt_batch *b, uint32_t k) {
     if (b->dirty && (rc = batch_build(b))) return rc;
     if (b->upload)
         for (auto &g : b->groups)
-            if ((rc = batch_upload(b, g))) return rc;
+            if ((rc = batch_upload(b, g, b->stream))) return rc;
     b->upload = false;
     // Members under a Gerbicz check count the squarings as checked iterations: the groups
     // stop at each of their block ends for the block step on the member's stream.
@@ -1317,12 +1383,16 @@ int lnt_batch_iterate(lnt_batch *b, uint32_t k) {
             if (e != hipSuccess && rc == LNT_OK)
                 rc = bfail(b, LNT_DEVICE_ERROR, std::string(what) + " (" + hipGetErrorString(e) + ")");
         };
-        hip(hipEventRecord(b->fork, b->stream), "hipEventRecord");
-        for (auto &g : b->groups) {
-            hip(hipStreamWaitEvent(g.side, b->fork, 0), "hipStreamWaitEvent");
-            if (rc == LNT_OK) rc = batch_group_run(b, g, step);
-            hip(hipEventRecord(g.join, g.side), "hipEventRecord");
-            hip(hipStreamWaitEvent(b->stream, g.join, 0), "hipStreamWaitEvent");
+        if (batch_short(b, step)) {
+            rc = batch_run_short(b, step);
+        } else {
+            hip(hipEventRecord(b->fork, b->stream), "hipEventRecord");
+            for (auto &g : b->groups) {
+                hip(hipStreamWaitEvent(g.side, b->fork, 0), "hipStreamWaitEvent");
+                if (rc == LNT_OK) rc = batch_group_run(b, g, step);
+                hip(hipEventRecord(g.join, g.side), "hipEventRecord");
+                hip(hipStreamWaitEvent(b->stream, g.join, 0), "hipStreamWaitEvent");
+            }
         }
         left -= step;
         hip(hipEventRecord(b->done, b->stream), "hipEventRecord");

@@ -177,8 +177,9 @@ int lnt_batch_create(int device, lnt_batch **out);
 int lnt_batch_add(lnt_batch *batch, lnt_ctx *ctx);
 int lnt_batch_remove(lnt_batch *batch, lnt_ctx *ctx);
 int lnt_batch_size(const lnt_batch *batch);
-/* out[0] members, [1] kernel-shape groups, [2] times the iteration graphs were captured (members
- * joining or leaving a group with free slots only rewrite its parameters).  cap >= 3. */
+/* out[0] members, [1] kernel-shape groups, [2] times the groups were formed, whose steps then
+ * capture their iteration graphs (members joining or leaving a group with free slots only
+ * rewrite its parameters).  cap >= 3. */
 int lnt_batch_stats(const lnt_batch *batch, uint64_t *out, int cap);
 /* Every member advances k iterations (asynchronous). */
 int lnt_batch_iterate(lnt_batch *batch, uint32_t k);

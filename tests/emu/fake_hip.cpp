@@ -1,8 +1,8 @@
 // A HIP runtime without a device, for tests of the engine's host side (tests/test_host_calls.py).
 // Loaded ahead of liblnt.so with RTLD_GLOBAL, it takes the library's HIP calls: device memory is
 // host memory, kernels do nothing, and every call that orders or launches work is written to a
-// log ("launch stream kernel", "graph stream nodes", "record stream event", "wait stream event",
-// "copy stream bytes", "sync stream").  A launch can be made to fail.
+// log ("launch stream kernel", "graph stream nodes", "capture stream nodes", "record stream event",
+// "wait stream event", "copy stream bytes", "sync stream").  A launch can be made to fail.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -131,7 +131,7 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
     *g = g_capturing[s];
     for (auto i = g_capturing.begin(); i != g_capturing.end();) i = i->second == *g ? g_capturing.erase(i) : std::next(i);
     for (auto i = g_captured.begin(); i != g_captured.end();) i = i->second == *g ? g_captured.erase(i) : std::next(i);
-    return hipSuccess;
+    return note("capture", s, std::to_string(g_nodes[*g])), hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *, char *, size_t) {
     return *e = (hipGraphExec_t)g, hipSuccess;

@@ -91,3 +91,38 @@ print(json.dumps(dict(log=log(), sa=sa, sb=sb, failed=failed, st=a.gerbicz_stats
     assert len(of_groups) >= 10
     assert of_groups <= seen[got["sa"]] and of_groups <= seen[got["sb"]]
     assert got["st"]["iteration"] == 80 and got["st"]["checks"] == (2 if block == 40 else 0)
+
+
+def test_short_batch_steps_replay_graphs(fake):
+    """Steps of one iteration, and of up to four with many groups, launch one graph of all groups
+    for each iteration from the second such step on, and the first captures nothing; a step of
+    16 with many groups is one graph launch for each once the members' "-2" flags are right."""
+    got = fake("""
+ps = (9689, 1000003, 2000003)  # one workgroup, rows and columns
+ts = [cuda_amd.LucasPRP(p) for p in ps]
+batch = cuda_amd.Batch()
+for t in ts:
+    batch.add(t)
+steps = []
+for k in (1, 1, 1):
+    fake.fake_clear()
+    batch.iterate(k)
+    steps.append([(l[0], l[2]) for l in log() if l[0] in ("launch", "graph", "capture")])
+ts += [cuda_amd.LucasPRP(p, prp=True) for p in (400009, 1000003, 2000003, 4000037)]
+for t in ts[3:]:
+    batch.add(t)
+fake.fake_clear()
+batch.iterate(3)
+batch.iterate(4)
+batch.iterate(16)
+steps.append([(l[0], l[2]) for l in log() if l[0] in ("launch", "graph", "capture")])
+print(json.dumps(steps))
+""")
+    one = ["graph", "7"]  # 1 + 3 + 3 kernels
+    assert [s[0] for s in got[0]] == ["launch"] * 7
+    assert got[1] == [["capture", "7"], one]
+    assert got[2] == [one]
+    assert [s[0] for s in got[3][:55]] == ["launch"] * 55  # 3 of 6 * 3 kernels, and 1
+    assert got[3][55:60] == [["capture", "19"]] + [["graph", "19"]] * 4
+    sixteen = [s for s in got[3][60:] if s[0] != "capture"]
+    assert sixteen[1:] == [["graph", "48"]] * 6 and sixteen[0][0] == "launch"
