@@ -126,3 +126,31 @@ print(json.dumps(steps))
     assert got[3][55:60] == [["capture", "19"]] + [["graph", "19"]] * 4
     sixteen = [s for s in got[3][60:] if s[0] != "capture"]
     assert sixteen[1:] == [["graph", "48"]] * 6 and sixteen[0][0] == "launch"
+
+
+def test_long_batch_steps_launch_the_groups_in_turns(fake):
+    """A stream takes only so many launches ahead of the device: in a long step no group's launches
+    run ahead of another's by more than a few hundred iterations."""
+    got = fake("""
+ts = [cuda_amd.LucasPRP(p) for p in (86243, 1000003, 2000003)]
+batch = cuda_amd.Batch()
+for t in ts:
+    batch.add(t)
+batch.iterate(5)
+fake.fake_clear()
+batch.iterate(20001)
+print(json.dumps([l for l in log() if l[0] in ("launch", "graph")]))
+""")
+    done, ahead = {}, 0  # graph and kernel launches: 48 and 1 thirds of an iteration
+    for op, stream, what in got:
+        if "small" in what:
+            continue
+        done[stream] = done.get(stream, 0) + (48 if op == "graph" else 1)
+        ahead = max(ahead, max(done.values()) - (min(done.values()) if len(done) == 2 else 0))
+    assert sorted(done.values()) == [60003, 60003] and ahead <= 3 * 300
+    small = [l for l in got if "small" in l[2]]
+    assert len(small) == -(-20001 // 256) and len({l[1] for l in got}) == 3
+    first = {}
+    for i, l in enumerate(got):
+        first.setdefault(l[1], i)
+    assert max(first.values()) < 60  # every group has begun after one turn of the others
