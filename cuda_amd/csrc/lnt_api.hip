@@ -751,8 +751,13 @@ int lnt_tune(lnt_ctx *c, int loops) {
         float ms;
         std::vector<uint64_t> out;
     };
-    // candidates: every row/column split, column tile and row variant this build has
+    // candidates: every row/column split, column tile and row variant this build has, and the
+    // one-workgroup plan where a row length was asked for at n = 2048 or 4096
     std::vector<PlanOpts> opts;
+    {
+        Plan def;
+        if (make_plan(c->p, n, def).empty() && def.small) opts.push_back(PlanOpts());
+    }
     for (uint32_t lc = 7; lc <= 14; lc++)
         for (uint32_t K : {16u, 8u, 4u})
             for (int r3 : {-1, 0, 1, 2})

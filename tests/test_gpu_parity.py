@@ -141,6 +141,29 @@ def test_splits_at_2048_and_4096_match_oracle(p, n, plans, monkeypatch):
     assert len(seen) >= (1 if n == 2048 else 3)
 
 
+@pytest.mark.parametrize("p,n", [(44497, 2048), (86243, 4096)])
+def test_tuning_returns_to_the_one_workgroup_plan(p, n, monkeypatch):
+    """A context on the row/column path of n = 2048 or 4096 can be tuned to the one-workgroup
+    kernel (at 2048 a quarter of its time) and keeps its residue."""
+    monkeypatch.setenv("LNT_PLAN", "lc=7")
+    t = cuda_amd.LucasPRP(p, n)
+    monkeypatch.delenv("LNT_PLAN")
+    say("tune back", n, t.describe())
+    assert t.describe()[0].startswith("LNT_2PASS")
+    t.iterate(7)
+    t.tune(200)
+    say(t.describe(), sorted(t.tune_results(), key=lambda r: r[1])[:4])
+    assert any("lnt_k_small16" in name for name, _ in t.tune_results())
+    if n == 2048:
+        assert t.describe()[1] == "lnt_k_small16<8>", t.tune_results()
+    t.iterate(6)
+    o = OracleTest(p, n, False)
+    o.iterate(13)
+    assert t.get_digits() == o.digits()
+    t.close()
+    cuda_amd.lnt.tune_import(f"0 {n} 0 0 -1 -1\n")  # the default plan for the tests after this one
+
+
 @pytest.mark.parametrize("p,n", [(318767093, 1 << 24), (600000001, 1 << 25), (1200000001, 1 << 26)])
 def test_longest_lengths_match_oracle(p, n):
     """n = 2^24, 2^25 and 2^26 (rows of 8192, 8192 and 16384 words, mixed-radix 3-phase row

@@ -154,3 +154,19 @@ print(json.dumps([l for l in log() if l[0] in ("launch", "graph")]))
     for i, l in enumerate(got):
         first.setdefault(l[1], i)
     assert max(first.values()) < 60  # every group has begun after one turn of the others
+
+
+def test_tuner_offers_the_one_workgroup_plan(fake):
+    """A context of 2048 or 4096 words on a row/column plan (a saved choice of its length) can be
+    tuned back to the one-workgroup kernel, which no row length names."""
+    got = fake("""
+out = []
+for p, n in ((44497, 2048), (86243, 4096)):
+    cuda_amd.lnt.tune_import("0 %d 7 16 -1 -1\\n" % n)
+    t = cuda_amd.LucasPRP(p, n)
+    out.append((t.describe()[0], (t.tune(10), [name for name, ms in t.tune_results()])[1]))
+print(json.dumps(out))
+""")
+    for (plan, names), kernel in zip(got, ("lnt_k_small16<8>", "lnt_k_small16<16>")):
+        assert plan.startswith("LNT_2PASS"), plan
+        assert any(kernel in name for name in names), names
