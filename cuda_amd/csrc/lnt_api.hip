@@ -487,12 +487,17 @@ const char *lnt_last_error(const lnt_ctx *c) {
 
 uint32_t lnt_secured_log2_length(uint32_t p) { return secured_log2_length(p); }
 
-// Tuned plans as text, one line per (device, length): "device n lc K row3 col3".
+// Tuned plans as text, one line per (device, length), "device n lc K row3 col3", under a line that
+// names the set of kernels they were chosen among.  The number counts those sets (row3 and col3
+// name variants; -1 leaves the choice to the plan): raise it when kernels join or leave.
+static const char kTuneSet[] = "# kernels 2";
+
 int lnt_tune_export(char *buf, size_t len) {
     if (!buf || !len) return fail(nullptr, LNT_INVALID_ARGUMENT, "bad argument");
     std::string out;
     {
         std::lock_guard<std::mutex> lk(g_tuned_mu);
+        if (!g_tuned.empty()) out = std::string(kTuneSet) + "\n";
         for (const auto &kv : g_tuned) {
             char line[96];
             std::snprintf(line, sizeof line, "%d %u %u %u %d %d\n", kv.first.first, kv.first.second, kv.second.lc,
@@ -508,15 +513,19 @@ int lnt_tune_import(const char *text) {
     if (!text) return fail(nullptr, LNT_INVALID_ARGUMENT, "bad argument");
     std::vector<std::pair<std::pair<int, uint32_t>, PlanOpts>> rows;
     const char *s = text;
+    bool same_set = false;
     while (*s) {
         const char *e = std::strchr(s, '\n');
         std::string line(s, e ? (size_t)(e - s) : std::strlen(s));
         s = e ? e + 1 : s + line.size();
-        if (line.find_first_not_of(" \t\r") == std::string::npos || line[0] == '#') continue;
+        while (!line.empty() && std::strchr(" \t\r", line.back())) line.pop_back();
+        if (line.compare(0, 10, kTuneSet, 10) == 0) same_set = line == kTuneSet;
+        if (line.empty() || line[0] == '#') continue;
         int dev = 0, r3 = -1, c3 = -1;
         unsigned n = 0, lc = 0, K = 0;
         if (std::sscanf(line.c_str(), "%d %u %u %u %d %d", &dev, &n, &lc, &K, &r3, &c3) != 6 || !n || (n & (n - 1)))
             return fail(nullptr, LNT_INVALID_ARGUMENT, "lnt_tune_import: bad line '" + line + "'");
+        if (!same_set && (r3 >= 0 || c3 >= 0)) continue;  // chosen among other kernels
         PlanOpts o;
         o.lc = lc;
         o.K = K;

@@ -144,7 +144,8 @@ def tune_export() -> str:
 
 
 def tune_import(text: str) -> None:
-    """Merge saved tuner choices (the format of tune_export) for later contexts."""
+    """Merge saved tuner choices (the format of tune_export, with its first line) for later
+    contexts; kernel variants chosen among another build's kernels are left out."""
     lib = load()
     rc = lib.lnt_tune_import(text.encode())
     if rc != LNT_OK:

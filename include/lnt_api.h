@@ -93,9 +93,11 @@ const char *lnt_last_error(const lnt_ctx *ctx);
 uint32_t lnt_secured_log2_length(uint32_t p);
 
 /* The tuner's choices as text, one line per device and length: "device n lc K row3 col3"
- * (new: the reference re-tunes at every start, process.cu:45-127).  Export fills buf
- * (LNT_INVALID_ARGUMENT if it is too small); import merges lines into the choices used
- * by later lnt_create calls.  Both are host-only. */
+ * (new: the reference re-tunes at every start, process.cu:45-127), under a comment line that
+ * names the set of kernels they were chosen among.  Export fills buf (LNT_INVALID_ARGUMENT if
+ * it is too small); import merges lines into the choices used by later lnt_create calls.
+ * Without that comment, or under another set's, lines that name a kernel variant (row3 or col3
+ * not -1) are left out.  Both are host-only. */
 int lnt_tune_export(char *buf, size_t len);
 int lnt_tune_import(const char *text);
 

@@ -56,3 +56,23 @@ def test_tuner_choices_round_trip_as_text():
     assert "0 4194304 12 16 -1 -1" in out and "0 65536 12 16 -1 -1" in out
     with pytest.raises(LntError):
         tune_import("0 1000 12 16 1 1\n")  # not a power of two
+
+
+def test_tuner_choices_of_other_kernels_are_left_out():
+    """Saved choices carry the set of kernels they were made among.  Of a text without it, or of
+    another set, only the lines that name no kernel variant count: a variant chosen among other
+    kernels would keep the present ones from being used."""
+    from cuda_amd.lnt import LntError, tune_export, tune_import
+    old, new = "0 2097152 12 16 1 1", "0 1048576 12 16 1 0"
+    tune_import(old + "\n0 524288 11 16 -1 -1\n")
+    out = tune_export().splitlines()
+    assert old not in out and "0 524288 11 16 -1 -1" in out
+    head = out[0]
+    assert head.startswith("# ")  # read as a comment by builds that know no header
+    tune_import(f"{head}\n{new}\n")
+    assert new in tune_export().splitlines()
+    tune_import(head[:-1] + str(int(head[-1]) + 1) + f"\n{old}\n")
+    assert old not in tune_export().splitlines()
+    for text in ("0 2097152 12 16 1\n", f"{head}\n0 1000 12 16 1 1\n"):
+        with pytest.raises(LntError):
+            tune_import(text)
