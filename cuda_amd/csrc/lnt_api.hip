@@ -870,8 +870,10 @@ int lnt_tune(lnt_ctx *c, int loops) {
 // ------------------------------------------------------------------ products, copies, faults
 
 static bool same_shape(const lnt_ctx *a, const lnt_ctx *b) {
-    // the transform-domain slot order depends on the split and on the row/column variants
-    return a->device == b->device && a->p == b->p && a->prp == b->prp && same_slots(a->pl, b->pl);
+    // residues lie in natural order whatever the kernels, and a product transforms both of its
+    // operands with the plan and tables of dst
+    return a->device == b->device && a->p == b->p && a->prp == b->prp && a->pl.n == b->pl.n && a->pl.C == b->pl.C &&
+           a->pl.R == b->pl.R;
 }
 
 int lnt_mul(lnt_ctx *dst, lnt_ctx *src) {

@@ -82,16 +82,6 @@ inline bool same_kernels(const Plan &a, const Plan &b) {
            a.colm == b.colm && a.col3 == b.col3 && a.cBB == b.cBB && a.cBC == b.cBC && a.M == b.M;
 }
 
-// Two plans order the transform domain the same way (the column tile width, rows per
-// workgroup and carry halo do not change where a frequency is stored).
-inline bool same_slots(const Plan &a, const Plan &b) {
-    Plan x = a;
-    x.K = b.K;
-    x.G = b.G;
-    x.M = b.M;
-    return same_kernels(x, b);
-}
-
 // Carry levels m such that digits stay bounded by D with every pre-carry value below P/2
 // in steady state, in exact integer arithmetic.  0 if no m <= 8 works.
 //  * Digits |d| <= D give convolution outputs |C| <= 2 n D^2 (the IBDWT factors

@@ -128,7 +128,8 @@ int lnt_profile(lnt_ctx *ctx, uint32_t iters, char *names, size_t names_len, flo
 /* ---- products, copies and the Gerbicz-checked PRP (new: the reference has no error
  * check and no general multiply) ---- */
 
-/* dst <- dst * src mod M_p.  Both contexts must share p, n, mode and row/column split. */
+/* dst <- dst * src mod M_p.  Both contexts must share p, n, mode and row/column split; the
+ * kernel variants may differ. */
 int lnt_mul(lnt_ctx *dst, lnt_ctx *src);
 
 /* dst <- src (residue and its bookkeeping). */

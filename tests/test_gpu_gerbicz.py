@@ -47,6 +47,33 @@ def test_product_matches_python(p, n, prp):
     assert value_of(x.get_digits(), p, n) == ((a * b % M) ** 2 - c) % M
 
 
+@pytest.mark.parametrize("p,n,plans", [(1279, 64, ("", "row3=0")), (19937, 1024, ("row3=0", "")),
+                                       (1000003, 65536, ("lc=8", "lc=8,row3=0")),
+                                       (2000003, 131072, ("lc=7,K=8", "lc=7"))])
+def test_product_of_two_variants_matches_python(p, n, plans, monkeypatch):
+    """Operands whose contexts share the split but run other kernels."""
+    say("product of variants", p, n, plans)
+    rnd = random.Random(p ^ n)
+    M = (1 << p) - 1
+    a, b = rnd.randrange(M), rnd.randrange(M)
+    ts = []
+    for plan, v in zip(plans, (a, b)):
+        monkeypatch.setenv("LNT_PLAN", plan)
+        t = cuda_amd.LucasPRP(p, n)
+        t.set_digits(digits_of(v, p, n))
+        t.iterate(1)
+        ts.append(t)
+    x, y = ts
+    assert x.describe() != y.describe()
+    a, b = (a * a - 2) % M, (b * b - 2) % M
+    x.mul(y)
+    assert value_of(x.get_digits(), p, n) == a * b % M
+    assert value_of(y.get_digits(), p, n) == b
+    y.copy_from(x)
+    y.iterate(1)
+    assert value_of(y.get_digits(), p, n) == ((a * b % M) ** 2 - 2) % M
+
+
 def run_checked(p, n, iters, block, per_check, inject_at=None, word=17, mask=1 << 9):
     t = cuda_amd.LucasPRP(p, n, prp=True)
     t.gerbicz_begin(block, per_check)

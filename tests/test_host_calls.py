@@ -170,3 +170,31 @@ print(json.dumps(out))
     for (plan, names), kernel in zip(got, ("lnt_k_small16<8>", "lnt_k_small16<16>")):
         assert plan.startswith("LNT_2PASS"), plan
         assert any(kernel in name for name in names), names
+
+
+def test_products_and_copies_take_every_variant_of_a_split(fake):
+    """lnt_mul and lnt_copy ask for the same p, n, mode and row/column split, whatever kernels the
+    two contexts run; another split is refused."""
+    got = fake("""
+import os
+def make(p, n, plan):
+    os.environ["LNT_PLAN"] = plan
+    return cuda_amd.LucasPRP(p, n, prp=True)
+out = []
+for p, n, a, b in ((70000027, 1 << 22, "", "K=8"), (16000057, 1 << 20, "", "col3=0"), (16000057, 1 << 20, "lc=10,K=16", "lc=10,K=8"),
+                   (1000003, 65536, "lc=8", "lc=8,row3=0"), (19937, 1024, "", "row3=0"), (1279, 64, "", "row3=0"),
+                   (1000003, 65536, "lc=9", "lc=10"), (1000003, 65536, "", "lc=12")):
+    x, y = make(p, n, a), make(p, n, b)
+    ok = []
+    for call in (x.mul, x.copy_from):
+        try:
+            call(y)
+            ok.append(True)
+        except cuda_amd.LntError:
+            ok.append(False)
+    out.append((n, a, b, x.describe() != y.describe(), ok))
+print(json.dumps(out))
+""")
+    for n, a, b, differ, ok in got:
+        assert differ, (n, a, b)
+        assert ok == [a + b not in ("lc=9lc=10", "lc=12")] * 2, (n, a, b, ok)
