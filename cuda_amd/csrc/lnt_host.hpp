@@ -6,8 +6,8 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -360,7 +360,7 @@ inline bool to_canonical_digits(const std::vector<uint8_t> &w, const uint64_t *x
     for (size_t k = 1; k < T; k++) {
         try {
             th[k] = std::thread(run, k);
-        } catch (const std::system_error &) {  // no thread available
+        } catch (const std::exception &) {  // no thread, or no memory to start one
             run(k);
         }
     }

@@ -489,6 +489,26 @@ extern "C" void emu_set_digits(void *h, const uint64_t *d) {
     e->pending = false;
 }
 
+// Allocations of this library, the nth of which from now on fails.
+static int g_fail_new = 0;
+void *operator new(size_t n) {
+    if (g_fail_new && --g_fail_new == 0) throw std::bad_alloc();
+    if (void *p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
+// The canonical digits of pre-carry words, in place; the fail_new-th allocation fails.
+extern "C" int emu_canonical(uint32_t p, uint32_t n, uint64_t *x, int sub2, int fail_new) {
+    std::vector<uint8_t> w;
+    widths(p, n, w);
+    g_fail_new = fail_new;
+    const bool zero = to_canonical_digits(w, x, sub2 != 0, x);
+    g_fail_new = 0;
+    return zero;
+}
+
 extern "C" void emu_batch_forms(void *h, int on) { ((Emu *)h)->batch_forms = on != 0; }
 extern "C" void emu_wide_rows(void *h, int on) { ((Emu *)h)->wide_rows = on != 0; }
 extern "C" uint32_t emu_levels(void *h) { return ((Emu *)h)->pl.levels; }

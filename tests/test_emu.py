@@ -395,6 +395,43 @@ def test_plan_fallback_is_the_default_plan():
                             assert tuple(out) == default, (n, lc, K, r3, c3, tuple(out), default)
 
 
+@pytest.mark.parametrize("p,n,sub2", [(4000037, 1 << 18, False), (16000057, 1 << 20, True)])
+def test_readout_carries_in_runs(p, n, sub2):
+    """Canonical digits of pre-carry words by 2 and 8 host threads, in place, against one carry
+    over all of them: random words, a zero, and carries that ripple through whole runs; also when
+    a thread cannot be started."""
+    import numpy as np
+    L = emu()
+    L.emu_canonical.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_int, ctypes.c_int]
+    i = np.arange(n + 1, dtype=np.uint64)
+    w = np.diff((np.uint64(p) * i + np.uint64(n - 1)) // np.uint64(n)).astype(np.int64)
+    mask = (np.int64(1) << w) - 1
+    rng = np.random.default_rng(p)
+    ones = mask.copy()
+    ones[0] += 1  # 2^p: the carry runs through every digit, and 1 is left
+    cases = [rng.integers(-(1 << 62), 1 << 62, n), np.zeros(n, np.int64), ones, -mask, mask.copy()]
+    for v in cases:
+        want, carry = v.tolist(), 0
+        if sub2:
+            want[0] -= 2
+        wl = w.tolist()
+        while True:  # 2^p = 1: the carry out of the last digit enters the first
+            for j, wj in enumerate(wl):
+                t = want[j] + carry
+                want[j], carry = t & ((1 << wj) - 1), t >> wj
+            if not carry:
+                break
+        if want == mask.tolist():
+            want = [0] * n
+        zero = not any(want)
+        P = (1 << 64) - (1 << 32) + 1
+        field = np.where(v < 0, v.astype(np.uint64) + np.uint64(P), v.astype(np.uint64))  # (mod 2^64)
+        for fail_new in (0, 1, 3):
+            x = field.copy()
+            assert L.emu_canonical(p, n, x.ctypes.data, int(sub2), fail_new) == int(zero)
+            assert x.tolist() == want, (p, fail_new)
+
+
 def test_biased_weight_multiply_matches_python():
     """gl_mul_biased(d + 2^31, w, -2^31 w mod P) = d w mod P for every 32-bit biased digit,
     edge operands and random ones (the column kernels' weight multiply on carried digits)."""
