@@ -549,8 +549,9 @@ extern "C" int emu_plan_retry(uint32_t p, uint32_t n, uint32_t lc, uint32_t K, i
         used = 0;
         if (!make_plan(p, n, pl, PlanOpts()).empty()) return -1;
     }
-    const uint32_t v[10] = {pl.n, pl.C, pl.R, pl.col3, pl.cBB, pl.cBC, pl.K, pl.row3, pl.row3m, pl.G};
-    for (int i = 0; i < 10; i++) out[i] = v[i];
+    const uint32_t v[12] = {pl.n,   pl.C,     pl.R, pl.col3, pl.cBB,  pl.cBC,
+                            pl.K,   pl.row3,  pl.row3m, pl.G, pl.rowm, pl.colm};
+    for (int i = 0; i < 12; i++) out[i] = v[i];
     *consistent = plan_consistent(pl) ? 1 : 0;
     return used;
 }

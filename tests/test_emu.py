@@ -376,7 +376,7 @@ def test_plan_fallback_is_the_default_plan():
     L.emu_plan_retry.argtypes[5] = ctypes.c_int
     L.emu_secured.argtypes = [ctypes.c_uint32]
     L.emu_secured.restype = ctypes.c_uint32
-    out = (ctypes.c_uint32 * 10)()
+    out = (ctypes.c_uint32 * 12)()
     ok = ctypes.c_int()
     for log_n in range(13, 27):
         n = 1 << log_n
@@ -387,8 +387,10 @@ def test_plan_fallback_is_the_default_plan():
         default = tuple(out)
         for lc in range(7, 15):
             for K in (16, 8, 4):
-                for r3 in (0, 1, 2):
-                    for c3 in (0, 1):
+                for r3 in (-1, 0, 1, 2):
+                    for c3 in (-1, 0, 1):
+                        if -1 in (r3, c3) and K != 16:
+                            continue  # matrix-core columns have one tile width
                         used = L.emu_plan_retry(p, n, lc, K, r3, c3, out, ctypes.byref(ok))
                         assert used in (0, 1) and ok.value == 1, (n, lc, K, r3, c3)
                         if used == 0:

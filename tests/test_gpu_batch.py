@@ -1,5 +1,5 @@
-"""GPU: batched tests (all members advance in one hipGraph launch per iteration) leave
-every member exactly where the same test run alone on the plain path leaves it.
+"""GPU: batched tests (members of one shape share batched launches, the shapes advance side by
+side) leave every member exactly where the same test run alone on the plain path leaves it.
 
 Bar: bit-exact residues (full digit vectors), across several graph replays with the
 program's own eager work between them, membership changes, a member re-planned by the
@@ -237,7 +237,8 @@ def test_membership_changes_reuse_the_graph():
 
 @pytest.mark.parametrize("ps", [[8000009 + 2 * i for i in range(6)],  # 2^19: 2048-word rows four to a workgroup
                                 [1048583, 4000037, 4000039],          # 2^18: 256-word columns, 8 and 4 halo digits
-                                [16000057]])                          # 2^20
+                                [16000057],                           # 2^20: 256-word columns in tiles of four waves
+                                [4194319, 16000057]])                 # the same with 8 and 4 halo digits
 def test_batch_kernel_forms_match_solo(ps):
     """The kernel forms that only batches launch leave the residues of the plain path's."""
     say("batch forms", ps)

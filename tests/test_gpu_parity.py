@@ -77,18 +77,41 @@ def test_large_random_state_matches_oracle(p, n, prp):
     t.close()
 
 
+@pytest.mark.parametrize("p,n", [(131, 64), (263, 128), (769, 256), (2063, 512), (4099, 1024), (8209, 2048),
+                                 (16411, 4096), (32771, 8192), (262147, 65536), (1048583, 1 << 18),
+                                 (4194319, 1 << 20), (20971529, 1 << 22)])
+def test_few_bits_per_digit_match_oracle(p, n):
+    """Digits of 2 to 5 bits take more than four carry levels: the kernels with a halo of eight
+    digits, from a random residue against the oracle digit for digit (LL, three iterations)."""
+    from helpers import random_digits_np
+    import numpy as np
+    say("eight halo digits", p, n)
+    d = random_digits_np(p, n, seed=p)
+    t = cuda_amd.LucasPRP(p, n)
+    t.set_digits(d)
+    t.iterate(3)
+    got = np.asarray(t.get_digits_buffer(), dtype=np.uint64)
+    t.close()
+    o = OracleTest(p, n, False, n0=1 if n <= 65536 else 1024)
+    o.set_digits_np(d)
+    o.iterate(3)
+    assert np.array_equal(got, o.digits_np())
+
+
 # The tuner's candidate grid (lnt_tune): row length 2^lc, column tile K, row and column
-# variants.  Shapes a length does not support fall back to its default plan, so the
-# distinct plans are those lnt_describe reports.
+# variants (-1: the plan's choice, the matrix-core kernels where there are any).  Shapes a
+# length does not support fall back to its default plan, so the distinct plans are those
+# lnt_describe reports.
 TUNER_GRID = [f"lc={lc},K={K},row3={r3},col3={c3}" for lc in range(7, 15) for K in (16, 8, 4)
-              for r3 in (0, 1, 2) for c3 in (0, 1)]
+              for r3 in (-1, 0, 1, 2) for c3 in (-1, 0, 1)]
 
 
 @pytest.mark.parametrize("p,n", [(2000003, 1 << 17), (16000057, 1 << 20), (70000027, 1 << 22),
                                  (140000041, 1 << 23)])
 def test_every_tunable_plan_matches_oracle(p, n, monkeypatch):
     """Every plan lnt_tune can choose at this length, forced through LNT_PLAN, against the
-    oracle digit for digit from a random residue (LL, two iterations)."""
+    oracle digit for digit from a random residue (LL, two iterations); every matrix-core row and
+    column kernel that a split of this length takes is among them."""
     import numpy as np
     from helpers import random_digits_np
     d = random_digits_np(p, n, seed=n + 5)
@@ -106,21 +129,27 @@ def test_every_tunable_plan_matches_oracle(p, n, monkeypatch):
             continue
         seen.add(desc)
         say("plan", n, plan, ";".join(desc))
-        t.set_digits(d.tolist())
+        t.set_digits(d)
         t.iterate(2)
         got = np.asarray(t.get_digits_buffer(), dtype=np.uint64)
         assert np.array_equal(got, want), (n, plan, desc)
         t.close()
     say("distinct plans", n, len(seen))
+    kernels, log_n = {k for desc in seen for k in desc}, n.bit_length() - 1
+    for lc in range(max(7, log_n - 12), min(14, log_n - 4) + 1):
+        if 8 <= lc <= 11:
+            assert f"lnt_k_rowm<{1 << (lc - 8)}>" in kernels
+        if log_n - lc in (8, 10):
+            assert f"lnt_k_colm_fwd<{1 << (log_n - lc - 8)}>" in kernels
     assert len(seen) >= 3
 
 
 @pytest.mark.parametrize("p,n,plans", [(44497, 2048, ["", "lc=7"]),
                                        (86243, 4096, ["", "lc=7", "lc=8", "lc=8,K=8", "row3=0"])])
 def test_splits_at_2048_and_4096_match_oracle(p, n, plans, monkeypatch):
-    """n = 2048 (three launches by default) and 4096 (one workgroup by default, or the
-    three-kernel path when a row length is asked for): every plan against the oracle digit
-    for digit from a random residue (LL, three iterations)."""
+    """n = 2048 and 4096 (one workgroup by default, or the three-kernel path when a row length is
+    asked for): every plan against the oracle digit for digit from a random residue (LL, three
+    iterations)."""
     rnd = random.Random(p + n)
     o = OracleTest(p, n, False)
     d = [rnd.getrandbits(wi) for wi in o.widths()]
@@ -138,7 +167,7 @@ def test_splits_at_2048_and_4096_match_oracle(p, n, plans, monkeypatch):
         t.iterate(3)
         assert t.get_digits() == want, (n, plan, desc)
         t.close()
-    assert len(seen) >= (1 if n == 2048 else 3)
+    assert len(seen) >= (2 if n == 2048 else 3)
 
 
 @pytest.mark.parametrize("p,n", [(44497, 2048), (86243, 4096)])
