@@ -1046,16 +1046,23 @@ int lnt_gerbicz_stats(lnt_ctx *c, uint64_t *out, int cap) {
 // ------------------------------------------------------------------ batches
 // Many independent tests advanced together: members with the same plan shape form a
 // group that runs as one batched launch per kernel (per-test parameters in a device
-// array).  Groups do not wait for each other inside a step: each runs its iterations on a
-// stream of its own, single-workgroup groups as one launch that loops over them, the others
+// array).  Groups do not wait for each other inside a step: they run their iterations on
+// streams of the batch, single-workgroup groups as one launch that loops over them, the others
 // as replays of a captured graph of GRAPH_ITERS iterations and the remainder one by one.
 // (Stepping all groups together, one graph launch per iteration with the groups as its
-// branches, spent 97 us per iteration on 24 tests of 2^11 .. 2^14 words; only short steps are
-// run so, see batch_short.)
+// branches, spent 97 us per iteration on 24 tests of 2^11 .. 2^14 words; only steps of one
+// iteration are run so, see batch_run_one.)
 
 struct lnt_batch {
     int device = 0;
     hipStream_t stream = nullptr;
+    // The groups' streams, as many as a process has hardware queues by default, made with the
+    // batch.  A stream goes to the least used queue when it is made: streams made for each new
+    // group landed between those of contexts that come and go, several on one queue, where the
+    // groups wait for each other (24 tests in four groups, 500 squarings: 20.6 ms, and 8.7 so;
+    // forming eight groups took 0.9 ms, and 0.3 so).
+    static constexpr int SIDES = 4;
+    hipStream_t sides[SIDES] = {};
     hipEvent_t ev_mark = nullptr;
     std::vector<lnt_ctx *> members;
     // Members of one kernel shape share one batched launch per kernel over `cap` parameter
@@ -1068,7 +1075,7 @@ struct lnt_batch {
         std::vector<lnt_ctx *> ctxs;  // cap slots, nullptr = empty
         std::vector<LntParams> h;     // cap slots, n = 0 = empty
         LntParams *d = nullptr;
-        hipStream_t side = nullptr;
+        hipStream_t side = nullptr;  // one of the batch's
         hipEvent_t join = nullptr;
         hipGraph_t graph = nullptr;  // GRAPH_ITERS iterations (not for single-workgroup tests)
         hipGraphExec_t exec = nullptr;
@@ -1077,9 +1084,9 @@ struct lnt_batch {
     std::vector<Group> groups;
     hipEvent_t fork = nullptr;
     hipEvent_t done = nullptr;  // end of the last batch_iterate: members' streams wait on it
-    hipGraph_t graph = nullptr;  // one iteration of every group (for short steps)
+    hipGraph_t graph = nullptr;  // one iteration of every group
     hipGraphExec_t exec = nullptr;
-    bool again = false;     // these groups have made a short step
+    bool again = false;     // these groups have made a step of one iteration
     bool dirty = true;      // the groups or their capacities changed: new groups and graphs
     bool upload = false;    // parameters changed: copy them to the device before the next step
     uint64_t captures = 0;  // times the groups were formed, whose steps capture their graphs
@@ -1115,7 +1122,6 @@ static void batch_release(lnt_batch *b) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (g.graph) (void)hipGraphDestroy(g.graph);
         if (g.d) (void)hipFree(g.d);
-        if (g.side) (void)hipStreamDestroy(g.side);
         if (g.join) (void)hipEventDestroy(g.join);
     }
     b->groups.clear();
@@ -1142,8 +1148,8 @@ static lnt_batch::Group *group_of(lnt_batch *b, const lnt_ctx *c) {
 }
 
 // Groups for the current members, each with room to grow (at least 8 slots, a power of
-// two, at least twice its members), their parameters and streams.  The first step that
-// replays a graph captures it.
+// two, at least twice its members), and their parameters.  The first step that replays a
+// graph captures it.
 static int batch_build(lnt_batch *b) {
     batch_release(b);
     for (lnt_ctx *c : b->members) {
@@ -1165,7 +1171,7 @@ static int batch_build(lnt_batch *b) {
         for (u32 i = 0; i < cap; i++)
             if (g.ctxs[i]) g.h[i] = member_params(g.ctxs[i]);
         BHIPCHK(b, hipMalloc(&g.d, g.h.size() * sizeof(LntParams)), "hipMalloc (batch parameters)");
-        BHIPCHK(b, hipStreamCreateWithFlags(&g.side, hipStreamNonBlocking), "hipStreamCreate");
+        g.side = b->sides[(&g - b->groups.data()) % lnt_batch::SIDES];
         BHIPCHK(b, hipEventCreateWithFlags(&g.join, hipEventDisableTiming), "hipEventCreate");
     }
     b->dirty = false;
@@ -1246,31 +1252,18 @@ static int batch_mark_pending(lnt_batch *b, lnt_batch::Group &g, hipStream_t s) 
     return changed ? batch_upload(b, g, s) : LNT_OK;
 }
 
-// Steps that launch the graph of all groups for each iteration.  One iteration on the groups'
-// own streams pays for forking and joining them: per call, graph against streams, 41 / 61 us
-// with one test of 2^16, 48 / 69 with four, 73 / 88 with two shapes, 147 / 185 with four, 246 / 322
-// with eight.  Over several iterations the streams are ahead (two shapes, four iterations: 215 /
-// 190) until the host is behind with their launches: eight shapes take 409 / 519, 574 / 689 and
-// 741 / 872 us for two, three and four, six 295 / 303, 416 / 401 and 546 / 493.
-// The first such step of new groups takes the streams: capturing (0.1 to 0.5 ms) pays from the
-// second on.
-static bool batch_short(lnt_batch *b, uint32_t step) {
-    if (step != 1 && (step > 4 || b->groups.size() <= 6)) return false;
-    const bool again = b->again;
-    b->again = true;
-    return again;
-}
-
-// `step` iterations of every group on the batch stream.
-static int batch_run_short(lnt_batch *b, uint32_t step) {
+// A step of one iteration as a graph of all groups, on the batch stream: the groups' streams
+// need not be forked and joined (per call, graph against streams, 40 / 62 us with one test of
+// 2^16, 47 / 71 with four, 75 / 89 with two shapes, 143 / 134 with four, 224 / 259 with eight;
+// steps of two and more are faster on the streams).  Capturing it takes 0.1 to 0.5 ms, which pays
+// from the second such step of the same groups on.
+static int batch_run_one(lnt_batch *b) {
     int rc;
     if (!b->exec && (rc = batch_capture_all(b))) return rc;
-    for (; step; step--) {
-        BHIPCHK(b, hipGraphLaunch(b->exec, b->stream), "hipGraphLaunch");
-        for (auto &g : b->groups) g.ran++;
-        for (auto &g : b->groups)
-            if ((rc = batch_mark_pending(b, g, b->stream))) return rc;
-    }
+    BHIPCHK(b, hipGraphLaunch(b->exec, b->stream), "hipGraphLaunch");
+    for (auto &g : b->groups) g.ran = 1;
+    for (auto &g : b->groups)
+        if ((rc = batch_mark_pending(b, g, b->stream))) return rc;
     return LNT_OK;
 }
 
@@ -1285,9 +1278,11 @@ static int batch_group_turn(lnt_batch *b, lnt_batch::Group &g, uint32_t step) {
     int rc;
     // the first launch reads the members' "-2" flags as they are, after it every member owes one:
     // one iteration goes ahead of the graph's where that changes a flag
-    // (a step of GRAPH_ITERS: the launches of a few groups keep ahead of the device, one test of 2^16
-    // takes 365 us and a replay 388, 24 tests in four groups 726 / 801; with six shapes it is 1725 / 1368)
-    bool steady = step > GRAPH_ITERS || b->groups.size() > 4;
+    // (a step of GRAPH_ITERS: the launches of one row/column group keep ahead of the device, 367 us
+    // at 2^16 against 391 for a replay; with two shapes it is 500 / 418, with four 1271 / 1082)
+    int lines = 0;
+    for (auto &o : b->groups) lines += !o.pl.small;
+    bool steady = step > GRAPH_ITERS || lines > 1;
     for (u32 i = 0; i < g.cap; i++) steady = steady && (!g.ctxs[i] || g.h[i].sub2 == (g.ll ? 1u : 0u));
     uint32_t turn = std::min(step - g.ran, g.pl.small ? small_chunk(g.pl) : TURN_ITERS + !steady);
     for (; turn; steady = true) {
@@ -1317,11 +1312,13 @@ int lnt_batch_create(int device, lnt_batch **out) {
     if (!out) return fail(nullptr, LNT_INVALID_ARGUMENT, "out is NULL");
     lnt_batch *b = new lnt_batch;
     b->device = device;
-    if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
+    bool sides = hipSetDevice(device) == hipSuccess;
+    for (auto &s : b->sides) sides = sides && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess;
+    if (!sides || hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&b->ev_mark) != hipSuccess || hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess ||
         hipEventRecord(b->ev_mark, b->stream) != hipSuccess) {
-        delete b;
+        lnt_batch_destroy(b);
         return fail(nullptr, LNT_DEVICE_ERROR, "lnt_batch_create: HIP stream/event set-up failed");
     }
     *out = b;
@@ -1406,8 +1403,10 @@ int lnt_batch_iterate(lnt_batch *b, uint32_t k) {
             if (e != hipSuccess && rc == LNT_OK)
                 rc = bfail(b, LNT_DEVICE_ERROR, std::string(what) + " (" + hipGetErrorString(e) + ")");
         };
-        if (batch_short(b, step)) {
-            rc = batch_run_short(b, step);
+        const bool again = b->again;
+        if (step == 1) b->again = true;
+        if (step == 1 && again) {
+            rc = batch_run_one(b);
         } else {
             hip(hipEventRecord(b->fork, b->stream), "hipEventRecord");
             for (auto &g : b->groups) hip(hipStreamWaitEvent(g.side, b->fork, 0), "hipStreamWaitEvent");
@@ -1466,6 +1465,8 @@ void lnt_batch_destroy(lnt_batch *b) {
     if (b->done) (void)hipEventDestroy(b->done);
     if (b->ev_mark) (void)hipEventDestroy(b->ev_mark);
     if (b->stream) (void)hipStreamDestroy(b->stream);
+    for (hipStream_t s : b->sides)
+        if (s) (void)hipStreamDestroy(s);
     delete b;
 }
 

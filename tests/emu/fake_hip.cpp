@@ -2,7 +2,7 @@
 // Loaded ahead of liblnt.so with RTLD_GLOBAL, it takes the library's HIP calls: device memory is
 // host memory, kernels do nothing, and every call that orders or launches work is written to a
 // log ("launch stream kernel", "graph stream nodes", "capture stream nodes", "record stream event",
-// "wait stream event", "copy stream bytes", "sync stream").  A launch can be made to fail.
+// "wait stream event", "copy stream bytes", "sync stream", "stream stream" where one is made).  A launch can be made to fail.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -100,7 +100,10 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
     return std::memmove(d, s, n), hipSuccess;
 }
 
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = handle<hipStream_t>(), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+    *s = handle<hipStream_t>();
+    return note("stream", *s), hipSuccess;
+}
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return note("sync", s), hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {

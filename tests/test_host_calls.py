@@ -94,9 +94,9 @@ print(json.dumps(dict(log=log(), sa=sa, sb=sb, failed=failed, st=a.gerbicz_stats
 
 
 def test_short_batch_steps_replay_graphs(fake):
-    """Steps of one iteration, and of up to four with many groups, launch one graph of all groups
-    for each iteration from the second such step on, and the first captures nothing; a step of
-    16 with many groups is one graph launch for each once the members' "-2" flags are right."""
+    """Steps of one iteration launch one graph of all groups from the second such step on, and the
+    first captures nothing; a step of 16 with several row/column groups is one graph launch for
+    each once the members' "-2" flags are right."""
     got = fake("""
 ps = (9689, 1000003, 2000003)  # one workgroup, rows and columns
 ts = [cuda_amd.LucasPRP(p) for p in ps]
@@ -104,28 +104,43 @@ batch = cuda_amd.Batch()
 for t in ts:
     batch.add(t)
 steps = []
-for k in (1, 1, 1):
+for k in (1, 1, 1, 16, 16, 1):
     fake.fake_clear()
     batch.iterate(k)
     steps.append([(l[0], l[2]) for l in log() if l[0] in ("launch", "graph", "capture")])
-ts += [cuda_amd.LucasPRP(p, prp=True) for p in (400009, 1000003, 2000003, 4000037)]
-for t in ts[3:]:
-    batch.add(t)
-fake.fake_clear()
-batch.iterate(3)
-batch.iterate(4)
-batch.iterate(16)
-steps.append([(l[0], l[2]) for l in log() if l[0] in ("launch", "graph", "capture")])
 print(json.dumps(steps))
 """)
     one = ["graph", "7"]  # 1 + 3 + 3 kernels
     assert [s[0] for s in got[0]] == ["launch"] * 7
     assert got[1] == [["capture", "7"], one]
-    assert got[2] == [one]
-    assert [s[0] for s in got[3][:55]] == ["launch"] * 55  # 3 of 6 * 3 kernels, and 1
-    assert got[3][55:60] == [["capture", "19"]] + [["graph", "19"]] * 4
-    sixteen = [s for s in got[3][60:] if s[0] != "capture"]
-    assert sixteen[1:] == [["graph", "48"]] * 6 and sixteen[0][0] == "launch"
+    assert got[2] == [one] and got[5] == [one]
+    for step, captures in ((got[3], 2), (got[4], 0)):
+        assert [s for s in step if s[0] == "graph"] == [["graph", "48"]] * 2
+        assert len([s for s in step if s[0] == "launch"]) == 1  # the one-workgroup test's
+        assert len([s for s in step if s[0] == "capture"]) == captures
+
+
+def test_batch_makes_its_streams_once(fake):
+    """Groups that are formed again as members come and go run on the streams that were made with
+    the batch, more groups than streams included."""
+    got = fake("""
+made = lambda: {l[1] for l in log() if l[0] == "stream"}
+batch = cuda_amd.Batch()
+streams = made()
+steps = []
+ts = []
+for p in (9689, 86243, 132049, 250007, 400009, 1000003, 2000003):
+    ts.append(cuda_amd.LucasPRP(p))
+    batch.add(ts[-1])
+    fake.fake_clear()
+    batch.iterate(3)
+    batch.iterate(40)
+    steps.append((len(made()), sorted({l[1] for l in log() if l[0] in ("launch", "graph")})))
+print(json.dumps(dict(streams=sorted(streams), steps=steps, groups=batch.stats()["groups"])))
+""")
+    assert got["groups"] == 7 and len(got["streams"]) == 5
+    for i, (made, used) in enumerate(got["steps"]):
+        assert made == 0 and set(used) < set(got["streams"]) and len(used) == min(i + 1, 4)
 
 
 def test_long_batch_steps_launch_the_groups_in_turns(fake):
