@@ -778,8 +778,10 @@ int lnt_tune(lnt_ctx *c, int loops) {
                     o.col3 = c3;
                     Plan tmp;
                     if (!make_plan(c->p, n, tmp, o).empty()) continue;
-                    // -1 elsewhere is one of the others
-                    if ((r3 >= 0 || tmp.rowm) && (c3 >= 0 || tmp.colm)) opts.push_back(o);
+                    // rows of 256 .. 2048 words on the matrix cores only: the register rows take
+                    // 1.0 to 3.1 times as long in the same split and were in no fastest plan of
+                    // 2^13 .. 2^23; -1 elsewhere is one of the others
+                    if ((r3 < 0) == (tmp.C >= 256 && tmp.C <= 2048) && (c3 >= 0 || tmp.colm)) opts.push_back(o);
                 }
     std::vector<Cand> cands;
     // warm-up long enough to capture the candidate's iteration graph, so the timed loops

@@ -98,10 +98,10 @@ def test_few_bits_per_digit_match_oracle(p, n):
     assert np.array_equal(got, o.digits_np())
 
 
-# The tuner's candidate grid (lnt_tune): row length 2^lc, column tile K, row and column
-# variants (-1: the plan's choice, the matrix-core kernels where there are any).  Shapes a
-# length does not support fall back to its default plan, so the distinct plans are those
-# lnt_describe reports.
+# Every plan LNT_PLAN can name, the tuner's candidates (lnt_tune) among them: row length 2^lc,
+# column tile K, row and column variants (-1: the plan's choice, the matrix-core kernels where
+# there are any).  Shapes a length does not support fall back to its default plan, so the
+# distinct plans are those lnt_describe reports.
 TUNER_GRID = [f"lc={lc},K={K},row3={r3},col3={c3}" for lc in range(7, 15) for K in (16, 8, 4)
               for r3 in (-1, 0, 1, 2) for c3 in (-1, 0, 1)]
 
@@ -109,8 +109,8 @@ TUNER_GRID = [f"lc={lc},K={K},row3={r3},col3={c3}" for lc in range(7, 15) for K 
 @pytest.mark.parametrize("p,n", [(2000003, 1 << 17), (16000057, 1 << 20), (70000027, 1 << 22),
                                  (140000041, 1 << 23)])
 def test_every_tunable_plan_matches_oracle(p, n, monkeypatch):
-    """Every plan lnt_tune can choose at this length, forced through LNT_PLAN, against the
-    oracle digit for digit from a random residue (LL, two iterations); every matrix-core row and
+    """Every plan of this length, those lnt_tune can choose included, forced through LNT_PLAN,
+    against the oracle digit for digit from a random residue (LL, two iterations); every matrix-core row and
     column kernel that a split of this length takes is among them."""
     import numpy as np
     from helpers import random_digits_np

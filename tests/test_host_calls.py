@@ -213,3 +213,22 @@ print(json.dumps(out))
     for n, a, b, differ, ok in got:
         assert differ, (n, a, b)
         assert ok == [a + b not in ("lc=9lc=10", "lc=12")] * 2, (n, a, b, ok)
+
+
+def test_tuner_leaves_out_register_rows(fake):
+    """Rows of 256 to 2048 words have the matrix-core kernels: the tuner times no others there, and
+    up to 2^20 no more plans than before those kernels came."""
+    got = fake("""
+out = []
+for p in (1000003, 4000037, 16000057, 70000027):
+    t = cuda_amd.LucasPRP(p)
+    t.tune(1)
+    out.append([name for name, ms in t.tune_results()])
+    t.close()
+print(json.dumps(out))
+""")
+    for names, most in zip(got, (10, 22, 23, 26)):
+        assert len(set(names)) == len(names) <= most, (len(names), most)
+        for name in names:
+            C = int(name.split("/")[0].split("x")[1])
+            assert ("lnt_k_rowm<" in name) == (256 <= C <= 2048), name
