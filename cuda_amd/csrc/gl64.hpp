@@ -93,14 +93,15 @@ GL_HD u64 gl_mul(u64 a, u64 b) {
     return gl_reduce128(hi, lo);
 }
 
-// a b 2^-64 mod P.  Montgomery reduction with radix 2^64 (Montgomery 1985): with lo = x1:x0
-// and P^-1 = 2^32 + 1 (mod 2^64), q = lo P^-1 = lo + (x0 << 32), and
+// a b 2^-64 mod P.  Montgomery reduction with radix 2^64 (Montgomery, "Modular multiplication
+// without trial division", 1985), for this modulus in the steps of Pornin, "EcGFp5: a
+// Specialized Elliptic Curve", 2022: with lo = x1:x0 and P^-1 = 2^32 + 1 (mod 2^64), q = lo P^-1 = lo + (x0 << 32), and
 // q P / 2^64 rounded up is q - (q >> 32) minus the carry of the sum that formed q, so the
 // result is hi - that, plus P on borrow.  Canonical for a canonical b (hi <= P - 1 then) and
 // any 64-bit a.  The tables hold their factors times GL_R = 2^64 mod P, so
 // gl_mmul(x, table) is the plain product; a square or a product of two field values leaves a
-// factor 2^-64, which the large path's unweighting table takes back.  The reduction is 8 VALU instructions
-// where gl_reduce128 takes 13 (whole product 20 against 25 as compiled for gfx950).
+// factor 2^-64, which the large path's unweighting table takes back.  The reduction is 8 VALU
+// instructions where gl_reduce128 takes 13 (whole product 20 against 25 as compiled for gfx950).
 GL_HD u64 gl_mmul(u64 a, u64 b) {
     u64 hi, lo;
     gl_mul_wide(a, b, hi, lo);

@@ -2,11 +2,17 @@
 // 3-phase kernels: with one tile per compute unit the load, the carry, the transform and the
 // store follow each other there, and only the transform got shorter).
 //
-// Batches with more tiles than compute units (a quarter of their slots counted) run the 256-word tiles
+// Of 128 registers 48 hold the DFT matrix.  The 1024-word forward kernel spills 6 (28 bytes per
+// lane, which is the 39.8 MB written per launch at n = 2^22 where the tile is 33.6; 27 with a halo
+// of eight digits), the four-wave form of the 256-word one 2 (24); the others spill none.
+//
+// Batches with more tiles than compute units run the 256-word tiles
 // with 4 waves of four groups each, four tiles on a unit that work past each other's loads and
 // barriers, where one test takes 16 waves a tile: per squaring of all, 16 tests of 2^20 402 -> 334 us,
 // 13 of 2^18 94 -> 79, one test of 2^20 in eight slots 81 -> 62; with fewer tiles the 16 waves stay
-// ahead (6 tests of 2^18 53 against 63).
+// ahead (6 tests of 2^18 53 against 63).  A quarter of the slots is counted: a group is formed with
+// two to four slots for each member, from five members on, and its graph stays the same while
+// members come and go, so a group that most members left keeps the form of its slots.
 #include "lnt_launch.hpp"
 
 // Compute units of an MI355X.

@@ -1,7 +1,7 @@
 // The 4096-word rows on the matrix cores.
 //
-// Bound by VALU issue: 234 VALU instructions per word (376 with register DFTs) and 24 matrix
-// instructions per 4 words; without its loads and stores the kernel takes 34 of its 43 us at
+// Bound by VALU issue: 234 VALU instructions per word (376 with register DFTs), the 24 matrix
+// instructions of a wave per word of its lanes among them; without its loads and stores the kernel takes 34 of its 43 us at
 // n = 2^22, without the matrix instructions as well 28.  128 registers keep four waves per
 // SIMD (48 hold the DFT matrix; three waves, or the next group's words fetched ahead at that
 // cost, measured 45 us).
@@ -38,6 +38,8 @@ bool lnt_launch_row16(const lnt::Plan &pl, const LntParams &P, hipStream_t s, in
 
 bool lnt_launch_batch_row16(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s) {
     if (pl.row3 != 16 || pl.C != 4096) return false;
+    // by all slots, of which a group has eight at least: the wide form is for up to 32 rows, whose
+    // launch is one row's latency whatever the slots hold
     if (pl.R * count <= ROW16_WIDE)
         hipLaunchKernelGGL(lnt_kb_row16<1>, dim3(pl.R * count), dim3(1024), 0, s, Ps, pl.R);
     else

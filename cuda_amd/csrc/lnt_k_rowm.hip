@@ -6,7 +6,7 @@
 
 // Batches that fill the chip: the 2048-word kernel's 166 registers leave a unit one workgroup of
 // eight waves, which waits for its own loads and exchanges.  Four rows per workgroup at 128
-// registers (lnt_rowm_rows_body) let two workgroups share a unit: 11 tests of 2^19 178 -> 152 us
+// registers (lnt_rowm_rows_body; 4 spilled) let two workgroups share a unit: 11 tests of 2^19 178 -> 152 us
 // per squaring of all.  With the rows of 14 tests of 2^17 (64 each) it gains nothing (62 / 60 us),
 // and the shorter rows already run several workgroups per unit (13 tests of 2^18 94 / 98 us).
 static constexpr u32 ROWM_ROWS = 4, ROWM_FULL = 1024;
@@ -36,7 +36,7 @@ bool lnt_launch_rowm(const lnt::Plan &pl, const LntParams &P, hipStream_t s, int
 bool lnt_launch_batch_rowm(const lnt::Plan &pl, const LntParams *Ps, u32 count, hipStream_t s) {
     if (pl.C != 256 * pl.rowm) return false;
     const dim3 block(64 * pl.rowm);
-    // from five members on a quarter of a batch's slots at least is in use
+    // a quarter of the slots, as for the columns (lnt_k_colm.hip)
     if (pl.rowm == 8 && pl.R % ROWM_ROWS == 0 && pl.R * (count / 4) >= ROWM_FULL) {
         const u32 wgs = pl.R / ROWM_ROWS;
         hipLaunchKernelGGL((lnt_kb_rowm_rows<8, ROWM_ROWS>), dim3(wgs * count), block, 0, s, Ps, wgs);

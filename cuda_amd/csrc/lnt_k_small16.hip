@@ -7,7 +7,8 @@
 // set for this file in the Makefile): with at most four waves per SIMD nothing else hides the
 // wait states of the carry chains (n = 256 .. 2048 2.8, 3.6, 4.1, 4.8 us without, 4096 equal).
 // At n = 4096 the addresses are formed again in every iteration: kept across it they spilled
-// (14.4 us).
+// (14.4 us).  Registers still spilled per lane: n = 2048 4 of 256 (12 with a halo of eight
+// digits), n = 4096 none of 128 (12), the others none.
 #include "lnt_launch.hpp"
 
 template <int S, int M>

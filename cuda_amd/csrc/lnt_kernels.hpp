@@ -1478,7 +1478,8 @@ LNT_KFN void lnt_tiny_body(int tid, LView lds, const LntParams &P, u32 iters, bo
 // between the carry and weights and the unweights.  One test is a chain of dependent steps on
 // one compute unit, so what counts is its latency: four words per thread put four times the
 // waves of the former 16-word kernels to work on it, an iteration has four barriers, and up to
-// S = 8 the factors of a thread's words stay in registers.  For n = 4096 that would take more
+// S = 8 the factors of a thread's words stay in registers (at S = 8, where eight waves have 256
+// registers each, all but 4 of them, and all but 12 with a halo of eight digits).  For n = 4096 that would take more
 // than the 128 registers of 16 waves: weights and twiddles are re-read (from the L2, ahead of
 // their use) and the unweights lie in LDS.
 // LDS: two regions, the residue (or its digits) in natural order in one while the other holds

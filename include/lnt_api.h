@@ -171,9 +171,8 @@ int lnt_iterate_static(uint32_t p, int mode, uint64_t *x, size_t n, uint32_t k, 
 
 /* ---- batches of independent tests (new: the reference runs one test per process) ----
  * Members keep their own residues; members of the same shape run as one batched launch
- * per kernel, and the shapes advance side by side on streams of their own, joined at the
- * end of the call (and at every Gerbicz block end).  Work issued
- * on a member after lnt_batch_iterate runs after the batch's work.  A context belongs to
+ * per kernel, and the shapes advance side by side on the batch's streams, joined at the end
+ * of the call (and at every Gerbicz block end).  Work issued on a member after lnt_batch_iterate runs after the batch's work.  A context belongs to
  * at most one batch; lnt_destroy takes it out of its batch. */
 typedef struct lnt_batch lnt_batch;
 int lnt_batch_create(int device, lnt_batch **out);
