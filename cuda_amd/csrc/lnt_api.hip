@@ -1251,7 +1251,9 @@ static int batch_mark_pending(lnt_batch *b, lnt_batch::Group &g, hipStream_t s) 
             changed = true;
         }
     }
-    return changed ? batch_upload(b, g, s) : LNT_OK;
+    const int rc = changed ? batch_upload(b, g, s) : LNT_OK;
+    if (rc != LNT_OK) b->upload = true;  // by the next step
+    return rc;
 }
 
 // A step of one iteration as a graph of all groups, on the batch stream: the groups' streams

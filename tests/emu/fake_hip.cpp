@@ -44,7 +44,7 @@ extern "C" {
 
 const char *fake_log() { return g_log.c_str(); }
 void fake_clear() { g_log.clear(); }
-// The nth following call of a kind ("launch": a kernel, "graph": a graph launch) fails.
+// The nth following call of a kind ("launch": a kernel, "graph": a graph launch, "copy") fails.
 void fake_fail(const char *kind, int nth) {
     g_fail_kind = kind;
     g_fail_in = nth;
@@ -96,6 +96,7 @@ hipError_t hipMalloc(void **p, size_t n) { return *p = std::calloc(1, n), *p ? h
 hipError_t hipFree(void *p) { return std::free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
+    if (fails("copy")) return hipErrorUnknown;
     note("copy", st, std::to_string(n));
     return std::memmove(d, s, n), hipSuccess;
 }

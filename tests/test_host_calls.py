@@ -93,6 +93,26 @@ print(json.dumps(dict(log=log(), sa=sa, sb=sb, failed=failed, st=a.gerbicz_stats
     assert got["st"]["iteration"] == 80 and got["st"]["checks"] == (2 if block == 40 else 0)
 
 
+def test_failed_parameter_copy_is_made_up_for(fake):
+    """The members' "-2" flags change after their first iteration; if copying them fails, the next
+    step copies them before it launches anything."""
+    got = fake("""
+t = cuda_amd.LucasPRP(1000003)
+batch = cuda_amd.Batch()
+batch.add(t)
+fake.fake_fail(b"copy", 2)  # the first is that of new groups
+try:
+    batch.iterate(5)
+    failed = False
+except cuda_amd.LntError:
+    failed = True
+fake.fake_clear()
+batch.iterate(5)
+print(json.dumps(dict(failed=failed, ops=[l[0] for l in log() if l[0] in ("copy", "launch")])))
+""")
+    assert got["failed"] and got["ops"] == ["copy"] + ["launch"] * 15
+
+
 def test_short_batch_steps_replay_graphs(fake):
     """Steps of one iteration launch one graph of all groups from the second such step on, and the
     first captures nothing; a step of 16 with several row/column groups is one graph launch for
